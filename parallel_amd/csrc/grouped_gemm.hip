@@ -9,12 +9,12 @@
 //
 // Tiling: WM x WN waves; each wave owns (BM/WM) x (BN/WN) of 32x32 MFMA
 // sub-tiles (v_mfma_f32_32x32x16_bf16, fp32 accumulators), its row sub-tiles
-// interleaved with the other wave rows'.  The expert GEMMs use 256x256 tiles
-// (384x128 when the output is at most 1024 columns wide) on 8 waves (two waves
+// interleaved with the other wave rows'.  The expert GEMMs use 256-column
+// tiles of 64 to 320 rows, by the mean rows per expert, on 8 waves (two waves
 // per SIMD, one workgroup per CU); the small router GEMMs use 128x128 on 4
 // waves.  Operands move from HBM to LDS by DMA (buffer_load_dwordx4 ... lds,
-// no register staging) into a 5-deep ring of 32-deep k-tiles that fills
-// the 160 KiB of LDS, so three or four k-tiles of loads are in flight while
+// no register staging) into a ring of 32- or 64-deep k-tiles (5 stages of 32
+// for 256x256 tiles) that fills the 160 KiB of LDS, so three or four k-tiles of loads are in flight while
 // one is multiplied; each wave fires its share of a k-tile's DMA between its
 // MFMA groups.  At the roughly 256 rows per expert of a training step the
 // expert GEMMs sit near the ridge of the roofline (about 256 flop per weight
@@ -197,10 +197,13 @@ struct TileCfg {
 };
 // Expert GEMMs and weight gradients: 160 KiB ring, 8 waves.
 using BigTile = TileCfg<256, 256, 32, 2, 4, 5>;
-// Expert GEMMs with narrow outputs: 384-row tiles, so that an expert of up to
-// 384 rows is one m-tile and its weights stream through LDS once per n-tile;
-// 160 KiB ring (5 x 32 KiB, so the block barrier pairs k-steps), 8 waves.
-using TallTile = TileCfg<384, 128, 32, 4, 2, 5>;
+// Expert GEMMs of few rows, bound by the weights' stream from HBM: 64-deep
+// k-tiles (a K-contiguous weight row's 128 bytes, a whole cache line, per
+// k-step) and as many weight bytes in flight as the LDS holds beside few rows:
+// 96 KiB with 64-row tiles (4-deep ring of 40 KiB stages), 64 KiB with 128-row
+// tiles (3-deep ring of 48 KiB), against 48 KiB with 320-row tiles.
+using SlimTile = TileCfg<64, 256, 64, 2, 4, 4>;
+using MidTile = TileCfg<128, 256, 64, 2, 4, 3>;
 // Router GEMMs (N = E = 128): 80 KiB ring, 4 waves (two workgroups per CU).
 using SmallTile = TileCfg<128, 128, 32, 2, 2, 5>;
 // The 256x256 loop with the fragment reads of each 16-deep half step
@@ -1366,43 +1369,66 @@ int launch(GemmParams& p, hipStream_t stream, const char* name) {
   return launch_status(name);
 }
 
-// Mean rows per expert from which the forward expert GEMMs take the
-// ping-pong loop (C4, 1024: the four row-grouped GEMMs 2769 against 2844 us;
-// C5, 512: 5297 against 5465 us; C2, 256: up_fwd 312 against 305 us).
-constexpr int64_t kPingMinMeanRows = 448;
-// Mean rows per expert up to which the expert GEMMs with wide outputs take
-// 320-row tiles.
+// Bounds of launch_expert's rule, in mean rows per expert.
+constexpr int64_t kSlimMaxMeanRows = 32;
+constexpr int64_t kMidMaxMeanRows = 128;
+constexpr int64_t kBigMaxMeanRows = 224;
 constexpr int64_t kWideMaxMeanRows = 288;
+constexpr int64_t kPingMinMeanRows = 448;
+// Weight rows of at least this many elements (8 KiB) keep the 32-deep k-tiles
+// up to kLongRowMaxMeanRows mean rows.
+constexpr int kLongRow = 4096;
+constexpr int64_t kLongRowMaxMeanRows = 64;
 
-// Expert GEMM over grouped rows.  256x256 tiles do the most MFMA work per
-// k-step of LDS traffic, but with few output columns their grid (about one
-// or two m-tiles per expert times the column tiles) ends in a poorly
-// balanced last round; 384x128 tiles give one m-tile per expert of up to 384
-// rows and twice the column tiles; they win when the experts hold about 256
-// rows each (a training step's uniform routing).  With more rows per expert
-// on average, or skewed counts, the 256x256 tile's intensity wins: the down
-// projection's input gradient took 631 against 723 us at 1024 rows per
-// expert (C4), 163 against 192 us at 380 rows with Zipf-skewed counts (C3).
+// Expert GEMM over grouped rows; the tile by the mean rows per expert (the
+// real counts stay on the device).  An expert that fits one m-tile streams its
+// weights through one CU's LDS per n-tile, so the tile is the smallest that
+// holds nearly every expert under uniform routing, which leaves the most LDS
+// for weights in flight; experts above it take further m-tiles.  The results
+// are the same bits for every tile.  Kernel times in us at H 2048, I 768, 128
+// experts, top-8 (up_fwd / down_fwd / down_dgrad with its SwiGLU pass /
+// up_dgrad), one box:
+//   mean rows   3 (T 48):   64-row tile 140 / 70 / 77 / 130, 128-row 143 / 74 /
+//                           82 / 129, 320-row (384x128 for down_dgrad) 170 / 98 /
+//                           112 / 136: 5.5 against 3.9-4.5 TB/s
+//              19 (T 301):  64-row 155 / 78 / 86 / 139, 320-row 173 / 94 / 114 / 142
+//              48 (T 768):  128-row 167 / 88 / 98 / 145, 64-row 188 / 95 / 97 / 157,
+//                           320-row 186 / 103 / 124 / 157
+//              96 (T 1531): 128-row 185 / 97 / 114 / 155, 256-row 198 / 108 / 126 /
+//                           162, 320-row 204 / 114 / 138 / 170
+//             156 (T 2500): 256-row 221 / 119 / 155 / 187, 128-row 236 / 124 / 145 /
+//                           209, 320-row 230 / 127 / 164 / 205
+//             219 (T 3500): 256-row 245 / 131 / 179 / 207, 320-row 265 / 141 / 190
+//                           (384x128) / 235, 128-row for down_dgrad 165
+//             256 (T 4096): 320-row 281 / 152 / - / 250, 256-row 307 / 160 / 229 /
+//                           267, down_dgrad 128-row 195 against 206 (384x128)
+// Narrow outputs (at most 1024 columns: down_dgrad at I 768) have few n-tiles,
+// and the 128-row tile's finer grid keeps winning up to kWideMaxMeanRows.
+// Weight rows of 8 KiB (H 4096) are faster on 32-deep k-tiles while they are
+// streamed for few rows (64 experts' rows of a k-step then spread over half as
+// many lines): up_fwd at 19 mean rows 562 on the 256-row tile against 597,
+// up_dgrad 504 on the 320-row tile against 552.
 template <bool B_KCONTIG, int EPI>
 int launch_expert(GemmParams& p, hipStream_t stream, const char* name) {
   const int out_cols = (EPI == EPI_SWIGLU_FWD) ? 2 * p.swiglu_I : p.N;
-  constexpr int64_t kTallMaxMeanRows = 288;
-  if (out_cols <= 1024 && static_cast<int64_t>(p.rows) <= kTallMaxMeanRows * p.G)
-    return launch<MODE_MG, B_KCONTIG, EPI, TallTile>(p, stream, name);
-  // A training step's routing (about 256 rows per expert, a few above):
-  // with 320-row tiles every expert of up to 320 rows is one m-tile, so its
-  // weights stream through one CU's LDS per n-tile instead of two (C2:
-  // up_fwd 280 against 318 us, down_fwd 155 against 167, up_dgrad 248
-  // against 272 on ping-pong).
-  if (static_cast<int64_t>(p.rows) <= kWideMaxMeanRows * p.G)
+  const int64_t rows = p.rows, G = p.G;
+  const bool long_rows = p.ldb >= kLongRow && rows <= kLongRowMaxMeanRows * G;
+  if (!long_rows && rows <= kSlimMaxMeanRows * G) return launch<MODE_MG, B_KCONTIG, EPI, SlimTile>(p, stream, name);
+  if (!long_rows && rows <= (out_cols <= 1024 ? kWideMaxMeanRows : kMidMaxMeanRows) * G)
+    return launch<MODE_MG, B_KCONTIG, EPI, MidTile>(p, stream, name);
+  // Up to 320 rows per expert in one m-tile, and the input gradients of long
+  // weight rows.
+  if (rows <= kWideMaxMeanRows * G && (rows > kBigMaxMeanRows * G || (long_rows && !B_KCONTIG)))
     return launch<MODE_MG, B_KCONTIG, EPI, WideTile>(p, stream, name);
   // The ping-pong loop keeps the matrix pipes fed while the partner waves
   // read fragments and fire the DMA.  It wins for the input gradients (two
   // transpose reads per weight fragment), and for the forward GEMMs once the
-  // experts average several m-tiles (their weight tiles then come from L2);
-  // with one or two m-tiles per expert the forward GEMMs stream every weight
-  // k-slice from HBM and time the same on both loops.
-  if (!B_KCONTIG || static_cast<int64_t>(p.rows) >= kPingMinMeanRows * p.G)
+  // experts average several m-tiles (their weight tiles then come from L2;
+  // the four row-grouped GEMMs at 1024 mean rows 2769 against 2844 us, at 512
+  // and H 4096 5297 against 5465 us); with one or two m-tiles per expert the
+  // forward GEMMs stream every weight k-slice from HBM and time the same on
+  // both loops.
+  if (!B_KCONTIG || rows >= kPingMinMeanRows * G)
     return launch<MODE_MG, B_KCONTIG, EPI, PingTile>(p, stream, name);
   return launch<MODE_MG, B_KCONTIG, EPI, BigTileP>(p, stream, name);
 }

@@ -432,6 +432,46 @@ def test_grouped_gemm_wgrad_skewed_routing(name, accumulate, f32):
     print(f"{name}: {G} groups, {M} rows, worst rel {float(rel[live].max()):.2e}")
 
 
+# Mean rows per expert on both sides of every bound of the row-tile rule, counts at the edges of the
+# 64- and 128-row tiles, K tails inside a 64-deep k-tile, weight rows of 4096 elements.
+ROW_TILE_CASES = [
+    ("slim", [64, 65, 1, 0, 17, 3, 63], 264, 200),
+    ("slim_shortk", [1, 0, 2, 1], 520, 40),
+    ("mid", [128, 129, 1, 64, 0, 127, 200], 264, 200),
+    ("mid_narrow", [288, 250, 320, 257, 1], 72, 520),
+    ("big", [256, 257, 100, 224], 1288, 136),
+    ("wide", [320, 321, 200, 230], 1288, 136),
+    ("long_rows_few", [64, 20, 0, 65], 1032, 4104),
+    ("long_rows_mid", [130, 90, 0, 128], 1032, 4104),
+]
+
+
+@pytest.mark.parametrize("name,cnt,N,K", ROW_TILE_CASES, ids=[c[0] for c in ROW_TILE_CASES])
+def test_row_tiles_give_the_exact_products(name, cnt, N, K):
+    """Small integers: every product and sum is exact in fp32 and every result below 2^8 in bf16, so
+    the outputs must be the float64 products rounded once, whatever the tile."""
+    counts, offs = _groups(cnt)
+    M, G = int(counts.sum()), len(cnt)
+    od = offs.to(DEV)
+    a = torch.randint(-1, 2, (M, K), generator=gen(21)).to(BF)
+    dc = torch.randint(-1, 2, (M, N), generator=gen(22)).to(BF)
+    w = torch.randint(-1, 2, (G, N, K), generator=gen(23)).to(BF)
+    ad, dcd, wd = a.to(DEV), dc.to(DEV), w.to(DEV)
+    c = torch.full((M, N), 7.0, dtype=BF, device=DEV)
+    da = torch.full((M, K), 7.0, dtype=BF, device=DEV)
+    s = _lib.stream_of(c)
+    _lib.call("moe_grouped_gemm_fwd", ad.data_ptr(), wd.data_ptr(), od.data_ptr(), G, M, N, K, c.data_ptr(), s)
+    _lib.call("moe_grouped_gemm_dgrad", dcd.data_ptr(), wd.data_ptr(), od.data_ptr(), G, M, N, K, da.data_ptr(), s)
+    torch.cuda.synchronize()
+    ref_c, ref_da, s0 = [], [], 0
+    for e, n in enumerate(counts.tolist()):
+        ref_c.append(a[s0:s0 + n].double() @ w[e].double().t())
+        ref_da.append(dc[s0:s0 + n].double() @ w[e].double())
+        s0 += n
+    assert torch.equal(c.cpu(), torch.cat(ref_c).to(BF)), f"{name}: forward"
+    assert torch.equal(da.cpu(), torch.cat(ref_da).to(BF)), f"{name}: input gradient"
+
+
 @pytest.mark.parametrize("cnt,I,H", [([256, 0, 300, 1, 128], 768, 2048), ([5, 64, 0, 17], 64, 96),
                                      ([600, 0, 1500, 5, 257], 768, 2048)])  # the last on the ping-pong loop
 def test_swiglu_fwd_and_fused_backward(cnt, I, H):

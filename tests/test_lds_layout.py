@@ -85,6 +85,26 @@ def test_transpose_read_layout_is_consistent_and_conflict_free(R, WT):
     assert check_mc(R, WT, mc_swizzle) == 0
 
 
+@pytest.mark.parametrize("R", [64, 128, 256])
+def test_64_deep_k_contiguous_layout_is_consistent_and_conflict_free(R):
+    """64-deep k-tiles: 8 chunks of 16 B per row, 8 rows per DMA instruction, chunk c of row r at slot
+    c ^ ((r >> 1) & 7); fragments of 32 rows, chunk 2 ks + lane / 32."""
+    where = {}
+    for li in range(R * 128 // 1024):
+        for lane in range(64):
+            r = li * 8 + (lane >> 3)
+            where[(r, (lane & 7) ^ ((r >> 1) & 7))] = li * 1024 + lane * 16
+    for row0 in range(0, R, 32):
+        for ks in range(4):
+            addrs = []
+            for lane in range(64):
+                l32, kh = lane & 31, lane >> 5
+                off = row0 * 128 + l32 * 128 + (((2 * ks + kh) ^ ((l32 >> 1) & 7)) << 4)
+                assert where[(row0 + l32, 2 * ks + kh)] == off
+                addrs.append(off)
+            assert bank_conflicts(addrs, 16, 16) == 0
+
+
 def test_model_flags_32_bank_swizzles():
     assert check_kc(256, lambda r: (r >> 1) & 3) > 0
     assert check_mc(256, 64, lambda kk: 2 * (kk & 3)) > 0
