@@ -5,7 +5,7 @@
 // act_fn(gate) * up, the weighted sum over the k routes).  These kernels run
 // that path on gfx950 with fp32 operands and fp32 arithmetic throughout:
 //   - one grouped GEMM, C(i, j) (+)= sum_r A(i, r) B(r, j) with arbitrary
-//     strides, on v_mfma_f32_32x32x2_f32 (one 32x32 output tile per wave),
+//     strides, on v_mfma_f32_32x32x2_f32 over LDS tiles,
 //     grouped over the output rows (the projections and their input
 //     gradients: rows of group g use weight g) or over the reduction rows
 //     (the weight gradients: group g's rows give weight g's gradient);
@@ -14,13 +14,14 @@
 // It serves fp32 modules (the C1 configuration); the bf16 path is the tuned
 // one.  The row permutation itself is moe_permute_fwd over the rows' bytes.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
 namespace moe {
 namespace {
 
-constexpr int kF32Waves = 4;  // waves (32x32 tiles) per block
+constexpr int kNumXcd = 8;
 
 struct F32Gemm {
   const float* A;
@@ -38,70 +39,298 @@ __device__ __forceinline__ void f32_group_rows(const int32_t* offs, int g, int n
   hi = min(max(offs[g], lo), n);
 }
 
-// One wave per 32x32 tile of C.  Lane l of an MFMA step supplies A(i0 + l % 32,
-// r + l / 32) and B(r + l / 32, j0 + l % 32), and holds D rows
-// 8 (q / 4) + 4 (l / 32) + q % 4 (q = 0..15) of column j0 + l % 32.
-__global__ __launch_bounds__(kF32Waves * kWave) void f32_grouped_gemm_kernel(const F32Gemm p, int tiles_j,
-                                                                            int64_t ntiles) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t tile = static_cast<int64_t>(blockIdx.x) * kF32Waves + (threadIdx.x >> 6);
-  if (tile >= ntiles) return;
-  const int tj = static_cast<int>(tile % tiles_j);
-  int64_t rest = tile / tiles_j;
-  int g = 0, i_begin = 0, i_end = p.M, r_begin = 0, r_end = p.K, i0;
+// How an operand reaches LDS: 16-byte loads along the reduction (its rows are
+// contiguous in r), 16-byte loads along the output dimension, or 4-byte loads
+// with any strides.
+enum F32Load { kAlongR = 0, kAlongOut = 1, kScalar = 2 };
+
+// Tile of C.  KSPLIT 1: WM x WN waves of SM x SN MFMA tiles of 32x32 each;
+// KSPLIT 4: one 32x32 tile whose four waves take a quarter of each k-tile and
+// are added at the end.  KW: k's per wave and k-tile.
+template <int SM_, int SN_, int WM_, int WN_, int KSPLIT_, int KW_>
+struct F32Tile {
+  static constexpr int SM = SM_, SN = SN_, WM = WM_, WN = WN_, KSPLIT = KSPLIT_, KW = KW_;
+  static constexpr int kThreads = kWave * WM * WN * KSPLIT;
+  static constexpr int BM = 32 * SM * WM, BN = 32 * SN * WN, BK = KW * KSPLIT;
+  // LDS rows (one k each) of 4 mod 16 floats: the lanes of a wave that write
+  // pieces of 4 k's, and the two half-waves that read k and k + 1, mostly fall
+  // on different banks.
+  static constexpr int LDA = BM + 36, LDB = BN + 36;
+};
+
+// One C tile per block.  The MFMA is v_mfma_f32_32x32x2_f32 (64 cycles), so a
+// 16-deep k-tile of a 64x64 block is 512 matrix cycles on every SIMD against
+// 8 KiB of operands: the matrix pipe is the bound as long as the operands
+// arrive, which they do from a double-buffered LDS tile filled through
+// registers, the next k-tile's loads in flight during the current one's
+// products and six blocks resident per CU (88 TFLOP/s on 8192 x 1024 x 1024
+// over 32 experts, padding of the experts' rows left out; the same products
+// loaded straight from memory into the MFMA operands, 4 strided bytes per
+// lane, ran at 17).  Each output's products are added in increasing r
+// (KSPLIT 4: in four interleaved quarters).  Lane l of an MFMA supplies
+// A(l % 32, r + l / 32) and B(r + l / 32, l % 32), and holds D rows
+// 8 (q / 4) + 4 (l / 32) + q % 4 (q = 0..15) of column l % 32.
+template <int LA, int LB, class T>
+__global__ __launch_bounds__(T::kThreads) void f32_grouped_gemm_kernel(const F32Gemm p, int tiles_j) {
+  constexpr int BM = T::BM, BN = T::BN, BK = T::BK, SM = T::SM, SN = T::SN;
+  constexpr int NVA = BM * BK / 4 / T::kThreads, NVB = BN * BK / 4 / T::kThreads;
+  static_assert(NVA >= 1 && NVB >= 1 && NVA * T::kThreads * 4 == BM * BK && NVB * T::kThreads * 4 == BN * BK,
+                "every thread stages whole 16-byte pieces of both operands");
+  constexpr int A_FLOATS = BK * T::LDA, STAGE = A_FLOATS + BK * T::LDB;
+  static_assert(T::KSPLIT == 1 || 4 * 32 * 32 <= 2 * STAGE, "the wave partials fit in the ring");
+  __shared__ __attribute__((aligned(16))) float lds[2 * STAGE];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, half = lane >> 5;
+
+  // The tile: block b is the (b / 8)-th of XCD b % 8's contiguous share of
+  // the real tiles (group-major, then m-tile, then n-tile).
+  const int xcd = blockIdx.x % kNumXcd;
+  const int64_t idx = blockIdx.x / kNumXcd;
+  int mtiles = 0;  // m-tiles over all groups
   if (p.mode == 0) {
-    // the rest-th 32-row tile over the groups' row ranges
-    int t = static_cast<int>(rest);
-    g = -1;
-    for (int gg = 0; gg < p.G; ++gg) {
-      int lo, hi;
-      f32_group_rows(p.offs, gg, p.M, lo, hi);
-      const int nt = (hi - lo + 31) / 32;
-      if (t < nt) {
-        g = gg;
-        i_begin = lo;
-        i_end = hi;
+    for (int c0 = 0; c0 < p.G; c0 += kWave) {
+      int lo = 0, hi = 0;
+      if (c0 + lane < p.G) f32_group_rows(p.offs, c0 + lane, p.M, lo, hi);
+      mtiles += __builtin_amdgcn_readlane(wave_inclusive_scan((hi - lo + BM - 1) / BM), kWave - 1);
+    }
+  } else {
+    mtiles = p.G * ((p.M + BM - 1) / BM);
+  }
+  const int64_t real = static_cast<int64_t>(mtiles) * tiles_j, share = (real + kNumXcd - 1) / kNumXcd;
+  const int64_t tile = xcd * share + idx;
+  if (idx >= share || tile >= real) return;
+  const int tj = static_cast<int>(tile % tiles_j);
+  const int mt = static_cast<int>(tile / tiles_j);
+  int g = 0, i0 = 0, i_end = p.M, r_begin = 0, r_end = p.K;
+  if (p.mode == 0) {
+    int base = 0;
+    for (int c0 = 0; c0 < p.G; c0 += kWave) {
+      int lo = 0, hi = 0;
+      if (c0 + lane < p.G) f32_group_rows(p.offs, c0 + lane, p.M, lo, hi);
+      const int nt = (hi - lo + BM - 1) / BM;
+      const int incl = wave_inclusive_scan(nt);
+      const int tot = __builtin_amdgcn_readlane(incl, kWave - 1);
+      if (mt < base + tot) {
+        const int q = __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(base + incl > mt)));
+        const int local = mt - base - __builtin_amdgcn_readlane(incl - nt, q);
+        const int n = __builtin_amdgcn_readlane(nt, q);
+        const int rows_lo = __builtin_amdgcn_readlane(lo, q), rows_hi = __builtin_amdgcn_readlane(hi, q);
+        // the group's rows split evenly over its m-tiles, in whole 32-row MFMA tiles
+        const int rpt = min(BM, ((rows_hi - rows_lo + n - 1) / n + 31) & ~31);
+        g = c0 + q;
+        i0 = rows_lo + local * rpt;
+        i_end = min(i0 + rpt, rows_hi);
         break;
       }
-      t -= nt;
+      base += tot;
     }
-    if (g < 0) return;  // past the last tile (the grid is sized for the worst case)
-    i0 = i_begin + 32 * t;
   } else {
-    const int tiles_i = (p.M + 31) / 32;
-    g = static_cast<int>(rest / tiles_i);
-    i0 = 32 * static_cast<int>(rest % tiles_i);
+    const int tiles_i = (p.M + BM - 1) / BM;
+    g = mt / tiles_i;
+    i0 = BM * (mt - g * tiles_i);
+    i_end = min(i0 + BM, p.M);
     if (p.K > 0) f32_group_rows(p.offs, g, p.K, r_begin, r_end);  // no reduction rows: every group is empty
   }
-  const int j0 = 32 * tj;
+  const int j0 = BN * tj;
   const float* B = p.B + (p.mode == 0 ? static_cast<int64_t>(g) * p.sBg : 0);
   float* C = p.C + (p.mode == 1 ? static_cast<int64_t>(g) * p.sCg : 0);
-  const int ia = i0 + (lane & 31), jb = j0 + (lane & 31), rl = lane >> 5;
-  const bool ia_ok = ia < i_end, jb_ok = jb < p.N;
-  f32x16_t acc;
+
+  // 16-byte piece v of this thread: its k and output index within the tile.
+  // Along r: BK / 4 lanes take one row; along the output: whole k-rows.
+  auto piece = [&](int v, int layout, int extent, int& k, int& o) __attribute__((always_inline)) {
+    const int id = v * T::kThreads + tid;
+    if (layout == kAlongR) {
+      k = (id % (BK / 4)) * 4;
+      o = id / (BK / 4);
+    } else {
+      k = id / (extent / 4);
+      o = (id % (extent / 4)) * 4;
+    }
+  };
+  // One piece from memory: elements (o + e, r) or (o, r + e), zeros outside
+  // [0, o_end) and past r_end.
+  auto fetch = [&](const float* P, int layout, int64_t so, int64_t sr, int o, int o_end, int r)
+                   __attribute__((always_inline)) {
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (layout == kScalar) {
+      if (r < r_end) {
+        const float* q = P + static_cast<int64_t>(r) * sr + static_cast<int64_t>(o) * so;
+        if (o < o_end) v.x = q[0];
+        if (o + 1 < o_end) v.y = q[so];
+        if (o + 2 < o_end) v.z = q[2 * so];
+        if (o + 3 < o_end) v.w = q[3 * so];
+      }
+    } else if (o < o_end && r < r_end) {  // (sizes are multiples of 4 along the piece: all in or all out)
+      v = *reinterpret_cast<const float4*>(P + (layout == kAlongR ? static_cast<int64_t>(o) * so + r
+                                                                  : static_cast<int64_t>(r) * sr + o));
+    }
+    return v;
+  };
+  float4 ra[NVA], rb[NVB];
+  auto load = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-  for (int q = 0; q < 16; ++q) acc[q] = 0.0f;
-  for (int r0 = r_begin; r0 < r_end; r0 += 16) {
-    float a[8], b[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int r = r0 + 2 * u + rl;
-      const bool r_ok = r < r_end;
-      a[u] = (ia_ok && r_ok) ? p.A[static_cast<int64_t>(ia) * p.sAi + static_cast<int64_t>(r) * p.sAr] : 0.0f;
-      b[u] = (jb_ok && r_ok) ? B[static_cast<int64_t>(r) * p.sBr + static_cast<int64_t>(jb) * p.sBj] : 0.0f;
+    for (int v = 0; v < NVA; ++v) {
+      int k, o;
+      piece(v, LA, BM, k, o);
+      ra[v] = fetch(p.A, LA, p.sAi, p.sAr, i0 + o, i_end, r_begin + t * BK + k);
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u], b[u], acc, 0, 0, 0);
-  }
-  if (!jb_ok) return;
-#pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int i = i0 + 8 * (q / 4) + 4 * (lane >> 5) + (q % 4);
-    if (i < i_end) {
-      float* c = C + static_cast<int64_t>(i) * p.sCi + static_cast<int64_t>(jb) * p.sCj;
-      *c = p.accumulate ? *c + acc[q] : acc[q];
+    for (int v = 0; v < NVB; ++v) {
+      int k, o;
+      piece(v, LB, BN, k, o);
+      rb[v] = fetch(B, LB, p.sBj, p.sBr, j0 + o, p.N, r_begin + t * BK + k);
     }
+  };
+  auto put = [&](float* s, int layout, int ld, int k, int o, const float4& v) __attribute__((always_inline)) {
+    if (layout == kAlongR) {
+      s[k * ld + o] = v.x;
+      s[(k + 1) * ld + o] = v.y;
+      s[(k + 2) * ld + o] = v.z;
+      s[(k + 3) * ld + o] = v.w;
+    } else {
+      *reinterpret_cast<float4*>(s + k * ld + o) = v;
+    }
+  };
+  auto stage = [&](int t) __attribute__((always_inline)) {
+    float* s = lds + (t & 1) * STAGE;
+#pragma unroll
+    for (int v = 0; v < NVA; ++v) {
+      int k, o;
+      piece(v, LA, BM, k, o);
+      put(s, LA, T::LDA, k, o, ra[v]);
+    }
+#pragma unroll
+    for (int v = 0; v < NVB; ++v) {
+      int k, o;
+      piece(v, LB, BN, k, o);
+      put(s + A_FLOATS, LB, T::LDB, k, o, rb[v]);
+    }
+  };
+
+  // A wave's 32-row tiles are interleaved with the other wave row's, so that
+  // the rows of a partly filled tile spread over the waves; tiles without
+  // rows skip their products.
+  const int wm = T::KSPLIT == 1 ? wave / T::WN : 0, wn = T::KSPLIT == 1 ? wave % T::WN : 0;
+  const int kw = T::KSPLIT == 1 ? 0 : wave * T::KW;  // this wave's k's within a k-tile
+  const int subs = (i_end - i0 + 31) / 32;
+  const int na = __builtin_amdgcn_readfirstlane(subs > wm ? (subs - wm + T::WM - 1) / T::WM : 0);
+  f32x16_t acc[SM][SN];
+#pragma unroll
+  for (int i = 0; i < SM; ++i)
+#pragma unroll
+    for (int j = 0; j < SN; ++j)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
+  static_assert(SM <= 2, "a wave has all its row tiles live, one or none");
+  const int nk = (r_end - r_begin + BK - 1) / BK;  // 0: an empty group's zeros
+  if (nk > 0) {
+    load(0);
+    stage(0);
+    __syncthreads();
   }
+  // One copy of the loop per count of live 32-row tiles: guards inside the
+  // unrolled products made the compiler move the accumulators around and kept
+  // it from spreading the LDS reads.
+  auto loop = [&](auto live) __attribute__((always_inline)) {
+    constexpr int NA = decltype(live)::value;
+    for (int t = 0; t < nk; ++t) {
+      if (t + 1 < nk) load(t + 1);
+      const float* sa = lds + (t & 1) * STAGE + kw * T::LDA + wm * 32 + l32;
+      const float* sb = lds + (t & 1) * STAGE + A_FLOATS + kw * T::LDB + wn * 32 * SN + l32;
+#pragma unroll
+      for (int u = 0; u < T::KW / 2; ++u) {
+        float a[SM], b[SN];
+#pragma unroll
+        for (int i = 0; i < NA; ++i) a[i] = sa[(2 * u + half) * T::LDA + i * T::WM * 32];
+#pragma unroll
+        for (int j = 0; j < (NA ? SN : 0); ++j) b[j] = sb[(2 * u + half) * T::LDB + j * 32];
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+#pragma unroll
+          for (int j = 0; j < SN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+      }
+      // The other buffer was last read in step t - 1, before that step's barrier.
+      if (t + 1 < nk) stage(t + 1);
+      __syncthreads();
+    }
+  };
+  if (na == SM) {
+    loop(std::integral_constant<int, SM>{});
+  } else if (na > 0) {
+    loop(std::integral_constant<int, 1>{});
+  } else {
+    loop(std::integral_constant<int, 0>{});
+  }
+  if constexpr (T::KSPLIT > 1) {
+    float* part = lds;  // [4][32][32], after the loop's last barrier
+#pragma unroll
+    for (int q = 0; q < 16; ++q) part[(wave * 32 + 8 * (q / 4) + 4 * half + (q % 4)) * 32 + l32] = acc[0][0][q];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 32 * 32 / T::kThreads; ++e) {
+      const int id = e * T::kThreads + tid, row = id / 32, col = id % 32;
+      const int i = i0 + row, j = j0 + col;
+      if (i < i_end && j < p.N) {
+        const float v = ((part[id] + part[1024 + id]) + part[2048 + id]) + part[3072 + id];
+        float* c = C + static_cast<int64_t>(i) * p.sCi + static_cast<int64_t>(j) * p.sCj;
+        *c = p.accumulate ? *c + v : v;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < SM; ++i)
+#pragma unroll
+      for (int j = 0; j < SN; ++j) {
+        const int jc = j0 + (wn * SN + j) * 32 + l32;
+        if (jc >= p.N) continue;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+          const int ir = i0 + (wm + T::WM * i) * 32 + 8 * (q / 4) + 4 * half + (q % 4);
+          if (ir < i_end) {
+            float* c = C + static_cast<int64_t>(ir) * p.sCi + static_cast<int64_t>(jc) * p.sCj;
+            *c = p.accumulate ? *c + acc[i][j][q] : acc[i][j][q];
+          }
+        }
+      }
+  }
+}
+
+template <int LA, int LB, class T>
+int f32_launch_tile(const F32Gemm& p, hipStream_t stream) {
+  const int tiles_j = (p.N + T::BN - 1) / T::BN;
+  // mode 0: every group's rows in BM-row tiles, at most M / BM + G of them
+  const int64_t tiles_i = p.mode == 0 ? (p.M + T::BM - 1) / T::BM + p.G
+                                      : static_cast<int64_t>(p.G) * ((p.M + T::BM - 1) / T::BM);
+  const int64_t blocks = (tiles_i * tiles_j + kNumXcd - 1) / kNumXcd * kNumXcd;
+  MOE_REQUIRE(blocks < (1ll << 31) && tiles_i < (1ll << 31), MOE_ERR_UNSUPPORTED, "f32 grouped gemm: too many tiles");
+  hipLaunchKernelGGL((f32_grouped_gemm_kernel<LA, LB, T>), dim3(static_cast<unsigned>(blocks)), dim3(T::kThreads), 0,
+                     stream, p, tiles_j);
+  return launch_status("moe_f32_grouped_gemm");
+}
+
+// The tile.  At 8192 rows over 32 experts, H 1024, I 512 (us; the straight
+// 32x32-per-wave kernel this replaced in brackets): row-grouped GEMMs on 64x64
+// up 193, down 103, their input gradients 108 and 198 (1020, 506, 310, 564);
+// on 128x128 with 8 waves 194, 102, 150, 199, and at smaller calls (H 256,
+// I 128, 128 rows per expert) 24 against 12: a 64x64 tile everywhere.  Weight
+// gradients, whose reduction is an expert's rows: 157 and 83 on 128x128 with 8
+// waves against 177 and 93 on 64x64 (290, 149), as long as those tiles fill
+// the chip.  A weight gradient of few tiles and a long reduction (a router's:
+// 32 x 1024 outputs over 2048 rows) is a serial chain on 16 blocks: 26 with
+// its k-tiles split over the waves of 32x32 tiles against 76 (112); the row-
+// grouped GEMMs keep one chain per output, whose sums are the router's logits.
+template <int LA, int LB>
+int f32_launch(const F32Gemm& p, hipStream_t stream) {
+  const int cus = device_cus(current_device());
+  auto tiles = [&](int bm, int bn) {  // of a weight gradient
+    return static_cast<int64_t>(p.G) * ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
+  };
+  if (p.mode == 1) {
+    if (tiles(128, 128) >= cus) return f32_launch_tile<LA, LB, F32Tile<2, 1, 2, 4, 1, 16>>(p, stream);
+    if (tiles(64, 64) < cus / 2 && p.K / p.G >= 512) return f32_launch_tile<LA, LB, F32Tile<1, 1, 1, 1, 4, 16>>(p, stream);
+  }
+  return f32_launch_tile<LA, LB, F32Tile<1, 1, 2, 2, 1, 16>>(p, stream);
 }
 
 // act[r, c] = silu(pre[r, c]) * pre[r, I + c] for the rows below n_valid.
@@ -228,15 +457,17 @@ extern "C" int moe_f32_grouped_gemm(const float* A, const float* B, const int32_
               "f32 grouped gemm: null pointer");
   F32Gemm p{A, B, C, offs, static_cast<int>(G), mode, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K),
             sAi, sAr, sBr, sBj, sCi, sCj, sBg, sCg, accumulate ? 1 : 0};
-  const int tiles_j = static_cast<int>((N + 31) / 32);
-  // mode 0: every group's rows in 32-row tiles, at most M / 32 + G of them
-  const int64_t tiles_i = mode == 0 ? (M + 31) / 32 + G : G * ((M + 31) / 32);
-  const int64_t ntiles = tiles_i * tiles_j;
-  const int64_t blocks = (ntiles + kF32Waves - 1) / kF32Waves;
-  MOE_REQUIRE(blocks < (1ll << 31), MOE_ERR_UNSUPPORTED, "f32 grouped gemm: too many tiles");
-  hipLaunchKernelGGL(f32_grouped_gemm_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kF32Waves * kWave), 0,
-                     as_stream(stream), p, tiles_j, ntiles);
-  return launch_status("moe_f32_grouped_gemm");
+  const bool a16 = aligned16(A), b16 = aligned16(B);
+  const bool b_out = b16 && sBj == 1 && sBr % 4 == 0 && N % 4 == 0 && (mode == 1 || sBg % 4 == 0);
+  hipStream_t st = as_stream(stream);
+  if (mode == 0) {
+    const bool a_r = a16 && sAr == 1 && sAi % 4 == 0 && K % 4 == 0;
+    if (a_r && b16 && sBr == 1 && sBj % 4 == 0 && sBg % 4 == 0) return f32_launch<kAlongR, kAlongR>(p, st);
+    if (a_r && b_out) return f32_launch<kAlongR, kAlongOut>(p, st);
+  } else if (a16 && sAi == 1 && sAr % 4 == 0 && M % 4 == 0 && b_out) {
+    return f32_launch<kAlongOut, kAlongOut>(p, st);
+  }
+  return f32_launch<kScalar, kScalar>(p, st);
 }
 
 extern "C" int moe_f32_swiglu_fwd(const float* pre, float* act, const int32_t* offsets, int64_t num_buckets,

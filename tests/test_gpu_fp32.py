@@ -13,7 +13,7 @@ import torch
 
 from conftest import close_bf16, routing_check
 from oracle import moe_oracle as O
-from parallel_amd import ops, register_experts_implementation
+from parallel_amd import _lib, ops, register_experts_implementation
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -180,3 +180,60 @@ def test_fp32_transformers_block_runs_on_the_plugin():
     want.square().sum().backward()
     close_f32(xg.grad, xr.grad, "fp32 plugin block d_hidden")
     close_f32(block.experts.gate_up_proj.grad, ref_block.experts.gate_up_proj.grad, "fp32 plugin d_gate_up")
+
+
+def _strided(t, order):
+    """``t`` with its last two dimensions stored in the given order: "row" (last contiguous), "col", or
+    "wide" (no contiguous dimension)."""
+    if order == "row":
+        return t.contiguous()
+    if order == "col":
+        return t.transpose(-1, -2).contiguous().transpose(-1, -2)
+    wide = torch.zeros(*t.shape[:-1], 2 * t.shape[-1], dtype=t.dtype, device=t.device)
+    wide[..., ::2] = t
+    return wide[..., ::2]
+
+
+# (mode, rows per group, M or 0, N, K or 0, order of A(i, r), order of B(r, j)): both 16-byte load paths and
+# the strided one, sizes off the multiples of 4 and of the tiles, groups at the 64-row tile's edge, the wide
+# weight-gradient tile (at least one per compute unit) and the split reduction of a small long one.
+F32_GEMMS = [
+    (0, [63, 0, 64, 65, 1, 33], 0, 132, 68, "row", "col"),
+    (0, [63, 0, 64, 65, 1, 33], 0, 132, 68, "row", "row"),
+    (0, [63, 0, 64, 65, 1, 33], 0, 131, 67, "row", "col"),
+    (0, [5, 200], 0, 70, 36, "wide", "wide"),
+    (1, [63, 0, 17, 65, 1, 33], 132, 68, 0, "col", "row"),
+    (1, [63, 0, 17, 65, 1, 33], 131, 67, 0, "row", "wide"),
+    (1, [40, 0, 3, 70], 1024, 1028, 0, "col", "row"),
+    (1, [1501], 36, 100, 0, "col", "row"),
+    (1, [1501], 33, 99, 0, "row", "col"),
+]
+
+
+@pytest.mark.parametrize("accumulate", [0, 1])
+@pytest.mark.parametrize("case", range(len(F32_GEMMS)))
+def test_f32_grouped_gemm_is_exact_on_integers(case, accumulate):
+    """Integers of up to 4 bits: every sum is exact in fp32, whatever the tile, layout and order."""
+    mode, rows, M, N, K, order_a, order_b = F32_GEMMS[case]
+    g = torch.Generator().manual_seed(case)
+    G, R = len(rows), sum(rows)
+    offs = torch.cumsum(torch.tensor(rows), 0).to(torch.int32).cuda()
+    M, K = (R, K) if mode == 0 else (M, R)
+
+    def ints(*shape):
+        return torch.randint(-8, 9, shape, generator=g).float().cuda()
+
+    A, B = _strided(ints(M, K), order_a), _strided(ints(*((G, K, N) if mode == 0 else (K, N))), order_b)
+    C = ints(*((M, N) if mode == 0 else (G, M, N)))
+    ref, lo = (C.double() if accumulate else torch.zeros_like(C, dtype=torch.float64)).cpu(), 0
+    for e, n in enumerate(rows):
+        a, b = A.cpu().double(), B.cpu().double()
+        if mode == 0:
+            ref[lo:lo + n] += a[lo:lo + n] @ b[e]
+        else:
+            ref[e] += a[:, lo:lo + n] @ b[lo:lo + n]
+        lo += n
+    _lib.call("moe_f32_grouped_gemm", A.data_ptr(), B.data_ptr(), offs.data_ptr(), G, mode, M, N, K, A.stride(0),
+              A.stride(1), B.stride(-2), B.stride(-1), B.stride(0) if mode == 0 else 0, C.data_ptr(), C.stride(-2),
+              C.stride(-1), C.stride(0) if mode == 1 else 0, accumulate, _lib.stream_of(C))
+    assert torch.equal(C.cpu().double(), ref)
