@@ -7,15 +7,19 @@
 // MG = groups partition the rows of the activation operand (variable M per
 // expert), KG = groups partition the reduction (variable K per expert).
 //
-// Tiling: WM x WN waves; each wave owns (BM/WM) x (BN/WN) of 32x32 MFMA
-// sub-tiles (v_mfma_f32_32x32x16_bf16, fp32 accumulators), its row sub-tiles
-// interleaved with the other wave rows'.  The expert GEMMs use 256-column
+// Tiling: WM x WN waves; each wave owns (BM/WM) x (BN/WN) of 32x32 sub-tiles,
+// its row sub-tiles interleaved with the other wave rows'.  The products are
+// v_mfma_f32_16x16x32_bf16 (four per sub-tile and 32 k, fp32 accumulators):
+// on random data these kernels run against the card's power limit, and this
+// shape reads and writes each accumulator once per 32 k where 32x32x16 does
+// once per 16 (65536 x 3072 x 4096 over 128 experts 1386 against 1528 us, the
+// same instruction time: on zeros both take 1125).  The expert GEMMs use 256-column
 // tiles of 64 to 320 rows, by the mean rows per expert, on 8 waves (two waves
 // per SIMD, one workgroup per CU); the small router GEMMs use 128x128 on 4
 // waves.  Operands move from HBM to LDS by DMA (buffer_load_dwordx4 ... lds,
-// no register staging) into a ring of 32- or 64-deep k-tiles (5 stages of 32
-// for 256x256 tiles) that fills the 160 KiB of LDS, so three or four k-tiles of loads are in flight while
-// one is multiplied; each wave fires its share of a k-tile's DMA between its
+// no register staging) into a ring of 32- or 64-deep k-tiles that fills the 160
+// KiB of LDS, so that 64 to 96 KiB of loads are in flight while one k-tile is
+// multiplied; each wave fires its share of a k-tile's DMA between its
 // MFMA groups.  At the roughly 256 rows per expert of a training step the
 // expert GEMMs sit near the ridge of the roofline (about 256 flop per weight
 // byte), and the weights stream from HBM only as fast as the bytes in flight
@@ -184,12 +188,10 @@ __device__ int2 kg_cost_split(const int32_t* offs, int G, int rows, int per_grou
 // Tile configurations: BK-deep k-tiles staged through a STAGES-deep LDS ring.
 // PIPE selects the k-loop:
 //   0  every wave reads its fragments, multiplies and fires its share of the
-//      DMA in each k-step (block barrier every second k-step);
-//   1  the same with the next 16-deep half step's fragments read while the
-//      current half step's MFMAs run (one barrier per k-step);
-//   2  ping-pong: the two waves of a SIMD take turns, one multiplying a k-step
-//      from registers while the other reads the next k-step's fragments and
-//      fires DMA (two barriers per k-step).
+//      DMA in each k-step (5-deep rings: block barrier every second k-step);
+//   1  ping-pong: the two waves of a SIMD take turns, one multiplying half a
+//      k-step from registers while the other reads the next half's fragments
+//      and fires DMA into a ring of single operand tiles.
 template <int BM_, int BN_, int BK_, int WM_, int WN_, int STAGES_, int PIPE_ = 0>
 struct TileCfg {
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, STAGES = STAGES_, PIPE = PIPE_;
@@ -206,16 +208,14 @@ using SlimTile = TileCfg<64, 256, 64, 2, 4, 4>;
 using MidTile = TileCfg<128, 256, 64, 2, 4, 3>;
 // Router GEMMs (N = E = 128): 80 KiB ring, 4 waves (two workgroups per CU).
 using SmallTile = TileCfg<128, 128, 32, 2, 2, 5>;
-// The 256x256 loop with the fragment reads of each 16-deep half step
-// overlapping the previous half step's MFMAs.
-using BigTileP = TileCfg<256, 256, 32, 2, 4, 5, 1>;
 // Experts of up to 320 rows in one m-tile: 320x256 tiles (five 32-row
 // sub-tiles per wave, 160 accumulator registers per lane), A staged as 384
 // rows, 4-deep ring of 40 KiB stages.
 using WideTile = TileCfg<320, 256, 32, 2, 4, 4>;
-// Ping-pong on 256x256 tiles: waves 0-3 (one per SIMD) own output columns
-// 0-127, waves 4-7 columns 128-255; wave w and wave w + 4 share a SIMD.
-using PingTile = TileCfg<256, 256, 32, 2, 4, 5, 2>;
+// Ping-pong on 256x256 tiles, 64-deep k-steps: waves 0-3 (one per SIMD) own
+// output columns 0-127, waves 4-7 columns 128-255; wave w and wave w + 4 share
+// a SIMD.  The ring holds five 32 KiB operand tiles.
+using PingTile = TileCfg<256, 256, 64, 2, 4, 5, 1>;
 
 // A wave-uniform pointer moved to scalar registers (buffer resources must be).
 template <class T>
@@ -281,13 +281,14 @@ template <int BK>
 __device__ __forceinline__ constexpr int kc_swizzle(int r) {
   return BK == 32 ? (r >> 2) & 3 : (r >> 1) & 7;
 }
-// A transpose-read pass reads 32 columns (4 chunks) of 4 consecutive k-rows:
-// k-row kk & 3 selects the 64-byte bank quarter (needs >= 16 chunks per k-row).
-__device__ __forceinline__ constexpr int mc_swizzle(int kk) { return 4 * (kk & 3); }
+// A transpose-read pass reads 16 columns (2 chunks) of k-rows kk .. kk + 3 and
+// kk + 8 .. kk + 11: k-row kk & 3 selects the 64-byte bank quarter, bit 3 of kk
+// the half of it (needs >= 16 chunks per k-row).
+__device__ __forceinline__ constexpr int mc_swizzle(int kk) { return 4 * (kk & 3) | 2 * ((kk >> 3) & 1); }
 // Epilogue staging of a wave's 32 x 64 bf16 pass (128-byte rows): chunk cc of
-// row r at slot cc ^ stg_swizzle(r), its 8-byte halves exchanged when bit 4 of
-// r is set; the 8-byte writes, the row reads and the SwiGLU gate/up reads are
-// then each on distinct banks.
+// row r at slot cc ^ stg_swizzle(r); the 8-byte writes (16 rows, both halves of
+// a chunk), the row reads and the SwiGLU gate/up reads are each on distinct
+// banks.
 __device__ __forceinline__ constexpr int stg_swizzle(int r) { return (((r >> 1) & 1) << 2) | ((r >> 2) & 3); }
 
 // Store instructions per wave per epilogue (all issued unconditionally).
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   constexpr int NI_A = A_BYTES / 1024, NI_B = B_BYTES / 1024;  // DMA instructions per k-tile
   // Ping-pong: the DMA of a k-tile is split by operand between the wave
   // groups (waves 0-3 fire A, waves 4-7 fire B), LPW instructions per wave.
-  constexpr bool PING = CFG::PIPE == 2;
+  constexpr bool PING = CFG::PIPE == 1;
   constexpr int LPW_A = PING ? 0 : NI_A / NWAVES, LPW_B = PING ? 0 : NI_B / NWAVES;  // ... per wave and operand
   constexpr int LPW = PING ? NI_A / 4 : LPW_A + LPW_B;
   // Barrier cadence.  With a 5-deep ring the DMA runs LEAD = 3 k-steps ahead
@@ -329,22 +330,11 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   // barrier.  Shallower rings synchronise every step with the DMA
   // STAGES - 1 steps ahead.
   //
-  // The pipelined loop (CFG::PIPE) keeps the 5-deep ring with the DMA 3
-  // k-steps ahead but synchronises once per k-step, in its middle: iteration
-  // c reads the second half step of k-tile c, multiplies the first, waits for
-  // k-tile c + 1 and synchronises, reads the first half step of c + 1 and
-  // multiplies the second half of c.  Half of the DMA of k-tile c + 3 is
-  // fired among each half's MFMAs.  Its stage last held k-tile c - 2, whose
-  // fragments every wave had consumed (waited for) before the barrier in the
-  // middle of iteration c - 1, and both halves of iteration c come after that
-  // barrier.  The DMA younger than the k-tile waited for is k-tile c + 2 and
-  // the first half of c + 3.
-  constexpr bool PIPE = CFG::PIPE == 1;
-  constexpr bool PAIR = STAGES == 5 && !PIPE && !PING;
-  constexpr int LEAD = (PAIR || PIPE || PING) ? STAGES - 2 : STAGES - 1;
-  // DMA younger than the k-tile waited for
-  constexpr int WAIT = PING ? 2 * LPW : PIPE ? LPW + LPW / 2 : PAIR ? LPW : (STAGES - 2) * LPW;
-  constexpr int RELAX = (PAIR || PIPE || PING) ? 2 : STAGES - 1;  // waits that an epilogue's stores precede
+  // (The ping-pong loop's schedule is written down at the loop.)
+  constexpr bool PAIR = STAGES == 5 && !PING;
+  constexpr int LEAD = PAIR ? STAGES - 2 : STAGES - 1;
+  constexpr int WAIT = PAIR ? LPW : (STAGES - 2) * LPW;  // DMA younger than the k-tile waited for
+  constexpr int RELAX = PING ? 1 : PAIR ? 2 : STAGES - 1;  // waits that an epilogue's stores precede
   constexpr int NST = epilogue_stores<EPI, WTM, SM, SN>();
   constexpr int SLOT = 32 * 64 * 2;  // staging bytes per wave (one 32-row x 64-column pass)
   static_assert(BK == 32 || BK == 64, "swizzles and DMA mapping cover 32- and 64-deep k-tiles");
@@ -352,13 +342,13 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   constexpr int CPR = BK / 8;     // 16-byte chunks per K-contiguous row
   constexpr int RPI = 64 / CPR;   // K-contiguous rows per DMA instruction
   static_assert(WTM % 32 == 0 && WTN == 64, "wave tiles are whole 32x32 sub-tiles, 64 columns wide");
-  static_assert(!PIPE || (STAGES == 5 && LPW % 2 == 0 && BK == 32), "the pipelined loop's stage and DMA schedule");
-  // (The weight gradients keep the paired-barrier loop: on ping-pong they
-  // measured 175 against 159 us (C2 down_wgrad) and 1906 against 1864 us
-  // (C5 up_wgrad), the same at C4.)
-  static_assert(!PING || (MODE == MODE_MG && STAGES == 5 && BK == 32 && NWAVES == 8 && WM == 2 && NI_A == NI_B &&
-                          NI_A % 4 == 0),
-                "the ping-pong loop's wave groups, stage and DMA schedule");
+  // (The weight gradients keep the paired-barrier loop: their tiles are a few
+  // k-steps each, and their operands' rows are whole lines already.  On the
+  // ping-pong loop the up projection's took 631 against 494 us at 512 rows per
+  // expert, 373 against 290 at 256.)
+  static_assert(!PING || (MODE == MODE_MG && STAGES == 5 && BK == 64 && NWAVES == 8 && WM == 2 && WN == 4 && NI_A == NI_B &&
+                          NI_A % 8 == 0),
+                "the ping-pong loop's wave groups, ring and DMA schedule");
   static_assert(PING || (NI_A % NWAVES == 0 && NI_B % NWAVES == 0), "DMA instructions of each operand split evenly over waves");
   static_assert(EPI != EPI_SWIGLU_FWD || (SN % 2 == 0), "SwiGLU forward pairs gate/up sub-tiles");
   static_assert(STAGES >= 2 && STAGES <= 5, "ring depth");
@@ -367,7 +357,7 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   static_assert(A_KC || BM >= 128, "transpose-read swizzle needs >= 16 chunks per k-row");
   static_assert(B_KC || BN >= 128, "transpose-read swizzle needs >= 16 chunks per k-row");
 
-  __shared__ __attribute__((aligned(1024))) char ring[STAGES * STAGE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char ring[STAGES * (PING ? A_BYTES : STAGE_BYTES)];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -378,8 +368,7 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   // 2 grp + 1; its four waves sit on the four SIMDs.
   const int grp = wave >> 2, w4 = wave & 3;
   const int wm = PING ? (w4 >> 1) : wave / WN, wn = PING ? grp * 2 + (w4 & 1) : wave % WN;
-  const int l32 = lane & 31;
-  const int khalf = lane >> 5;
+  const int i16 = lane & 15, q16 = lane >> 4;  // the lane's row (column) and k-group in an MFMA operand
 
   // ------------------------------------------------------ this block's tiles
   const int nbx = gridDim.x / kNumXcd;  // the grid is a multiple of kNumXcd
@@ -584,20 +573,18 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
     if constexpr (PING) return w4 * LPW + j;
     return is_a ? wave * LPW_A + j : wave * LPW_B + (j - LPW_A);
   };
-  int dma_lds[LPW], dma_k[LPW], dma_col[LPW];
+  int dma_lds[LPW], dma_k[LPW];
 #pragma unroll
   for (int j = 0; j < LPW; ++j) {
     bool is_a;
     const int li = slot_inst(j, is_a);
-    dma_lds[j] = __builtin_amdgcn_readfirstlane((is_a ? 0 : A_BYTES) + li * 1024);
-    dma_col[j] = 0;
+    dma_lds[j] = __builtin_amdgcn_readfirstlane((is_a || PING ? 0 : A_BYTES) + li * 1024);
     if (is_a ? A_KC : B_KC) {
       const int r = li * RPI + lane / CPR;
       dma_k[j] = ((lane % CPR) ^ kc_swizzle<BK>(r)) * 8;
     } else {
       const int cpk = (is_a ? BM : BN) / 8;  // 16-byte chunks per k-row
       dma_k[j] = li * (64 / cpk) + lane / cpk;
-      dma_col[j] = ((lane % cpk) ^ mc_swizzle(dma_k[j])) * 8;  // first of the chunk's 8 columns
     }
   }
 
@@ -666,7 +653,8 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
         }
         dma_pre[j2] = ok ? row_bytes + static_cast<uint32_t>(c) * 16u + static_cast<uint32_t>(dt.k_begin) * 2u : kOOB;
       } else {
-        const int col = (is_a ? dt.m0 : dt.n0) + dma_col[j2];
+        // first of the chunk's 8 columns
+        const int col = (is_a ? dt.m0 : dt.n0) + ((lane % ((is_a ? BM : BN) / 8)) ^ mc_swizzle(dma_k[j2])) * 8;
         const uint32_t ld = is_a ? lda2 : ldb2;
         dma_pre[j2] = col < (is_a ? p.M : p.N)
                           ? static_cast<uint32_t>(mc_row0 + dma_k[j2]) * ld + static_cast<uint32_t>(col) * 2u
@@ -674,18 +662,21 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
       }
     }
   };
-  // The DMA of the cursor's next k-step into ring stage `st`, in three parts:
-  // dma_prepare computes the per-lane offsets of the wave's LPW slots,
-  // dma_fire(j) issues slot j, dma_advance moves the cursor.  The compute
-  // loop fires the slots between its MFMA groups, so that the texture unit
-  // works through the k-step's DMA while the matrix cores run instead of
-  // taking every wave's burst at once.  Every k-step fires exactly LPW
+  // The DMA of the cursor's next k-step into the ring, in three parts:
+  // dma_prepare fixes the stage and the k-step, dma_fire(j) computes slot j's
+  // offset and issues it, dma_advance moves the cursor.  The compute loop
+  // fires the slots between its MFMA groups (ping-pong: its fragment reads),
+  // so that the texture unit works through the k-step's DMA while the matrix
+  // cores run instead of taking every wave's burst at once; the offsets live
+  // in registers only around their own load.  Every k-step fires exactly LPW
   // instructions per wave.
-  uint32_t doff[LPW], dlds[LPW];
+  uint32_t dma_at = 0;
+  int dma_k0 = 0, dma_left = 0;  // the k-step's first k (or k-row) in the tile, and how many are left from there
   u32x4_t ra, rb;
-  auto dma_prepare = [&](int st) __attribute__((always_inline)) {
-    const int k0 = dk * BK;
-    const int k_left = dt.kred - k0;  // k (K-contiguous) or k-rows (M/N-contiguous) left in the tile
+  // `at`: LDS byte offset of the stage (ping-pong: of the operand tile's slot).
+  auto dma_prepare = [&](int at) __attribute__((always_inline)) {
+    dma_k0 = dk * BK;
+    dma_left = dt.kred - dma_k0;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       if constexpr (PING) {
@@ -697,29 +688,21 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
         rb[w] = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(rsB[w]));
       }
     }
-    const uint32_t stage_lds = lds_address(ring) + st * STAGE_BYTES;
-#pragma unroll
-    for (int j = 0; j < LPW; ++j) {
-      const bool is_a = slot_is_a(j);
-      const uint32_t step = (is_a ? A_KC : B_KC) ? 2u : (is_a ? lda2 : ldb2);
-      // Past the last tile dma_pre is kOOB and stays out of range (the
-      // added offset is below the 2 GiB operand limit).
-      doff[j] = dma_k[j] < k_left ? dma_pre[j] + static_cast<uint32_t>(k0) * step : kOOB;
-      dlds[j] = __builtin_amdgcn_readfirstlane(stage_lds + dma_lds[j]);
-    }
+    dma_at = lds_address(ring) + at;
   };
   auto dma_fire = [&](int j) __attribute__((always_inline)) {
-    if constexpr (PING) {
-      dma16(ra, doff[j], dlds[j]);
-    } else {
-      dma16(j < LPW_A ? ra : rb, doff[j], dlds[j]);
-    }
+    const bool is_a = slot_is_a(j);
+    const uint32_t step = (is_a ? A_KC : B_KC) ? 2u : (is_a ? lda2 : ldb2);
+    // Past the last tile dma_pre is kOOB and stays out of range (the added
+    // offset is below the 2 GiB operand limit).
+    const uint32_t off = dma_k[j] < dma_left ? dma_pre[j] + static_cast<uint32_t>(dma_k0) * step : kOOB;
+    dma16(PING || j < LPW_A ? ra : rb, off, __builtin_amdgcn_readfirstlane(dma_at + dma_lds[j]));
   };
   auto dma_advance = [&]() __attribute__((always_inline)) {
     if (dj < ntiles && ++dk == dt.nk) dma_seek(dj + 1);
   };
-  auto dma_issue = [&](int st) __attribute__((always_inline)) {
-    dma_prepare(st);
+  auto dma_issue = [&](int at) __attribute__((always_inline)) {
+    dma_prepare(at);
 #pragma unroll
     for (int j = 0; j < LPW; ++j) dma_fire(j);
     dma_advance();
@@ -731,87 +714,100 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   // partly filled tile spread over all waves (and SIMDs).  Its SN column
   // sub-tiles are contiguous: columns wn*WTN + 32 j.
   //
-  // Each lane's byte offset within a stage is precomputed per fragment class;
-  // a fragment address is the stage base plus a lane offset plus a constant.
-  // K-contiguous [R rows][CPR chunks]: lane reads row (tile_row + l32), chunk
-  // 2 ks + khalf; fragment rows start on 32-row boundaries, so the swizzle
-  // of row tile_row + l32 is that of l32.
+  // A fragment is 16 rows (columns) x 32 k, lane l holding row l % 16, k
+  // 8 (l / 16) .. + 7; a 32-row sub-tile is two of them.  Each lane's byte
+  // offset within a stage is precomputed per fragment class; a fragment
+  // address is the stage base plus a lane offset plus a constant.
+  // K-contiguous [R rows][CPR chunks]: lane reads row (tile_row + i16), chunk
+  // 4 ks + q16; fragment rows start on 16-row boundaries, so the swizzle of
+  // row tile_row + i16 is that of i16.
+  constexpr int KS = BK / 32;
   auto sub_row = [&](int i) { return (wm + WM * i) * 32; };
-  int a_kc[BK / 16], b_kc[BK / 16];
+  constexpr int B_OFF = PING ? 0 : A_BYTES;  // B's offset from the base its fragments are read with
+  int a_kc[KS], b_kc[KS];
 #pragma unroll
-  for (int ks = 0; ks < BK / 16; ++ks) {
-    const int lane_off = l32 * RB + (((2 * ks + khalf) ^ kc_swizzle<BK>(l32)) << 4);
+  for (int ks = 0; ks < KS; ++ks) {
+    const int lane_off = i16 * RB + (((4 * ks + q16) ^ kc_swizzle<BK>(i16)) << 4);
     a_kc[ks] = sub_row(0) * RB + lane_off;
-    b_kc[ks] = A_BYTES + wn * WTN * RB + lane_off;
+    b_kc[ks] = B_OFF + wn * WTN * RB + lane_off;
   }
-  // M/N-contiguous [BK k-rows][R cols] (transpose reads): lane = 16 q + i reads
-  // k-rows 16 ks + 8 (q/2) + 4 h + i/4 and columns tile_col + 16 (q%2) + 4 (i%4).
-  // The swizzle depends only on k-row & 3 == i/4, so each 32-column sub-tile
-  // has one lane offset; ks and h add constants.
-  const int q16 = lane >> 4, i16 = lane & 15;
-  const int tr_krow = 8 * (q16 >> 1) + (i16 >> 2);
-  const int tr_col = 16 * (q16 & 1) + 4 * (i16 & 3);
-  const int half8 = ((tr_col >> 2) & 1) << 3;
-  int a_mc[SM], b_mc[SN];
+  // M/N-contiguous [BK k-rows][R cols] (transpose reads): lane reads k-rows
+  // 32 ks + 8 q16 + 4 h + i16 / 4 and columns tile_col + 4 (i16 % 4).  The
+  // swizzle depends only on bits 0, 1 and 3 of the k-row, so each 16-column
+  // fragment has one lane offset; ks and h add constants.
+  const int tr_krow = 8 * q16 + (i16 >> 2);
+  const int tr_col = 4 * (i16 & 3);
+  const int half8 = (i16 & 1) << 3;
+  int a_mc[2 * SM], b_mc[2 * SN];
 #pragma unroll
-  for (int t = 0; t < SM; ++t)
-    a_mc[t] = tr_krow * BM * 2 + ((((sub_row(t) + tr_col) >> 3) ^ mc_swizzle(tr_krow)) << 4) + half8;
+  for (int t = 0; t < 2 * SM; ++t)
+    a_mc[t] = tr_krow * BM * 2 + ((((sub_row(t / 2) + 16 * (t % 2) + tr_col) >> 3) ^ mc_swizzle(tr_krow)) << 4) + half8;
 #pragma unroll
-  for (int t = 0; t < SN; ++t)
-    b_mc[t] = A_BYTES + tr_krow * BN * 2 + ((((wn * WTN + 32 * t + tr_col) >> 3) ^ mc_swizzle(tr_krow)) << 4) + half8;
+  for (int t = 0; t < 2 * SN; ++t)
+    b_mc[t] = B_OFF + tr_krow * BN * 2 + ((((wn * WTN + 16 * t + tr_col) >> 3) ^ mc_swizzle(tr_krow)) << 4) + half8;
+  auto tr_read = [](const char* at, int row_bytes) __attribute__((always_inline)) {
+    const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)at);
+    const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(at + 4 * row_bytes));
+    return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  // Fragment t of A (sub-tile t / 2's rows 16 (t % 2) ..) or of B (columns
+  // 16 t .. of the wave's) for k's 32 ks .. of the k-tile at `base`.
+  auto read_a = [&](const char* base, int ks, int t) __attribute__((always_inline)) {
+    if constexpr (A_KC) {
+      return *reinterpret_cast<const bf16x8_t*>(base + a_kc[ks] + ((t / 2) * WM * 32 + (t % 2) * 16) * RB);
+    } else {
+      return tr_read(base + a_mc[t] + 32 * ks * BM * 2, BM * 2);
+    }
+  };
+  auto read_b = [&](const char* base, int ks, int t) __attribute__((always_inline)) {
+    if constexpr (B_KC) {
+      return *reinterpret_cast<const bf16x8_t*>(base + b_kc[ks] + t * 16 * RB);
+    } else {
+      return tr_read(base + b_mc[t] + 32 * ks * BN * 2, BN * 2);
+    }
+  };
 
-  f32x16_t acc[SM][SN];
+  // acc[2 i + h][t]: rows 16 h .. of row sub-tile i, columns 16 t .. of the wave's.
+  f32x4_t acc[2 * SM][2 * SN];
   auto zero_acc = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < SM; ++i)
+    for (int i = 0; i < 2 * SM; ++i)
 #pragma unroll
-      for (int j = 0; j < SN; ++j)
+      for (int j = 0; j < 2 * SN; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  };
+  // Operands swapped: the result holds C^T fragments, so each lane owns one
+  // output row and runs of 4 consecutive output columns.
+  auto mfma_row = [&](int i, const bf16x8_t& a, const bf16x8_t (&b)[2 * SN]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    for (int j = 0; j < 2 * SN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a, acc[i][j], 0, 0, 0);
   };
 
   // One k-tile of MFMAs over the first `na` row sub-tiles (the others hold no
   // rows of this tile; `na` is wave-uniform, so the guards are scalar
   // branches), with the prepared DMA slots fired between the MFMA groups:
-  // slot s after group (ks, i) = s * (BK / 16) SM / LPW.
+  // slot s after group (ks, i) = s * KS SM / LPW.  The next row sub-tile's
+  // fragments are read before the current one's MFMAs.
   auto compute = [&](int na, const char* stage) __attribute__((always_inline)) {
 #pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      bf16x8_t af[SM], bfr[SN];
+    for (int ks = 0; ks < KS; ++ks) {
+      bf16x8_t af[2][2], bfr[2 * SN];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) af[0][h] = read_a(stage, ks, h);
+#pragma unroll
+      for (int j = 0; j < 2 * SN; ++j) bfr[j] = read_b(stage, ks, j);
 #pragma unroll
       for (int i = 0; i < SM; ++i) {
-        if constexpr (A_KC) {
-          af[i] = *reinterpret_cast<const bf16x8_t*>(stage + a_kc[ks] + i * WM * 32 * RB);
-        } else {
-          const char* q = stage + a_mc[i] + 16 * ks * BM * 2;
-          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)q);
-          const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(q + 4 * BM * 2));
-          af[i] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        }
-      }
+        if (i + 1 < SM) {
 #pragma unroll
-      for (int j = 0; j < SN; ++j) {
-        if constexpr (B_KC) {
-          bfr[j] = *reinterpret_cast<const bf16x8_t*>(stage + b_kc[ks] + j * 32 * RB);
-        } else {
-          const char* q = stage + b_mc[j] + 16 * ks * BN * 2;
-          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)q);
-          const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(q + 4 * BN * 2));
-          bfr[j] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+          for (int h = 0; h < 2; ++h) af[(i + 1) & 1][h] = read_a(stage, ks, 2 * (i + 1) + h);
         }
-      }
-#pragma unroll
-      for (int i = 0; i < SM; ++i) {
         if (i == 0 || i < na) {
 #pragma unroll
-          for (int j = 0; j < SN; ++j)
-            // Operands swapped: the result holds C^T fragments, so each lane
-            // owns one output row and runs of 4 consecutive output columns.
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[j], af[i], acc[i][j], 0, 0, 0);
+          for (int h = 0; h < 2; ++h) mfma_row(2 * i + h, af[i & 1][h], bfr);
         }
 #pragma unroll
         for (int s2 = 0; s2 < LPW; ++s2) {
-          if ((s2 * (BK / 16) * SM) / LPW == ks * SM + i) {
+          if ((s2 * KS * SM) / LPW == ks * SM + i) {
             __builtin_amdgcn_sched_barrier(0);
             dma_fire(s2);
             __builtin_amdgcn_sched_barrier(0);
@@ -831,8 +827,8 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   };
 
   // ------------------------------------------------------ epilogue
-  // Lane owns output row  m0 + sub_row(i) + l32  and columns
-  // wcol0 + j*32 + 8*q + 4*khalf + {0..3} holding acc[i][j][4q..4q+3].
+  // Lane owns output rows m0 + sub_row(i) + 16 h + i16 and columns
+  // wcol0 + 16 t + 4 q16 + {0..3}, holding acc[2 i + h][t].
   // This wave's staging slot (no other wave touches it) in the ring stage
   // that the compute cursor has just finished: no DMA targets that stage
   // before the next block barrier, and a barrier before the epilogue
@@ -840,8 +836,7 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   // stream starts (empty weight-gradient groups) use the last stage, which
   // the prologue DMA leaves alone and no k-step fills before the first
   // barrier.
-  char* slot = ring + (STAGES - 1) * STAGE_BYTES + wave * SLOT;
-  auto swap_halves = [](uint4 v) { return make_uint4(v.z, v.w, v.x, v.y); };
+  char* slot = ring + (STAGES - 1) * (PING ? A_BYTES : STAGE_BYTES) + wave * SLOT;
   auto to_f32x8 = [](uint4 v, float* f) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -872,18 +867,16 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
     if (EPI == EPI_F32 || (EPI == EPI_WGRAD && p.ldp)) {
       // fp32 outputs (split-K partials, fp32 weight gradients): direct 16-byte stores.
 #pragma unroll
-      for (int i = 0; i < SM; ++i) {
-        const int row = t.m0 + sub_row(i) + l32;
+      for (int i = 0; i < 2 * SM; ++i) {
+        const int row = t.m0 + sub_row(i / 2) + 16 * (i % 2) + i16;
 #pragma unroll
-        for (int j = 0; j < SN; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int col = wcol0 + j * 32 + 8 * q + 4 * khalf;
+        for (int j = 0; j < 2 * SN; ++j) {
+            const int col = wcol0 + j * 16 + 4 * q16;
             const uint32_t off = (row < row_limit && col < p.N)
                                      ? (static_cast<uint32_t>(row) * static_cast<uint32_t>(p.ldc) +
                                         static_cast<uint32_t>(col)) * 4u
                                      : kOOB;
-            float4 v = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+            float4 v = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
             if (EPI == EPI_WGRAD && p.accumulate) {
               const uint4 o = load16(rsC, off);
               v.x += __uint_as_float(o.x);
@@ -904,8 +897,8 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
     }
     // bf16 outputs go through this wave's LDS slot one 32-row pass at a time,
     // so that every store is 16 bytes per lane over whole 128-byte row segments.
-    const int stg_lane = l32 * 128 + ((khalf ^ ((l32 >> 4) & 1)) << 3);
-    const int stg_swz = stg_swizzle(l32);
+    const int stg_lane = i16 * 128 + ((q16 & 1) << 3);
+    const int stg_swz = stg_swizzle(i16);  // (row 16 + i16 has the same)
     const int rr8 = lane >> 3, c8 = lane & 7;  // row-read lane mapping: row 8n + rr8, chunk c8
     // One pass per 32 rows (row sub-tile i) and 64 columns (column group h:
     // sub-tiles 2h and 2h + 1).
@@ -930,14 +923,14 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
         }
       }
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj)
+      for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int j = 2 * h + jj;
+        for (int tt = 0; tt < 4; ++tt) {
+          const f32x4_t& c = acc[2 * i + hh][4 * h + tt];
           uint2 v;
-          v.x = pack_bf16x2(acc[i][j][4 * q], acc[i][j][4 * q + 1]);
-          v.y = pack_bf16x2(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-          *reinterpret_cast<uint2*>(slot + stg_lane + (((jj * 4 + q) ^ stg_swz) << 4)) = v;
+          v.x = pack_bf16x2(c[0], c[1]);
+          v.y = pack_bf16x2(c[2], c[3]);
+          *reinterpret_cast<uint2*>(slot + stg_lane + hh * 16 * 128 + (((2 * tt + (q16 >> 1)) ^ stg_swz) << 4)) = v;
         }
       if constexpr (EPI == EPI_SWIGLU_FWD) {
         // Slot columns 0-31 are gate, 32-63 the matching up columns.  A lane
@@ -950,12 +943,8 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
         for (int n = 0; n < 2; ++n) {
           const int r = 16 * n + rr;
           const int swz = stg_swizzle(r);
-          uint4 gv = *reinterpret_cast<const uint4*>(slot + r * 128 + ((c4 ^ swz) << 4));
-          uint4 uv = *reinterpret_cast<const uint4*>(slot + r * 128 + (((c4 + 4) ^ swz) << 4));
-          if (n & 1) {
-            gv = swap_halves(gv);
-            uv = swap_halves(uv);
-          }
+          const uint4 gv = *reinterpret_cast<const uint4*>(slot + r * 128 + ((c4 ^ swz) << 4));
+          const uint4 uv = *reinterpret_cast<const uint4*>(slot + r * 128 + (((c4 + 4) ^ swz) << 4));
           const int row = prow0 + r;
           const bool ok = row < row_limit && act_col < p.swiglu_I;
           float gf[8], uf[8], af[8];
@@ -978,7 +967,6 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
         for (int n = 0; n < 4; ++n) {
           const int r = 8 * n + rr8;
           uint4 v = *reinterpret_cast<const uint4*>(slot + r * 128 + ((c8 ^ stg_swizzle(r)) << 4));
-          if ((n >> 1) & 1) v = swap_halves(v);
           if constexpr (EPI == EPI_BF16) {
             store16(rsC, out_off[n], v);
           } else if constexpr (EPI == EPI_WGRAD) {
@@ -1048,227 +1036,160 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   // wait already covers them.
   relax = 0;
 #pragma unroll
-  for (int s = 0; s < LEAD; ++s) dma_issue(s);
-  int cstage = 0, dstage = LEAD;
-  int parity = 0;  // k-step count of the stream, mod 2
+  for (int s = 0; s < (PING ? 0 : LEAD); ++s) dma_issue(s * STAGE_BYTES);
   if constexpr (PING) {
-    // Ping-pong.  k-tile c of the block's stream sits in ring stage c % 5.
-    // Group 0 (waves 0-3) reads k-tile c's fragments in phase 2c and
-    // multiplies them in phase 2c + 1; group 1 (waves 4-7) reads them in
-    // phase 2c + 1 and multiplies in phase 2c + 2.  Each phase ends with a
-    // block barrier, so on every SIMD one wave issues MFMAs from registers
-    // while its partner reads fragments and fires DMA.
+    // Ping-pong over a ring of operand tiles.  A k-step is 64 deep, so that the
+    // DMA of a K-contiguous operand moves whole 128-byte lines (with 32-deep
+    // k-tiles the DMA of 65536 x 3072 x 4096 over 128 experts alone takes 1344
+    // us, the loop 1630; with 64-deep ones 1059, and 1386 the loop).  k-step
+    // c's B tile sits in ring slot 2c % 5, its A tile in slot (2c + 1) % 5.
     //
-    // DMA: k-tile c's A half is fired by group 0 in phase 2c - 6 and its B
-    // half by group 1 in phase 2c - 5 (the memory phases of k-tile c - 3),
-    // spread among the fragment reads.  Its stage last held k-tile c - 5,
-    // which group 1 read in phase 2c - 9.  Before group 0 reads k-tile c, the
-    // barrier ending phase 2c - 1 follows group 0's wait for its A half (end
-    // of its compute phase 2c - 1: its DMA of phases 2c - 4 and 2c - 2 may be
-    // in flight) and group 1's wait for its B half (end of its memory phase
-    // 2c - 1: its DMA of phases 2c - 3 and 2c - 1 may be in flight).
+    // A k-step is two halves of 32 k.  In phase 4c + 2h (h = 0, 1) group 0
+    // (waves 0-3) reads the fragments of half h, in phase 4c + 2h + 1 it
+    // multiplies them; group 1 (waves 4-7) runs one phase later.  Each phase
+    // ends with a block barrier, so on every SIMD one wave issues MFMAs from
+    // registers while its partner reads fragments and fires DMA.
     //
-    // A tile ending with k-tile c is written out by group 0 in phase 2c + 2
-    // and by group 1 in phase 2c + 3, each staging through its half of stage
-    // c % 5 (the A half for group 0, the B half for group 1), which the DMA
-    // refills only from phase 2c + 4 (A) and 2c + 5 (B).
-    constexpr int NR = (BK / 16) * (SM + SN);  // fragment reads per memory phase
-    bf16x8_t fa[BK / 16][SM], fb[BK / 16][SN];
-    auto read_frag = [&](const char* stage, int ks, int q) __attribute__((always_inline)) {
-      if (q < SM) {
-        const int i = q;
-        if constexpr (A_KC) {
-          fa[ks][i] = *reinterpret_cast<const bf16x8_t*>(stage + a_kc[ks] + i * WM * 32 * RB);
-        } else {
-          const char* a = stage + a_mc[i] + 16 * ks * BM * 2;
-          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)a);
-          const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(a + 4 * BM * 2));
-          fa[ks][i] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        }
+    // DMA: group 0 fires all of A tile c + 1 in phase 4c.  Its slot held B
+    // tile c - 1, read last in phase 4c - 1.  Group 1 fires B tile c + 2 in
+    // phases 4c + 1 and 4c + 3, half in each; its slot held A tile c - 1.
+    // Before group 0 reads k-step c + 1, the barrier ending phase 4c + 3
+    // follows group 0's wait for A tile c + 1 (all its DMA) and group 1's for B
+    // tile c + 1 (fired in phases 4c - 3 and 4c - 1: the LPW instructions of B
+    // tile c + 2 may be in flight).  The weights, which come from HBM, are thus
+    // fired 7 to 11 phases ahead, the activation rows, mostly in L2, 4.
+    //
+    // A tile ending with k-step c is written out by group 0 in phase 4c + 4 and
+    // by group 1 in phase 4c + 5, after the phase's DMA, so that the next waits
+    // leave the stores in flight.  Both stage through A tile c's slot: group 1
+    // refills it from phase 4c + 5 on, each wave 8 KiB of it, the first half of
+    // that in phase 4c + 5 and the second, where the wave stages, in phase
+    // 4c + 7.
+    constexpr int NF = 2 * (SM + SN);  // fragments of a half k-step
+    static_assert(LPW == 8 && SLOT == 4096, "group 1 stages in the half of its DMA share fired last");
+    bf16x8_t fa[2 * SM], fb[2 * SN];
+    auto read_frag = [&](const char* sa, const char* sb, int h, int n) __attribute__((always_inline)) {
+      if (n < 2 * SM) {
+        fa[n] = read_a(sa, h, n);
       } else {
-        const int j = q - SM;
-        if constexpr (B_KC) {
-          fb[ks][j] = *reinterpret_cast<const bf16x8_t*>(stage + b_kc[ks] + j * 32 * RB);
-        } else {
-          const char* b = stage + b_mc[j] + 16 * ks * BN * 2;
-          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)b);
-          const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(b + 4 * BN * 2));
-          fb[ks][j] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        }
+        fb[n - 2 * SM] = read_b(sb, h, n - 2 * SM);
       }
     };
-    // This wave's half of k-tile 0 landed (its halves of k-tiles 1 and 2 are
-    // younger), then every wave's, via the barrier; group 1 then waits one
-    // phase.
-    wait_vmcnt<WAIT>();
+    auto fire_range = [&](int lo, int hi) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < LPW; ++j)
+        if (j >= lo && j < hi) dma_fire(j);
+    };
+    auto next2 = [](int slot5) { return slot5 >= 3 ? slot5 - 3 : slot5 + 2; };
+    // Row sub-tiles without rows of the tile skip their MFMAs (wave-uniform branches).
+    auto multiply = [&]() __attribute__((always_inline)) {
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int i = 0; i < SM; ++i)
+        if (i < n_act) {
+          mfma_row(2 * i, fa[2 * i], fb);
+          mfma_row(2 * i + 1, fa[2 * i + 1], fb);
+        }
+      __builtin_amdgcn_s_setprio(0);
+    };
+    // Prologue: A tile 0, B tiles 0 and 1.
+    int dslot = grp == 0 ? 1 : 0;
+    dma_issue(dslot * A_BYTES);
+    dslot = next2(dslot);
+    if (grp == 0) {
+      wait_vmcnt<0>();
+    } else {
+      dma_issue(dslot * A_BYTES);
+      dslot = next2(dslot);
+      wait_vmcnt<LPW>();
+    }
     barrier();
     if (grp == 1) barrier();
     bool pending = false;  // a finished tile waits for its epilogue
-    int pstage = 0;        // ... and stages through this stage's half
+    int pslot = 0;         // ... and stages through this slot
     Tile pt = ct;
+    int cb = 0;  // slot of the current B tile; A's is the next one
     for (;;) {
-      // ---- memory phase of k-tile c (the stream's k-tile at cstage)
+      const int ca = cb == 4 ? 0 : cb + 1;
+      const char* sa = ring + ca * A_BYTES;
+      const char* sb = ring + cb * A_BYTES;
+      // ---- memory phase of the first half
+      dma_prepare(dslot * A_BYTES);
+      dslot = next2(dslot);
       if (pending) {
         pending = false;
-        slot = ring + pstage * STAGE_BYTES + wave * SLOT;
+        fire_range(0, LPW / 2);
+        if (grp == 0) fire_range(LPW / 2, LPW);
+        slot = ring + pslot * A_BYTES + (grp == 0 ? w4 * SLOT : w4 * 2 * SLOT + SLOT);
         epilogue(pt);
         relax = RELAX;
         if (!compute_seek(cj + 1)) break;
-      }
-      const char* cur = ring + cstage * STAGE_BYTES;
-      dma_prepare(dstage);
 #pragma unroll
-      for (int ks = 0; ks < BK / 16; ++ks)
+        for (int n = 0; n < NF; ++n) read_frag(sa, sb, 0, n);
+      } else {
 #pragma unroll
-        for (int q = 0; q < SM + SN; ++q) {
-          read_frag(cur, ks, q);
-          const int r = ks * (SM + SN) + q;
+        for (int n = 0; n < NF; ++n) {
+          read_frag(sa, sb, 0, n);
 #pragma unroll
-          for (int s2 = 0; s2 < LPW; ++s2)
-            if (r == (s2 + 1) * NR / LPW - 1) {
+          for (int f = 0; f < LPW / 2; ++f)
+            if (n == (f + 1) * NF / (LPW / 2) - 1) {
               __builtin_amdgcn_sched_barrier(0);
-              dma_fire(s2);
+              dma_fire(f);
+              if (grp == 0) dma_fire(LPW / 2 + f);
               __builtin_amdgcn_sched_barrier(0);
             }
         }
+      }
+      wait_lgkmcnt0();  // the fragments are in registers
+      barrier();
+      multiply();
+      barrier();
+      // ---- memory phase of the second half
+#pragma unroll
+      for (int n = 0; n < NF; ++n) {
+        read_frag(sa, sb, 1, n);
+        if (grp == 1) {
+#pragma unroll
+          for (int f = 0; f < LPW / 2; ++f)
+            if (n == (f + 1) * NF / (LPW / 2) - 1) {
+              __builtin_amdgcn_sched_barrier(0);
+              dma_fire(LPW / 2 + f);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+      }
       dma_advance();
-      wait_lgkmcnt0();  // the fragments are in registers before the stage can be refilled
+      wait_lgkmcnt0();  // ... before the slots can be refilled
       const bool drain = relax > 0;
+      relax = 0;
       if (grp == 1) {
-        if (relax > 0) --relax;
         if (drain) {
-          wait_vmcnt<WAIT + NST>();
+          wait_vmcnt<LPW + NST>();
         } else {
-          wait_vmcnt<WAIT>();
+          wait_vmcnt<LPW>();
         }
       }
       barrier();
-      // ---- compute phase of k-tile c: row sub-tiles without rows of the
-      // tile skip their MFMAs (wave-uniform branches).
-#pragma unroll
-      for (int ks = 0; ks < BK / 16; ++ks)
-#pragma unroll
-        for (int i = 0; i < SM; ++i)
-          if (i < n_act) {
-#pragma unroll
-            for (int j = 0; j < SN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[ks][j], fa[ks][i], acc[i][j], 0, 0, 0);
-          }
+      multiply();
       if (grp == 0) {
-        const bool drain0 = relax > 0;
-        if (relax > 0) --relax;
-        if (drain0) {
-          wait_vmcnt<WAIT + NST>();
+        if (drain) {
+          wait_vmcnt<NST>();
         } else {
-          wait_vmcnt<WAIT>();
+          wait_vmcnt<0>();
         }
       }
       barrier();
-      const int done_stage = cstage;
-      dstage = dstage + 1 == STAGES ? 0 : dstage + 1;
-      cstage = cstage + 1 == STAGES ? 0 : cstage + 1;
       if (++ck == ct.nk) {
         pending = true;
         pt = ct;
-        pstage = done_stage;
+        pslot = ca;
       }
+      cb = next2(cb);
     }
     if (grp == 0) barrier();
-  } else if constexpr (PIPE) {
-    // One wave per SIMD: the matrix pipe is fed only while this wave issues
-    // MFMAs, so the fragments of the next half step are read into the other
-    // register set while the current half step's MFMAs run, and the block
-    // barrier sits where the wave has just issued a run of MFMAs.
-    constexpr int HALF = LPW / 2;  // DMA instructions fired among one half step's MFMAs
-    bf16x8_t fa0[SM], fb0[SN], fa1[SM], fb1[SN];
-    auto read_half = [&](bf16x8_t (&fa)[SM], bf16x8_t (&fb)[SN], const char* stage, int ks)
-                         __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < SM; ++i) {
-        if constexpr (A_KC) {
-          fa[i] = *reinterpret_cast<const bf16x8_t*>(stage + a_kc[ks] + i * WM * 32 * RB);
-        } else {
-          const char* q = stage + a_mc[i] + 16 * ks * BM * 2;
-          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)q);
-          const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(q + 4 * BM * 2));
-          fa[i] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < SN; ++j) {
-        if constexpr (B_KC) {
-          fb[j] = *reinterpret_cast<const bf16x8_t*>(stage + b_kc[ks] + j * 32 * RB);
-        } else {
-          const char* q = stage + b_mc[j] + 16 * ks * BN * 2;
-          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)q);
-          const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(q + 4 * BN * 2));
-          fb[j] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        }
-      }
-    };
-    // One half step's MFMAs over the first `na` row sub-tiles, with DMA slots
-    // slot0 .. slot0 + HALF - 1 fired between the row groups.
-    auto mfma_half = [&](const bf16x8_t (&fa)[SM], const bf16x8_t (&fb)[SN], int na, int slot0)
-                         __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < SM; ++i) {
-        if (i < na) {
-#pragma unroll
-          for (int j = 0; j < SN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
-        }
-#pragma unroll
-        for (int s2 = 0; s2 < HALF; ++s2) {
-          if ((s2 * SM) / HALF == i) {
-            __builtin_amdgcn_sched_barrier(0);
-            dma_fire(slot0 + s2);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }
-      }
-    };
-    if (any) {
-      // k-tile 0 landed (all but k-tiles 1 and 2 of this wave's DMA), then everyone's.
-      wait_vmcnt<2 * LPW>();
-      barrier();
-      read_half(fa0, fb0, ring, 0);
-      for (;;) {
-        const char* cur = ring + cstage * STAGE_BYTES;
-        const int nstage = cstage + 1 == STAGES ? 0 : cstage + 1;
-        read_half(fa1, fb1, cur, 1);
-        dma_prepare(dstage);
-        __builtin_amdgcn_sched_barrier(0);
-        mfma_half(fa0, fb0, n_act, 0);
-        // k-tile c + 1 landed: this wave's DMA (all but the WAIT younger
-        // instructions, plus the last epilogue's stores while they drain),
-        // then every wave's, via the barrier.
-        const bool drain = relax > 0;
-        if (relax > 0) --relax;
-        if (drain) {
-          wait_vmcnt<WAIT + NST>();
-        } else {
-          wait_vmcnt<WAIT>();
-        }
-        barrier();
-        read_half(fa0, fb0, ring + nstage * STAGE_BYTES, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        mfma_half(fa1, fb1, n_act, HALF);
-        dma_advance();
-        dstage = dstage + 1 == STAGES ? 0 : dstage + 1;
-        cstage = nstage;
-        if (++ck == ct.nk) {
-          // Stage the tile through the ring stage of its last k-tile: after
-          // this barrier every wave has consumed its fragments, and the DMA
-          // reaches that stage only two barriers later.
-          slot = ring + (cstage == 0 ? STAGES - 1 : cstage - 1) * STAGE_BYTES + wave * SLOT;
-          barrier();
-          epilogue(ct);
-          relax = RELAX;
-          if (!compute_seek(cj + 1)) break;
-        }
-      }
-    }
   } else if (any) {
+    int cstage = 0, dstage = LEAD;
+    int parity = 0;  // k-step count of the stream, mod 2
     for (;;) {
       // k-tiles of this step (and, pairwise, the next) landed: this wave's
       // DMA (all but the WAIT younger instructions, plus the last epilogue's
@@ -1285,7 +1206,7 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
         barrier();
       }
       parity ^= 1;
-      dma_prepare(dstage);
+      dma_prepare(dstage * STAGE_BYTES);
       if (n_act > 0) {
         // Issue priority while the wave feeds its MFMAs, so that on a shared
         // SIMD the wave with matrix work ready goes before the other wave's
@@ -1371,12 +1292,12 @@ int launch(GemmParams& p, hipStream_t stream, const char* name) {
 
 // Bounds of launch_expert's rule, in mean rows per expert.
 constexpr int64_t kSlimMaxMeanRows = 32;
-constexpr int64_t kMidMaxMeanRows = 128;
+constexpr int64_t kMidMaxMeanRows = 112;
 constexpr int64_t kBigMaxMeanRows = 224;
 constexpr int64_t kWideMaxMeanRows = 288;
-constexpr int64_t kPingMinMeanRows = 448;
-// Weight rows of at least this many elements (8 KiB) keep the 32-deep k-tiles
-// up to kLongRowMaxMeanRows mean rows.
+constexpr int64_t kMidAgainMaxMeanRows = 352;
+// Weight rows of at least this many elements (8 KiB) keep the larger tiles
+// down to the fewest rows, up to kLongRowMaxMeanRows mean rows.
 constexpr int kLongRow = 4096;
 constexpr int64_t kLongRowMaxMeanRows = 64;
 
@@ -1384,53 +1305,43 @@ constexpr int64_t kLongRowMaxMeanRows = 64;
 // real counts stay on the device).  An expert that fits one m-tile streams its
 // weights through one CU's LDS per n-tile, so the tile is the smallest that
 // holds nearly every expert under uniform routing, which leaves the most LDS
-// for weights in flight; experts above it take further m-tiles.  The results
-// are the same bits for every tile.  Kernel times in us at H 2048, I 768, 128
-// experts, top-8 (up_fwd / down_fwd / down_dgrad with its SwiGLU pass /
-// up_dgrad), one box:
-//   mean rows   3 (T 48):   64-row tile 140 / 70 / 77 / 130, 128-row 143 / 74 /
-//                           82 / 129, 320-row (384x128 for down_dgrad) 170 / 98 /
-//                           112 / 136: 5.5 against 3.9-4.5 TB/s
-//              19 (T 301):  64-row 155 / 78 / 86 / 139, 320-row 173 / 94 / 114 / 142
-//              48 (T 768):  128-row 167 / 88 / 98 / 145, 64-row 188 / 95 / 97 / 157,
-//                           320-row 186 / 103 / 124 / 157
-//              96 (T 1531): 128-row 185 / 97 / 114 / 155, 256-row 198 / 108 / 126 /
-//                           162, 320-row 204 / 114 / 138 / 170
-//             156 (T 2500): 256-row 221 / 119 / 155 / 187, 128-row 236 / 124 / 145 /
-//                           209, 320-row 230 / 127 / 164 / 205
-//             219 (T 3500): 256-row 245 / 131 / 179 / 207, 320-row 265 / 141 / 190
-//                           (384x128) / 235, 128-row for down_dgrad 165
-//             256 (T 4096): 320-row 281 / 152 / - / 250, 256-row 307 / 160 / 229 /
-//                           267, down_dgrad 128-row 195 against 206 (384x128)
+// for weights in flight; experts above it take further m-tiles.  Every tile
+// adds an output's products in the same order: the results are the same bits.
+// Kernel times in us at H 2048, I 768, 128 experts, top-8 (up_fwd / down_fwd /
+// down_dgrad with its SwiGLU pass / up_dgrad; 64-, 128-, 320-row tiles and the
+// 256-row ping-pong one, timed in turn):
+//   mean rows      64-row             128-row            320-row            256-row
+//     3 (T 48)     154/ 70/ 78/130    156/ 71/ 79/130    173/ 89/ 89/129    172/ 87/103/153
+//    19 (T 301)    168/ 78/ 86/139    168/ 79/ 86/140    186/ 93/ 96/137    182/ 93/108/160
+//    48 (T 768)    198/ 95/ 97/160    182/ 88/ 98/147    197/103/110/154    188/101/117/173
+//    96 (T 1531)   216/109/118/182    197/ 98/117/157    214/113/130/173    204/108/132/186
+//   131 (T 2100)   242/127/145/217    218/117/147/194    232/122/148/185    217/114/146/197
+//   162 (T 2600)   267/138/169/240    240/123/146/203    243/126/163/206    226/117/156/199
+//   200 (T 3200)   309/164/193/279    253/129/156/215    260/134/178/232    235/122/168/212
+//   256 (T 4096)   363/202/229/338    289/152/191/259    281/148/205/256    297/151/222/283
+//   312 (T 5000)   407/227/259/395    322/170/219/299    353/201/222/336    333/180/217/338
 // Narrow outputs (at most 1024 columns: down_dgrad at I 768) have few n-tiles,
 // and the 128-row tile's finer grid keeps winning up to kWideMaxMeanRows.
-// Weight rows of 8 KiB (H 4096) are faster on 32-deep k-tiles while they are
-// streamed for few rows (64 experts' rows of a k-step then spread over half as
-// many lines): up_fwd at 19 mean rows 562 on the 256-row tile against 597,
-// up_dgrad 504 on the 320-row tile against 552.
+// Past that, up to kMidAgainMaxMeanRows, an expert is two m-tiles of the
+// larger tiles, little more than half filled, and three nearly full ones of
+// the 128-row tile.  Weight rows of 8 KiB (H 4096) are faster on the larger
+// tiles while they are streamed for few rows: at 19 mean rows up_fwd takes 574
+// on the 256-row tile against 592 to 594, up_dgrad 501 on the 320-row tile
+// against 548 to 554.
 template <bool B_KCONTIG, int EPI>
 int launch_expert(GemmParams& p, hipStream_t stream, const char* name) {
   const int out_cols = (EPI == EPI_SWIGLU_FWD) ? 2 * p.swiglu_I : p.N;
   const int64_t rows = p.rows, G = p.G;
   const bool long_rows = p.ldb >= kLongRow && rows <= kLongRowMaxMeanRows * G;
   if (!long_rows && rows <= kSlimMaxMeanRows * G) return launch<MODE_MG, B_KCONTIG, EPI, SlimTile>(p, stream, name);
-  if (!long_rows && rows <= (out_cols <= 1024 ? kWideMaxMeanRows : kMidMaxMeanRows) * G)
+  if ((!long_rows && rows <= (out_cols <= 1024 ? kWideMaxMeanRows : kMidMaxMeanRows) * G) ||
+      (rows > kWideMaxMeanRows * G && rows <= kMidAgainMaxMeanRows * G))
     return launch<MODE_MG, B_KCONTIG, EPI, MidTile>(p, stream, name);
   // Up to 320 rows per expert in one m-tile, and the input gradients of long
   // weight rows.
   if (rows <= kWideMaxMeanRows * G && (rows > kBigMaxMeanRows * G || (long_rows && !B_KCONTIG)))
     return launch<MODE_MG, B_KCONTIG, EPI, WideTile>(p, stream, name);
-  // The ping-pong loop keeps the matrix pipes fed while the partner waves
-  // read fragments and fire the DMA.  It wins for the input gradients (two
-  // transpose reads per weight fragment), and for the forward GEMMs once the
-  // experts average several m-tiles (their weight tiles then come from L2;
-  // the four row-grouped GEMMs at 1024 mean rows 2769 against 2844 us, at 512
-  // and H 4096 5297 against 5465 us); with one or two m-tiles per expert the
-  // forward GEMMs stream every weight k-slice from HBM and time the same on
-  // both loops.
-  if (!B_KCONTIG || rows >= kPingMinMeanRows * G)
-    return launch<MODE_MG, B_KCONTIG, EPI, PingTile>(p, stream, name);
-  return launch<MODE_MG, B_KCONTIG, EPI, BigTileP>(p, stream, name);
+  return launch<MODE_MG, B_KCONTIG, EPI, PingTile>(p, stream, name);
 }
 
 // Operand checks.  `a` holds M rows, as does `b` when b_rows (the weight
@@ -1716,7 +1627,7 @@ int wgrad(const void* dc, const void* a, const int32_t* offs, int64_t G, int64_t
   p.bucket_rows = static_cast<int>(bucket_rows);
   p.bucket_stride = bucket_stride;
   if ((rc = set_bytes(p, M * N * 2, M * K * 2, N * K * (dw_is_f32 ? 4 : 2), name))) return rc;
-  return launch<MODE_KG, false, EPI_WGRAD, BigTile>(p, as_stream(stream), name);
+    return launch<MODE_KG, false, EPI_WGRAD, BigTile>(p, as_stream(stream), name);
 }
 }  // namespace
 

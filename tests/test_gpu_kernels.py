@@ -441,6 +441,13 @@ ROW_TILE_CASES = [
     ("mid_narrow", [288, 250, 320, 257, 1], 72, 520),
     ("big", [256, 257, 100, 224], 1288, 136),
     ("wide", [320, 321, 200, 230], 1288, 136),
+    # the ping-pong loop: one k-step, an odd and an even number of 64-deep ones with a tail in either half,
+    # tiles one after the other in a block (several n-tiles), a group without rows between two with some
+    ("ping_one_kstep", [513, 0, 600, 511], 520, 40),
+    ("ping_odd", [256, 257, 1100, 0, 300], 264, 168),
+    ("ping_even", [400, 0, 512, 700], 264, 232),
+    ("ping_many_tiles", [380, 384, 420, 360, 400, 410, 390, 370], 6152, 72),
+    ("mid_again", [320, 290, 330, 300], 1288, 136),
     ("long_rows_few", [64, 20, 0, 65], 1032, 4104),
     ("long_rows_mid", [130, 90, 0, 128], 1032, 4104),
 ]
@@ -448,8 +455,8 @@ ROW_TILE_CASES = [
 
 @pytest.mark.parametrize("name,cnt,N,K", ROW_TILE_CASES, ids=[c[0] for c in ROW_TILE_CASES])
 def test_row_tiles_give_the_exact_products(name, cnt, N, K):
-    """Small integers: every product and sum is exact in fp32 and every result below 2^8 in bf16, so
-    the outputs must be the float64 products rounded once, whatever the tile."""
+    """Small integers: every product and sum is exact in fp32, so the outputs must be the float64
+    products rounded to bf16 once, whatever the tile."""
     counts, offs = _groups(cnt)
     M, G = int(counts.sum()), len(cnt)
     od = offs.to(DEV)
