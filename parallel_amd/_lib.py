@@ -180,4 +180,4 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 def stream_of(t: torch.Tensor) -> int:
     """Raw hipStream_t of torch's current stream on the tensor's device."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())

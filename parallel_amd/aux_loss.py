@@ -18,7 +18,7 @@ from .groups import require_single_rank
 
 
 def _aux(logits: Tensor, num_experts: int, top_k: int, token_weight: Tensor | None) -> Tensor:
-    aux, _ = ops.aux_loss_fwd(logits, token_weight, num_experts, top_k)
+    aux, _ = ops.run_aux_loss_fwd(logits, token_weight, num_experts, top_k)
     return aux
 
 

@@ -59,9 +59,9 @@ class TopKRouter(nn.Module):
         hidden_states = hidden_states.reshape(-1, self.hidden_dim)
         if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16:
             with torch.autocast("cuda", enabled=False):
-                return ops.router_fwd_bf16(hidden_states.to(torch.bfloat16), self.weight.to(torch.bfloat16),
+                return ops.run_router_fwd_bf16(hidden_states.to(torch.bfloat16), self.weight.to(torch.bfloat16),
                                            self.top_k, self.norm_topk_prob)[:3]
-        return ops.router_fwd(hidden_states, self.weight, self.top_k, self.norm_topk_prob)
+        return ops.run_router_fwd(hidden_states, self.weight, self.top_k, self.norm_topk_prob)
 
 
 def _check_gated_silu(module) -> None:

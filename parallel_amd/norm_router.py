@@ -41,13 +41,13 @@ def norm_router_aux(
     for this layer.  ``attention_mask`` [B, S] weights tokens as in the
     reference's masked branch.
     """
-    x, _ = ops.rmsnorm_fwd(hidden, norm_weight, float(eps))
+    x, _ = ops.run_rmsnorm_fwd(hidden, norm_weight, float(eps))
     H = hidden.shape[-1]
     tw = None
     if attention_mask is not None:
         tw = attention_mask.to(device=hidden.device, dtype=torch.float32).reshape(-1)
         if tw.numel() != x.numel() // H:
             raise ValueError(f"attention_mask has {tw.numel()} entries for {x.numel() // H} tokens")
-    logits, scores, idx, aux, _stats = ops.router_aux_fwd(x.reshape(-1, H), router_weight, top_k, norm_topk_prob, tw,
+    logits, scores, idx, aux, _stats = ops.run_router_aux_fwd(x.reshape(-1, H), router_weight, top_k, norm_topk_prob, tw,
                                                           logit_bias)
     return x, (logits, scores, idx), aux

@@ -23,6 +23,8 @@ weight-gradient target (fsdp_bucket uses it to write into an FSDP bucket).
 
 from __future__ import annotations
 
+import inspect
+
 import torch
 from torch import Tensor
 
@@ -31,6 +33,88 @@ from ._lib import call, ptr
 
 LIB = "parallel_amd"
 BF16 = torch.bfloat16
+
+
+# ------------------------------------------------------------------- routes
+#
+# Every op is a torch.library custom op, which tracing, FakeTensor, functorch
+# transforms and dispatch modes go through.  A custom op's Python route through
+# the dispatcher costs about 16 us of host time per call without gradients and
+# about 100 us with them (forward and backward), more than many of these
+# launches take on the GPU, so an ordinary eager call, with none of those
+# active and on plain tensors, runs the op's kernels directly, or under an
+# autograd.Function (50 us) with the op's own setup and backward.
+
+_kernels: dict[str, object] = {}  # op name -> its implementation
+
+
+def _op(name: str):
+    """torch.library.custom_op with the implementation kept for direct calls."""
+
+    def wrap(fn):
+        _kernels[name] = fn
+        return torch.library.custom_op(f"{LIB}::{name}", mutates_args=())(fn)
+
+    return wrap
+
+
+_SCALARS = frozenset({int, float, bool, type(None)})
+
+
+def _plain_eager(args) -> bool:
+    """Whether a call with these arguments is ordinary eager execution on plain
+    GPU tensors: no tensor subclass, proxy, symbolic size or meta tensor among
+    them, no compilation or tracing, no torch function or dispatch mode, no
+    functorch transform, no forward-mode differentiation."""
+    for a in args:
+        t = type(a)
+        if t is Tensor or t is torch.nn.Parameter:
+            if not a.is_cuda:
+                return False
+        elif t not in _SCALARS:
+            return False
+    return not (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+                or torch._C._len_torch_function_stack() or torch._C._get_tracing_state() is not None
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
+def _wants_grad(args) -> bool:
+    return torch.is_grad_enabled() and any(isinstance(a, Tensor) and a.requires_grad for a in args)
+
+
+def _direct(name: str, *args):
+    """The op's kernels run directly where nothing observes the op and no
+    gradient is recorded; otherwise the op.  (Used by the backward formulas:
+    under create_graph they still go through the op.)"""
+    if _plain_eager(args) and not _wants_grad(args):
+        return _kernels[name](*args)
+    return getattr(torch.ops.parallel_amd, name)(*args)
+
+
+def _eager_route(name: str, op, setup, backward):
+    """The function that callers inside this package use for a differentiable
+    op: ``op`` itself, or for ordinary eager calls its kernels, recorded by an
+    autograd.Function where an argument requires a gradient."""
+    kernels = _kernels[name]
+    defaults = [p.default for p in inspect.signature(kernels).parameters.values()]
+
+    def forward(ctx, *args):
+        out = kernels(*args)
+        setup(ctx, args, out)
+        return out
+
+    fn = type(f"_{name}", (torch.autograd.Function,),
+              {"forward": staticmethod(forward), "backward": staticmethod(backward)})
+
+    def route(*args):
+        if not _plain_eager(args):
+            return op(*args)
+        if not _wants_grad(args):
+            return kernels(*args)
+        return fn.apply(*args, *defaults[len(args):])  # the backward returns one gradient per parameter
+
+    return route
 
 
 # ---------------------------------------------------------------- validation
@@ -65,7 +149,7 @@ def _ids64(t: Tensor) -> Tensor:
 # ------------------------------------------------------------------- router
 
 
-@torch.library.custom_op(f"{LIB}::router_topk", mutates_args=())
+@_op("router_topk")
 def router_topk(logits: Tensor, top_k: int, norm_topk_prob: bool) -> tuple[Tensor, Tensor]:
     """(scores [T,k] f32, indices [T,k] int64) of softmax(logits) (TF modeling_qwen3_moe.py:261-265)."""
     _require_gpu(logits)
@@ -84,7 +168,7 @@ def _(logits, top_k, norm_topk_prob):
     return logits.new_empty(T, top_k, dtype=torch.float32), logits.new_empty(T, top_k, dtype=torch.int64)
 
 
-@torch.library.custom_op(f"{LIB}::router_fwd", mutates_args=())
+@_op("router_fwd")
 def router_fwd(x: Tensor, weight: Tensor, top_k: int, norm_topk_prob: bool,
                logit_bias: Tensor | None = None) -> tuple[Tensor, Tensor, Tensor]:
     """Qwen3MoeTopKRouter.forward (TF modeling_qwen3_moe.py:258-267) with fp32 logits.
@@ -238,7 +322,7 @@ def _router_gemm_bwd(x: Tensor, weight: Tensor, dl_bf16: Tensor,
     return dx, (None if dw_target is not None else dw)
 
 
-@torch.library.custom_op(f"{LIB}::router_bwd", mutates_args=())
+@_op("router_bwd")
 def router_bwd(x: Tensor, weight: Tensor, logits: Tensor, indices: Tensor, d_logits: Tensor | None,
                d_scores: Tensor | None, norm_topk_prob: bool) -> tuple[Tensor, Tensor]:
     """(dx [T,H] bf16, dweight [E,H] bf16) through top-k/renorm/softmax and the router GEMM."""
@@ -261,14 +345,15 @@ def _router_setup(ctx, inputs, output):
 
 def _router_backward(ctx, d_logits, d_scores, _d_idx):
     x, weight, logits, idx = ctx.saved_tensors
-    dx, dw = router_bwd(x, weight, logits, idx, d_logits, d_scores, ctx.norm)
+    dx, dw = _direct("router_bwd", x, weight, logits, idx, d_logits, d_scores, ctx.norm)
     return dx, dw, None, None, None
 
 
 router_fwd.register_autograd(_router_backward, setup_context=_router_setup)
+run_router_fwd = _eager_route("router_fwd", router_fwd, _router_setup, _router_backward)
 
 
-@torch.library.custom_op(f"{LIB}::router_fwd_bf16", mutates_args=())
+@_op("router_fwd_bf16")
 def router_fwd_bf16(x: Tensor, weight: Tensor, top_k: int, norm_topk_prob: bool,
                     logit_bias: Tensor | None = None) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """router_fwd with the logits of a bf16 linear, as Qwen3MoeTopKRouter computes
@@ -321,12 +406,13 @@ def _router_bf16_backward(ctx, d_logits, d_scores, _d_idx, _d_logits32):
 
 
 router_fwd_bf16.register_autograd(_router_bf16_backward, setup_context=_router_bf16_setup)
+run_router_fwd_bf16 = _eager_route("router_fwd_bf16", router_fwd_bf16, _router_bf16_setup, _router_bf16_backward)
 
 
 # ----------------------------------------------------------------- aux loss
 
 
-@torch.library.custom_op(f"{LIB}::aux_loss_fwd", mutates_args=())
+@_op("aux_loss_fwd")
 def aux_loss_fwd(logits: Tensor, token_weight: Tensor | None, num_experts: int, top_k: int) -> tuple[Tensor, Tensor]:
     """(aux scalar f32, stats [E+1] = per-expert routed counts and the token total)."""
     _require_gpu(logits, token_weight)
@@ -349,7 +435,7 @@ def _(logits, token_weight, num_experts, top_k):
     return logits.new_empty((), dtype=torch.float32), logits.new_empty(num_experts + 1, dtype=torch.float32)
 
 
-@torch.library.custom_op(f"{LIB}::aux_loss_bwd", mutates_args=())
+@_op("aux_loss_bwd")
 def aux_loss_bwd(logits: Tensor, token_weight: Tensor | None, stats: Tensor, d_aux: Tensor) -> Tensor:
     logits = logits.float().contiguous()
     T, E = logits.shape
@@ -379,17 +465,18 @@ def _aux_backward(ctx, d_aux, _d_stats):
     logits, token_weight, stats = ctx.saved_tensors
     if d_aux is None:
         return None, None, None, None
-    dl = aux_loss_bwd(logits, token_weight, stats, d_aux)
+    dl = _direct("aux_loss_bwd", logits, token_weight, stats, d_aux)
     return dl.to(ctx.logits_dtype), None, None, None
 
 
 aux_loss_fwd.register_autograd(_aux_backward, setup_context=_aux_setup)
+run_aux_loss_fwd = _eager_route("aux_loss_fwd", aux_loss_fwd, _aux_setup, _aux_backward)
 
 
 # ------------------------------------------- the step before: norm -> router
 
 
-@torch.library.custom_op(f"{LIB}::rmsnorm_fwd", mutates_args=())
+@_op("rmsnorm_fwd")
 def rmsnorm_fwd(hidden: Tensor, weight: Tensor, eps: float) -> tuple[Tensor, Tensor]:
     """Qwen3MoeRMSNorm.forward (TF modeling_qwen3_moe.py:294-299): (x like hidden, rstd [T] f32)."""
     _require_gpu(hidden, weight)
@@ -398,11 +485,11 @@ def rmsnorm_fwd(hidden: Tensor, weight: Tensor, eps: float) -> tuple[Tensor, Ten
     H = hidden.shape[-1]
     h2 = hidden.reshape(-1, H).contiguous()
     T = h2.shape[0]
-    x = torch.empty_like(h2)
+    x = torch.empty(hidden.shape, dtype=hidden.dtype, device=hidden.device)
     rstd = torch.empty(T, dtype=torch.float32, device=hidden.device)
     call("moe_rmsnorm_fwd", ptr(h2), ptr(weight.contiguous()), T, H, float(eps), ptr(x), ptr(rstd),
          _stream(hidden), tag="norm_fwd")
-    return x.view(hidden.shape), rstd
+    return x, rstd
 
 
 @rmsnorm_fwd.register_fake
@@ -410,19 +497,19 @@ def _(hidden, weight, eps):
     return torch.empty_like(hidden), hidden.new_empty(hidden.numel() // hidden.shape[-1], dtype=torch.float32)
 
 
-@torch.library.custom_op(f"{LIB}::rmsnorm_bwd", mutates_args=())
+@_op("rmsnorm_bwd")
 def rmsnorm_bwd(dx: Tensor, hidden: Tensor, weight: Tensor, rstd: Tensor) -> tuple[Tensor, Tensor]:
     """(dhidden, dweight) of rmsnorm_fwd (autograd of TF modeling_qwen3_moe.py:294-299)."""
     H = hidden.shape[-1]
     h2 = hidden.reshape(-1, H).contiguous()
     T = h2.shape[0]
     g = dx.to(BF16).reshape(-1, H).contiguous()
-    dh = torch.empty_like(h2)
+    dh = torch.empty(hidden.shape, dtype=hidden.dtype, device=hidden.device)
     dw = torch.empty(H, dtype=BF16, device=hidden.device)
     ws = _ws(_lib.load().moe_rmsnorm_bwd_workspace_bytes(T, H), hidden.device)
     call("moe_rmsnorm_bwd", ptr(g), None, ptr(h2), ptr(weight.contiguous()), ptr(rstd), T, H, ptr(dh), ptr(dw),
          ptr(ws), ws.numel(), _stream(hidden), tag="norm_bwd")
-    return dh.view(hidden.shape), dw
+    return dh, dw
 
 
 @rmsnorm_bwd.register_fake
@@ -439,14 +526,15 @@ def _norm_setup(ctx, inputs, output):
 
 def _norm_backward(ctx, dx, _drstd):
     hidden, weight, rstd = ctx.saved_tensors
-    dh, dw = rmsnorm_bwd(dx, hidden, weight, rstd)
+    dh, dw = _direct("rmsnorm_bwd", dx, hidden, weight, rstd)
     return dh, dw, None
 
 
 rmsnorm_fwd.register_autograd(_norm_backward, setup_context=_norm_setup)
+run_rmsnorm_fwd = _eager_route("rmsnorm_fwd", rmsnorm_fwd, _norm_setup, _norm_backward)
 
 
-@torch.library.custom_op(f"{LIB}::router_aux_fwd", mutates_args=())
+@_op("router_aux_fwd")
 def router_aux_fwd(x: Tensor, weight: Tensor, top_k: int, norm_topk_prob: bool, token_weight: Tensor | None = None,
                    logit_bias: Tensor | None = None) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
     """router_fwd plus the Switch aux loss from the same softmax and top-k: (logits, scores, indices,
@@ -520,12 +608,13 @@ def _router_aux_backward(ctx, d_logits, d_scores, _d_idx, d_aux, _d_stats):
 
 
 router_aux_fwd.register_autograd(_router_aux_backward, setup_context=_router_aux_setup)
+run_router_aux_fwd = _eager_route("router_aux_fwd", router_aux_fwd, _router_aux_setup, _router_aux_backward)
 
 
 # ------------------------------------------------------------------ permute
 
 
-@torch.library.custom_op(f"{LIB}::permute_fwd", mutates_args=())
+@_op("permute_fwd")
 def permute_fwd(hidden: Tensor, ids: Tensor, divisor: int, num_buckets: int,
                 gather_rows: bool) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
     """Stable sort of slots by ids // divisor.
@@ -596,7 +685,7 @@ def _check_experts(hidden: Tensor, top_k_index: Tensor, top_k_weights: Tensor, g
     return T, H, k, E, I2 // 2
 
 
-@torch.library.custom_op(f"{LIB}::experts_fwd", mutates_args=())
+@_op("experts_fwd")
 def experts_fwd(hidden: Tensor, top_k_index: Tensor, top_k_weights: Tensor, gate_up_proj: Tensor,
                 down_proj: Tensor, accumulate_grad: bool = False
                 ) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
@@ -786,7 +875,7 @@ def experts_bwd_kernels(d_out: Tensor, top_k_weights: Tensor, gate_up_proj: Tens
     return d_hidden, d_w, d_gu, d_down
 
 
-@torch.library.custom_op(f"{LIB}::experts_bwd", mutates_args=())
+@_op("experts_bwd")
 def experts_bwd(d_out: Tensor, top_k_weights: Tensor, gate_up_proj: Tensor, down_proj: Tensor, xp: Tensor,
                 pre: Tensor, act: Tensor, y: Tensor, pos_of_slot: Tensor,
                 offsets: Tensor) -> tuple[Tensor, Tensor, Tensor, Tensor]:
@@ -836,7 +925,7 @@ def _experts_backward(ctx, d_out, *_unused):
         return None, None, None, None, None, None
     targets = [_grad_target(p) for p in ctx.params] if ctx.params is not None else [None, None]
     if targets[0] is None and targets[1] is None:
-        d_hidden, d_w, d_gu, d_dn = experts_bwd(d_out, w, gu, dn, xp, pre, act, y, pos, offsets)
+        d_hidden, d_w, d_gu, d_dn = _direct("experts_bwd", d_out, w, gu, dn, xp, pre, act, y, pos, offsets)
     else:
         d_hidden, d_w, d_gu, d_dn = experts_bwd_accumulate(d_out, w, gu, dn, xp, pre, act, y, pos, offsets,
                                                            targets[0], targets[1])
@@ -844,6 +933,7 @@ def _experts_backward(ctx, d_out, *_unused):
 
 
 experts_fwd.register_autograd(_experts_backward, setup_context=_experts_setup)
+_run_experts_fwd = _eager_route("experts_fwd", experts_fwd, _experts_setup, _experts_backward)
 
 
 def experts_bwd_accumulate(d_out, top_k_weights, gate_up_proj, down_proj, xp, pre, act, y, pos_of_slot, offsets,
@@ -890,7 +980,7 @@ def experts(hidden: Tensor, top_k_index: Tensor, top_k_weights: Tensor, gate_up_
     hooks and post-accumulate-grad hooks of such a weight do not run, and
     under ``torch.compile`` (AOTAutograd) the option is refused."""
     _refuse_traced_accumulation(accumulate_grad, "experts")
-    return experts_fwd(hidden, top_k_index, top_k_weights, gate_up_proj, down_proj, accumulate_grad)[0]
+    return _run_experts_fwd(hidden, top_k_index, top_k_weights, gate_up_proj, down_proj, accumulate_grad)[0]
 
 
 def _refuse_traced_accumulation(accumulate_grad: bool, what: str) -> None:
@@ -904,7 +994,7 @@ def _refuse_traced_accumulation(accumulate_grad: bool, what: str) -> None:
 # --------------------------------------------- the whole block in one op
 
 
-@torch.library.custom_op(f"{LIB}::moe_block_fwd", mutates_args=())
+@_op("moe_block_fwd")
 def moe_block_fwd(x: Tensor, router_weight: Tensor, gate_up_proj: Tensor, down_proj: Tensor, top_k: int,
                   norm_topk_prob: bool, token_weight: Tensor | None = None, logit_bias: Tensor | None = None,
                   accumulate_grad: bool = False, bf16_logits: bool = False
@@ -1024,6 +1114,7 @@ def _block_backward(ctx, d_out, d_logits, d_scores, _d_idx, d_aux, *_unused):
 
 
 moe_block_fwd.register_autograd(_block_backward, setup_context=_block_setup)
+_run_moe_block_fwd = _eager_route("moe_block_fwd", moe_block_fwd, _block_setup, _block_backward)
 
 
 def moe_block(x: Tensor, router_weight: Tensor, gate_up_proj: Tensor, down_proj: Tensor, top_k: int,
@@ -1053,15 +1144,16 @@ def moe_block(x: Tensor, router_weight: Tensor, gate_up_proj: Tensor, down_proj:
     ``experts`` does for the expert weights (with the same limits: no grad
     hooks for those weights, refused under ``torch.compile``)."""
     _refuse_traced_accumulation(accumulate_grad, "moe_block")
-    out, logits, scores, idx, aux = moe_block_fwd(x, router_weight, gate_up_proj, down_proj, top_k, norm_topk_prob,
-                                                  token_weight, logit_bias, accumulate_grad, bf16_logits)[:5]
+    out, logits, scores, idx, aux = _run_moe_block_fwd(x, router_weight, gate_up_proj, down_proj, top_k,
+                                                       norm_topk_prob, token_weight, logit_bias, accumulate_grad,
+                                                       bf16_logits)[:5]
     return out, logits, scores, idx, aux
 
 
 # ------------------------------------------------------- token dispatch ops
 
 
-@torch.library.custom_op(f"{LIB}::dispatch_fwd", mutates_args=())
+@_op("dispatch_fwd")
 def dispatch_fwd(hidden: Tensor, global_indices: Tensor, scores: Tensor, local_count: int,
                  ep_size: int) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
     """Owner-major send buffers of TokenDispatcher.dispatch (token_dispatch.py:101-125).
@@ -1119,16 +1211,18 @@ def _dispatch_backward(ctx, d_send_hidden, _d_experts, d_send_scores, *_unused):
     (pos,) = ctx.saved_tensors
     d_hidden = d_scores = None
     if d_send_hidden is not None:
-        d_hidden = combine_rows_fwd(d_send_hidden.to(BF16).contiguous(), pos, ctx.T, ctx.k).to(ctx.hidden_dtype)
+        d_hidden = _direct("combine_rows_fwd", d_send_hidden.to(BF16).contiguous(), pos, ctx.T,
+                           ctx.k).to(ctx.hidden_dtype)
     if d_send_scores is not None:
         d_scores = d_send_scores.index_select(0, pos.long()).view(ctx.T, ctx.k).to(ctx.scores_dtype)
     return d_hidden, None, d_scores, None, None
 
 
 dispatch_fwd.register_autograd(_dispatch_backward, setup_context=_dispatch_setup)
+run_dispatch_fwd = _eager_route("dispatch_fwd", dispatch_fwd, _dispatch_setup, _dispatch_backward)
 
 
-@torch.library.custom_op(f"{LIB}::combine_rows_fwd", mutates_args=())
+@_op("combine_rows_fwd")
 def combine_rows_fwd(rows: Tensor, pos_of_slot: Tensor, num_tokens: int, top_k: int) -> Tensor:
     """out[t] = sum_j rows[pos_of_slot[t*k+j]] — TokenDispatcher.combine's index_add in gather form."""
     _require_gpu(rows, pos_of_slot)
@@ -1148,7 +1242,7 @@ def _(rows, pos_of_slot, num_tokens, top_k):
     return rows.new_empty(num_tokens, rows.shape[1])
 
 
-@torch.library.custom_op(f"{LIB}::combine_rows_bwd", mutates_args=())
+@_op("combine_rows_bwd")
 def combine_rows_bwd(d_out: Tensor, pos_of_slot: Tensor, top_k: int) -> Tensor:
     """d_rows[pos_of_slot[t*k+j]] = d_out[t]."""
     T, H = d_out.shape
@@ -1176,7 +1270,8 @@ def _combine_backward(ctx, d_out):
     (pos,) = ctx.saved_tensors
     if d_out is None:
         return None, None, None, None
-    return combine_rows_bwd(d_out, pos, ctx.top_k), None, None, None
+    return _direct("combine_rows_bwd", d_out, pos, ctx.top_k), None, None, None
 
 
 combine_rows_fwd.register_autograd(_combine_backward, setup_context=_combine_setup)
+run_combine_rows_fwd = _eager_route("combine_rows_fwd", combine_rows_fwd, _combine_setup, _combine_backward)

@@ -106,7 +106,7 @@ class TokenDispatcher:
         if global_indices.shape != scores.shape:
             raise ValueError("Expert indices and scores must have the same shape")
         tokens, top_k = global_indices.shape
-        send_hidden, send_experts, send_scores, source_tokens, pos_of_slot, counts = ops.dispatch_fwd(
+        send_hidden, send_experts, send_scores, source_tokens, pos_of_slot, counts = ops.run_dispatch_fwd(
             hidden_states, global_indices, scores, self.partition.local_count, self.partition.ep_size
         )
         send_splits, receive_splits = self._exchange_splits(counts)
@@ -120,4 +120,4 @@ class TokenDispatcher:
         returned = self._exchange(expert_output, state.receive_splits, state.send_splits, "combine_hidden")
         if state.pos_of_slot is None:
             raise ValueError("DispatchState has no inverse permutation; it was not produced by this dispatcher")
-        return ops.combine_rows_fwd(returned, state.pos_of_slot, state.num_source_tokens, state.top_k)
+        return ops.run_combine_rows_fwd(returned, state.pos_of_slot, state.num_source_tokens, state.top_k)
