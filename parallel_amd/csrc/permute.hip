@@ -1,7 +1,8 @@
 // Token permutation into expert-contiguous (or owner-rank-contiguous) order.
 //
 // A stable counting sort of the S = T*k routed slots by bucket = id / divisor,
-// in two small launches plus one bandwidth-bound row gather:
+// in two small launches plus one bandwidth-bound row copy (one launch for it
+// all up to one chunk of slots):
 //   1. count:   each block histograms a CHUNK of slots in LDS (integer
 //               atomics, so counts are exact and order-free);
 //   2. scatter: each block reads the [blocks x buckets] histogram for its
@@ -12,7 +13,7 @@
 //               ballot per key bit, ranks a slot by the popcount of equal-key
 //               lanes below it, and waves are ordered through per-round LDS
 //               counters, which keeps the sort stable;
-//   3. gather:  one wave per sorted row copies hidden[perm/k] (16-byte lanes).
+//   3. rows:    one wave per token copies its row to its slots' sorted rows.
 // Sentinel slots (bucket >= num_buckets) land after every real bucket.
 //
 // Reference: TF/integrations/moe.py:389-437 (sort/gather/histc/cumsum,
@@ -60,13 +61,104 @@ __global__ __launch_bounds__(kPermThreads) void permute_count_kernel(const int64
   for (int i = threadIdx.x; i < nb1; i += kPermThreads) hist[static_cast<int64_t>(blockIdx.x) * nb1 + i] = h[i];
 }
 
-// Each block first places its chunk from the count kernel's histogram
-// hist[nblk][nb + 1]: per bucket, the counts of the blocks before it (its
-// first position within the bucket) and of all blocks (the bucket's size); an
-// exclusive scan of the sizes gives the buckets' starts, the sentinel bucket's
-// after every real one.  Block 0 also writes counts[e] and the inclusive
-// offsets[e] of the real buckets.  (One launch fewer than a separate scan
-// kernel; each block reads the nblk x (nb + 1) histogram from L2.)
+struct SortLds {
+  int running[kMaxBuckets + 1];  // next free position of the chunk in each bucket
+  int total[kMaxBuckets + 1];    // all slots of each bucket
+  int wave_cnt[kPermThreads / kWave][kMaxBuckets + 1];
+  int wsum[kPermThreads / kWave];
+};
+
+// Places the chunk's slots [begin, end) (thread t holds the ids of slots
+// begin + r kPermThreads + t), given per bucket l.total, the slots of the
+// chunks before this one in l.running, and zeros in l.wave_cnt: emit(s, pos)
+// for every slot.  An exclusive scan of the totals gives the buckets' starts,
+// the sentinel bucket's after every real one; with write_totals the block
+// also writes counts[e] and the inclusive offsets[e] of the real buckets.
+// Returns the slots of the real buckets.
+template <class Emit>
+__device__ __forceinline__ int place_chunk(SortLds& l, const int64_t (&id)[kPerThread], int begin, int end,
+                                           int64_t divisor, int nb, bool write_totals, int32_t* __restrict__ counts,
+                                           int32_t* __restrict__ offsets, Emit emit) {
+  const int nb1 = nb + 1;
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1), wave = tid >> 6;
+  __syncthreads();
+  // Buckets' starts: thread t scans the real buckets t G .. t G + G - 1
+  // (G = ceil(nb / kPermThreads) <= 4) in order, the threads in turn.
+  constexpr int kG = (kMaxBuckets + kPermThreads - 1) / kPermThreads;
+  const int G = (nb + kPermThreads - 1) / kPermThreads;
+  int size[kG];
+  int sum = 0;
+#pragma unroll
+  for (int j = 0; j < kG; ++j) {
+    const int e = tid * G + j;
+    size[j] = (j < G && e < nb) ? l.total[e] : 0;
+    sum += size[j];
+  }
+  const int incl = wave_inclusive_scan(sum);
+  if (lane == kWave - 1) l.wsum[wave] = incl;
+  __syncthreads();
+  int run = incl - sum, n_valid = 0;
+#pragma unroll
+  for (int w = 0; w < kPermThreads / kWave; ++w) {
+    run += w < wave ? l.wsum[w] : 0;
+    n_valid += l.wsum[w];
+  }
+#pragma unroll
+  for (int j = 0; j < kG; ++j) {
+    const int e = tid * G + j;
+    if (j < G && e < nb) {
+      if (write_totals) {
+        counts[e] = size[j];
+        offsets[e] = run + size[j];
+      }
+      l.running[e] += run;
+      run += size[j];
+    }
+  }
+  if (tid == 0) l.running[nb] += n_valid;
+  __syncthreads();
+  int nbits = 1;
+  while ((1 << nbits) < nb1) ++nbits;
+  const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+  for (int r = 0; r < kPerThread; ++r) {
+    const int r0 = begin + r * kPermThreads;
+    if (r0 >= end) break;
+    const int s = r0 + tid;
+    const bool live = s < end;
+    const int key = live ? bucket_of(id[r], divisor, nb) : 0;
+    // Lanes holding the same key: intersect one ballot per key bit.
+    unsigned long long match = __ballot(live);
+#pragma unroll 1
+    for (int b = 0; b < nbits; ++b) {
+      unsigned long long set = __ballot(live && ((key >> b) & 1));
+      match &= ((key >> b) & 1) ? set : ~set;
+    }
+    const int rank = __popcll(match & lt_mask);
+    const bool leader = live && rank == 0;
+    if (leader) l.wave_cnt[wave][key] = __popcll(match);
+    __syncthreads();
+    if (live) {
+      int pos = l.running[key] + rank;
+      for (int w = 0; w < wave; ++w) pos += l.wave_cnt[w][key];
+      emit(s, pos);
+    }
+    __syncthreads();
+    if (leader) {
+      atomicAdd(&l.running[key], l.wave_cnt[wave][key]);
+      l.wave_cnt[wave][key] = 0;
+    }
+    __syncthreads();
+  }
+  return n_valid;
+}
+
+// Each block first finds, from the count kernel's histogram
+// hist[nblk][nb + 1], per bucket the counts of the blocks before it (its
+// first position within the bucket) and of all blocks (the bucket's size),
+// then places its chunk.  (One launch fewer than a separate scan kernel; each
+// block reads the nblk x (nb + 1) histogram from L2.)
 __global__ __launch_bounds__(kPermThreads) void permute_scatter_kernel(const int64_t* __restrict__ ids, int S,
                                                                         int64_t divisor, int nb,
                                                                         const int32_t* __restrict__ hist, int nblk,
@@ -74,13 +166,9 @@ __global__ __launch_bounds__(kPermThreads) void permute_scatter_kernel(const int
                                                                         int32_t* __restrict__ offsets,
                                                                         int32_t* __restrict__ perm,
                                                                         int32_t* __restrict__ pos_of_slot) {
-  __shared__ int running[kMaxBuckets + 1];
-  __shared__ int total[kMaxBuckets + 1];
-  __shared__ int wave_cnt[kPermThreads / kWave][kMaxBuckets + 1];
-  __shared__ int wsum[kPermThreads / kWave];
+  __shared__ SortLds l;
   const int nb1 = nb + 1;
   const int tid = threadIdx.x;
-  const int lane = tid & (kWave - 1), wave = tid >> 6;
   const int begin = blockIdx.x * kChunk;
   const int end = min(begin + kChunk, S);
   // Every round's ids in flight before the first round.
@@ -106,83 +194,93 @@ __global__ __launch_bounds__(kPermThreads) void permute_scatter_kernel(const int
         all += c[r];
       }
     }
-    running[e] = before;
-    total[e] = all;
+    l.running[e] = before;
+    l.total[e] = all;
 #pragma unroll
-    for (int w = 0; w < kPermThreads / kWave; ++w) wave_cnt[w][e] = 0;
+    for (int w = 0; w < kPermThreads / kWave; ++w) l.wave_cnt[w][e] = 0;
   }
-  __syncthreads();
-  // Buckets' starts: thread t scans the real buckets t G .. t G + G - 1
-  // (G = ceil(nb / kPermThreads) <= 4) in order, the threads in turn.
-  constexpr int kG = (kMaxBuckets + kPermThreads - 1) / kPermThreads;
-  const int G = (nb + kPermThreads - 1) / kPermThreads;
-  int size[kG];
-  int sum = 0;
+  place_chunk(l, id, begin, end, divisor, nb, me == 0, counts, offsets, [&](int slot, int pos) {
+    if (pos >= 0 && pos < S) {  // always true for a consistent histogram; never write outside
+      perm[pos] = slot;
+      pos_of_slot[slot] = pos;
+    }
+  });
+}
+
+// One token's row to the sorted rows pos[j] of its slots (zeros where
+// pos[j] >= n_valid), by one wave: up to four 16-byte chunks per lane in
+// flight before their stores.
+template <int KM>
+__device__ __forceinline__ void copy_token_rows(const bf16_t* __restrict__ row, int H, const int (&pos)[KM], int S,
+                                                int n_valid, bf16_t* __restrict__ out) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int nchunk = H / 8;
+  const uint4* src = reinterpret_cast<const uint4*>(row);
+  for (int c0 = lane; c0 < nchunk; c0 += 4 * kWave) {
+    uint4 v[4];
 #pragma unroll
-  for (int j = 0; j < kG; ++j) {
-    const int e = tid * G + j;
-    size[j] = (j < G && e < nb) ? total[e] : 0;
-    sum += size[j];
-  }
-  const int incl = wave_inclusive_scan(sum);
-  if (lane == kWave - 1) wsum[wave] = incl;
-  __syncthreads();
-  int run = incl - sum, n_valid = 0;
+    for (int u = 0; u < 4; ++u) v[u] = c0 + u * kWave < nchunk ? src[c0 + u * kWave] : make_uint4(0, 0, 0, 0);
 #pragma unroll
-  for (int w = 0; w < kPermThreads / kWave; ++w) {
-    run += w < wave ? wsum[w] : 0;
-    n_valid += wsum[w];
-  }
+    for (int j = 0; j < KM; ++j) {
+      const int p = pos[j];
+      if (p >= 0 && p < S) {  // (always, for a permutation; a wave-uniform guard)
+        uint4* dst = reinterpret_cast<uint4*>(out + static_cast<int64_t>(p) * H);
 #pragma unroll
-  for (int j = 0; j < kG; ++j) {
-    const int e = tid * G + j;
-    if (j < G && e < nb) {
-      if (me == 0) {
-        counts[e] = size[j];
-        offsets[e] = run + size[j];
+        for (int u = 0; u < 4; ++u)
+          if (c0 + u * kWave < nchunk) dst[c0 + u * kWave] = p < n_valid ? v[u] : make_uint4(0, 0, 0, 0);
       }
-      running[e] += run;
-      run += size[j];
     }
   }
-  if (tid == 0) running[nb] += n_valid;
-  __syncthreads();
-  int nbits = 1;
-  while ((1 << nbits) < nb1) ++nbits;
-  const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+}
+
+// The whole permutation in one launch for at most one chunk of slots (a
+// decoding batch): every block sorts the chunk for itself, from a histogram in
+// LDS, and copies the rows of its own tokens; block 0 writes the maps and
+// counts.  At such sizes the launches are the cost: 8 slots (one token, H 2048)
+// took 1.7 + 4.2 + 4.1 us in three.
+template <int KT>
+__global__ __launch_bounds__(kPermThreads) void permute_small_kernel(
+    const int64_t* __restrict__ ids, int S, int64_t divisor, int nb, const bf16_t* __restrict__ hidden, int H, int T,
+    int k, int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ perm,
+    int32_t* __restrict__ pos_of_slot, bf16_t* __restrict__ out) {
+  constexpr int KM = KT ? KT : kMaxSlots;
+  __shared__ SortLds l;
+  __shared__ int slot_pos[kChunk];
+  const int tid = threadIdx.x;
+  const bool first = blockIdx.x == 0;
+  int64_t id[kPerThread];
 #pragma unroll
   for (int r = 0; r < kPerThread; ++r) {
-    const int r0 = begin + r * kPermThreads;
-    if (r0 >= end) break;
-    const int s = r0 + threadIdx.x;
-    const bool live = s < end;
-    const int key = live ? bucket_of(id[r], divisor, nb) : 0;
-    // Lanes holding the same key: intersect one ballot per key bit.
-    unsigned long long match = __ballot(live);
-#pragma unroll 1
-    for (int b = 0; b < nbits; ++b) {
-      unsigned long long set = __ballot(live && ((key >> b) & 1));
-      match &= ((key >> b) & 1) ? set : ~set;
-    }
-    const int rank = __popcll(match & lt_mask);
-    const bool leader = live && rank == 0;
-    if (leader) wave_cnt[wave][key] = __popcll(match);
-    __syncthreads();
-    if (live) {
-      int pos = running[key] + rank;
-      for (int w = 0; w < wave; ++w) pos += wave_cnt[w][key];
-      if (pos >= 0 && pos < S) {  // always true for a consistent histogram; never write outside
-        perm[pos] = s;
-        pos_of_slot[s] = pos;
-      }
-    }
-    __syncthreads();
-    if (leader) {
-      atomicAdd(&running[key], wave_cnt[wave][key]);
-      wave_cnt[wave][key] = 0;
-    }
-    __syncthreads();
+    const int s = r * kPermThreads + tid;
+    id[r] = s < S ? ids[s] : -1;
   }
+  for (int e = tid; e <= nb; e += kPermThreads) {
+    l.running[e] = l.total[e] = 0;
+#pragma unroll
+    for (int w = 0; w < kPermThreads / kWave; ++w) l.wave_cnt[w][e] = 0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kPerThread; ++r)
+    if (r * kPermThreads + tid < S) atomicAdd(&l.total[bucket_of(id[r], divisor, nb)], 1);
+  const int n_valid = place_chunk(l, id, 0, S, divisor, nb, first, counts, offsets, [&](int slot, int pos) {
+    slot_pos[slot] = pos;
+    if (first) {
+      perm[pos] = slot;
+      pos_of_slot[slot] = pos;
+    }
+  });
+  if (!out) return;
+  __syncthreads();
+  const int t = blockIdx.x * (kPermThreads / kWave) + (tid >> 6);
+  if (t >= T) return;
+  int pos[KM];
+#pragma unroll
+  for (int j = 0; j < KM; ++j) {
+    const bool live = KT ? true : j < k;
+    pos[j] = __builtin_amdgcn_readfirstlane(live ? slot_pos[t * k + j] : -1);
+  }
+  copy_token_rows(hidden + static_cast<int64_t>(t) * H, H, pos, S, n_valid, out);
 }
 
 // permuted[pos_of_slot[t k + j]] = hidden[t] for the token's slots that sort
@@ -197,9 +295,7 @@ __global__ __launch_bounds__(kPermThreads) void scatter_rows_kernel(const bf16_t
                                                                      const int32_t* __restrict__ n_valid_ptr,
                                                                      bf16_t* __restrict__ out) {
   constexpr int KM = KT ? KT : kMaxSlots;
-  const int lane = threadIdx.x & (kWave - 1);
   const int n_valid = *n_valid_ptr;
-  const int nchunk = H / 8;
   for (int t = blockIdx.x * (kPermThreads / kWave) + (threadIdx.x >> 6); t < T;
        t += gridDim.x * (kPermThreads / kWave)) {
     int pos[KM];
@@ -208,23 +304,7 @@ __global__ __launch_bounds__(kPermThreads) void scatter_rows_kernel(const bf16_t
       const bool live = KT ? true : j < k;
       pos[j] = __builtin_amdgcn_readfirstlane(live ? pos_of_slot[static_cast<int64_t>(t) * k + j] : -1);
     }
-    const uint4* src = reinterpret_cast<const uint4*>(hidden + static_cast<int64_t>(t) * H);
-    // Up to four 16-byte chunks per lane in flight before their stores.
-    for (int c0 = lane; c0 < nchunk; c0 += 4 * kWave) {
-      uint4 v[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = c0 + u * kWave < nchunk ? src[c0 + u * kWave] : make_uint4(0, 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < KM; ++j) {
-        const int p = pos[j];
-        if (p >= 0 && p < S) {  // (always, for a permutation; a wave-uniform guard)
-          uint4* dst = reinterpret_cast<uint4*>(out + static_cast<int64_t>(p) * H);
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            if (c0 + u * kWave < nchunk) dst[c0 + u * kWave] = p < n_valid ? v[u] : make_uint4(0, 0, 0, 0);
-        }
-      }
-    }
+    copy_token_rows(hidden + static_cast<int64_t>(t) * H, H, pos, S, n_valid, out);
   }
 }
 
@@ -345,6 +425,12 @@ int permute_fwd_run(const void* hidden, int64_t T, int64_t H, const int64_t* ids
   hipStream_t st = as_stream(stream);
   int32_t* hist = static_cast<int32_t*>(workspace);
   const int nblk = (S + kChunk - 1) / kChunk;
+  if (nblk == 1) {  // (row_grid's cap is far above a chunk's tokens: one wave per token)
+    MOE_DISPATCH_K(k, permute_small_kernel, dim3(permuted ? row_grid(T) : 1), dim3(kPermThreads), 0, st, ids, S,
+                   divisor, nb, static_cast<const bf16_t*>(hidden), static_cast<int>(H), static_cast<int>(T),
+                   static_cast<int>(k), counts, offsets, perm, pos_of_slot, static_cast<bf16_t*>(permuted));
+    return launch_status("moe_permute_fwd(small)");
+  }
   if (nblk > 0) {
     hipLaunchKernelGGL(permute_count_kernel, dim3(nblk), dim3(kPermThreads), 0, st, ids, S, divisor, nb, hist);
     int rc = launch_status("moe_permute_fwd(count)");

@@ -273,6 +273,25 @@ def test_permute_out_of_range_ids_are_sentinels(divisor, nb):
     assert not rows.cpu()[n_valid:].any()
 
 
+@pytest.mark.parametrize("T,k,divisor,nb", [(1, 8, 1, 128), (5, 3, 1, 1024), (64, 8, 1, 128), (512, 1, 4, 9),
+                                            (73, 7, 3, 5), (171, 3, 1, 16)])
+def test_permute_of_one_chunk(T, k, divisor, nb):
+    """Up to 512 slots are sorted and copied in one launch (the last case is one slot past it): repeated
+    ids, sentinels on both sides, several blocks of tokens."""
+    g = gen(T * 100 + nb)
+    ids = torch.randint(-divisor, (nb + 1) * divisor, (T, k), generator=g)
+    hidden = torch.randn(T, 264, generator=g).to(BF)
+    rows, perm, pos, counts, offsets = ops.permute_fwd(hidden.to(DEV), ids.to(DEV), divisor, nb, True)
+    r_perm, r_pos, r_counts, r_off = O.stable_permutation(ids.numpy(), divisor, nb)
+    assert np.array_equal(perm.cpu().numpy(), r_perm) and np.array_equal(pos.cpu().numpy(), r_pos)
+    assert np.array_equal(counts.cpu().numpy(), r_counts) and np.array_equal(offsets.cpu().numpy(), r_off)
+    n_valid = int(r_off[-1])
+    assert torch.equal(rows.cpu()[:n_valid], hidden[torch.from_numpy(r_perm[:n_valid]) // k])
+    assert not rows.cpu()[n_valid:].any()
+    none, perm2, pos2, _, _ = ops.permute_fwd(hidden.to(DEV), ids.to(DEV), divisor, nb, False)
+    assert none.numel() == 0 and torch.equal(perm2, perm) and torch.equal(pos2, pos)
+
+
 def test_permute_empty_input():
     _, perm, pos, counts, offsets = ops.permute_fwd(torch.empty(0, 64, dtype=BF, device=DEV),
                                                     torch.empty(0, 8, dtype=torch.long, device=DEV), 1, 16, True)
