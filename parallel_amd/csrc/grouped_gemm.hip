@@ -87,18 +87,6 @@ struct GemmParams {
 
 // ---------------------------------------------------------------- helpers
 
-// Raw buffer loads: offsets at or past the resource's byte size read as zero
-// in hardware, so out-of-range rows and the K tail need no branches.
-constexpr uint32_t kOOB = 0x80000000u;  // >= every resource size (host checks < 2 GiB)
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
-}
-
-// silu(g) = g * sigmoid(g), with the hardware exp and reciprocal (1 ulp).
-__device__ __forceinline__ float sigmoid_f(float g) { return __builtin_amdgcn_rcpf(1.0f + __expf(-g)); }
-__device__ __forceinline__ float silu_f(float g) { return g * sigmoid_f(g); }
-
 // Total tiles over all groups, sum_g n_mult * ceil(cnt_g / BM) (wave-uniform).
 template <int BM>
 __device__ __forceinline__ int count_tiles(const int32_t* offs, int G, int rows, int n_mult) {
@@ -1291,6 +1279,7 @@ int launch(GemmParams& p, hipStream_t stream, const char* name) {
 }
 
 // Bounds of launch_expert's rule, in mean rows per expert.
+constexpr int64_t kFewMaxMeanRows = 2;
 constexpr int64_t kSlimMaxMeanRows = 32;
 constexpr int64_t kMidMaxMeanRows = 112;
 constexpr int64_t kBigMaxMeanRows = 224;
@@ -1328,10 +1317,25 @@ constexpr int64_t kLongRowMaxMeanRows = 64;
 // tiles while they are streamed for few rows: at 19 mean rows up_fwd takes 574
 // on the 256-row tile against 592 to 594, up_dgrad 501 on the 320-row tile
 // against 548 to 554.
+//
+// The forward GEMMs of a few decoded tokens go to few_rows (up / down, against
+// the 64-row tile; H 2048, I 768: 1 token 14/11 against 22/12, 4 tokens 34/18
+// against 35/18, 16 tokens 105/52 against 122/50, 48 tokens, 3 mean rows,
+// 147/72 against 141/71; H 4096, I 1536: 1 token 35/19 against 78/20, 16 tokens
+// 341/175 against 371/185).  It adds the products in another order, eight
+// partial sums over K.
 template <bool B_KCONTIG, int EPI>
 int launch_expert(GemmParams& p, hipStream_t stream, const char* name) {
   const int out_cols = (EPI == EPI_SWIGLU_FWD) ? 2 * p.swiglu_I : p.N;
   const int64_t rows = p.rows, G = p.G;
+  if constexpr (B_KCONTIG) {
+    if (rows <= kFewMaxMeanRows * G && few_rows_takes(p.K)) {
+      constexpr bool swiglu = EPI == EPI_SWIGLU_FWD;
+      return few_rows(FewRows{p.A, p.B, static_cast<bf16_t*>(p.C), static_cast<bf16_t*>(p.C2), p.offs, p.G, p.rows,
+                              swiglu ? p.swiglu_I : p.N, p.K},
+                      swiglu, stream, name);
+    }
+  }
   const bool long_rows = p.ldb >= kLongRow && rows <= kLongRowMaxMeanRows * G;
   if (!long_rows && rows <= kSlimMaxMeanRows * G) return launch<MODE_MG, B_KCONTIG, EPI, SlimTile>(p, stream, name);
   if ((!long_rows && rows <= (out_cols <= 1024 ? kWideMaxMeanRows : kMidMaxMeanRows) * G) ||

@@ -451,6 +451,54 @@ def test_grouped_gemm_wgrad_skewed_routing(name, accumulate, f32):
     print(f"{name}: {G} groups, {M} rows, worst rel {float(rel[live].max()):.2e}")
 
 
+# At most 2 mean rows per expert (a decoding batch): one row, several 16-row chunks of one expert, more
+# groups than a wave has lanes, N off the multiples of 16 and 64, K inside a wave's last k-step, a K that
+# leaves waves idle, the largest K, and one past it (the tiled kernel).
+FEW_ROWS_CASES = [
+    ("one", [0] * 5 + [1] + [0] * 2, 64, 2048),
+    ("chunks", [0] * 30 + [33, 16, 1] + [0] * 10, 72, 512),
+    ("many_groups", ([0, 1, 2] * 70)[:200], 88, 264),
+    ("idle_waves", [1, 0, 2, 3, 0, 0], 200, 640),
+    ("k1536", [2, 0, 2, 1, 0, 0], 136, 1536),
+    ("k_tail", [1, 3, 0, 0], 40, 1000),
+    ("k4096", [1, 0, 2, 0], 56, 4096),
+    ("past_k", [1, 0, 2, 0], 56, 4104),
+]
+
+
+@pytest.mark.parametrize("name,cnt,N,K", FEW_ROWS_CASES, ids=[c[0] for c in FEW_ROWS_CASES])
+def test_few_rows_forward_is_exact_on_integers(name, cnt, N, K):
+    """Small integers: every sum is exact in fp32 in any order, so the output is the float64 product
+    rounded to bf16 once; rows past the groups stay untouched.  The SwiGLU form on the same products:
+    gate | up exact, act with the reference's roundings (the hardware sigmoid: 2 bf16 steps)."""
+    counts, offs = _groups(cnt)
+    M, G = int(counts.sum()) + 3, len(cnt)
+    n = M - 3
+    a = torch.randint(-1, 2, (M, K), generator=gen(31)).to(BF)
+    w = torch.randint(-1, 2, (G, 2 * N, K), generator=gen(32)).to(BF)
+    ad, wd, od = a.to(DEV), w.to(DEV), offs.to(DEV)
+    w_half = wd[:, :N].contiguous()
+    c = torch.full((M, N), 7.0, dtype=BF, device=DEV)
+    act, pre = torch.full((M, N), 7.0, dtype=BF, device=DEV), torch.full((M, 2 * N), 7.0, dtype=BF, device=DEV)
+    act2 = torch.full((M, N), 7.0, dtype=BF, device=DEV)
+    s = _lib.stream_of(c)
+    _lib.call("moe_grouped_gemm_fwd", ad.data_ptr(), w_half.data_ptr(), od.data_ptr(), G, M, N, K, c.data_ptr(), s)
+    _lib.call("moe_grouped_gemm_swiglu_fwd", ad.data_ptr(), wd.data_ptr(), od.data_ptr(), G, M, K, N, act.data_ptr(),
+              pre.data_ptr(), s)
+    _lib.call("moe_grouped_gemm_swiglu_fwd", ad.data_ptr(), wd.data_ptr(), od.data_ptr(), G, M, K, N, act2.data_ptr(),
+              None, s)
+    torch.cuda.synchronize()
+    ref = torch.cat([a[o - c_:o].double() @ w[e].double().t()
+                     for e, (o, c_) in enumerate(zip(offs.tolist(), cnt))]).to(BF)
+    assert torch.equal(c[:n].cpu(), ref[:, :N]) and torch.equal(pre[:n].cpu(), ref), name
+    gate, up = ref.float().chunk(2, dim=-1)
+    want = F.silu(gate).to(BF).float() * up
+    assert torch.allclose(act[:n].cpu().float(), want, rtol=2 ** -6, atol=1e-6), name
+    assert torch.equal(act, act2)
+    for t in (c, act, pre):
+        assert (t[n:].float() == 7.0).all(), "rows past offs[-1] were written"
+
+
 # Mean rows per expert on both sides of every bound of the row-tile rule, counts at the edges of the
 # 64- and 128-row tiles, K tails inside a 64-deep k-tile, weight rows of 4096 elements.
 ROW_TILE_CASES = [
