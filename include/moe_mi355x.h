@@ -269,6 +269,20 @@ int moe_dispatch_meta(const int64_t* ids, const float* scores,
                       int64_t k, int64_t* local_ids, float* routed_scores,
                       int64_t* source_tokens, void* stream);
 
+/* One owner's block, rows [lo, lo + rows) of the sorted order:
+ * scatter: block[pos_of_slot[t*k+j] - lo,:] = hidden[t,:] for the slots that
+ *   sort into the block, the others dropped;
+ * gather: out[t,:] = the sum of block[pos_of_slot[t*k+j] - lo,:] over the same
+ *   slots, fp32 in slot order, zeros for a token without any.
+ * bf16 rows, H % 8 == 0; each is the other's backward.  The exchange of
+ * token_dispatch.py:127-148 and :160-174 for a rank whose peers are absent. */
+int moe_scatter_block(const void* hidden, const int32_t* pos_of_slot, int64_t T,
+                      int64_t H, int64_t k, int64_t lo, int64_t rows,
+                      void* block, void* stream);
+int moe_gather_block(const void* block, const int32_t* pos_of_slot, int64_t T,
+                     int64_t H, int64_t k, int64_t lo, int64_t rows, void* out,
+                     void* stream);
+
 /* Backward of the row gather: d_hidden[t,:] = sum_j d_permuted[pos_of_slot[t*k+j],:]
  * over valid positions (pos < offsets[nb-1]), fp32 accumulation, plus
  * d_add[t,:] when d_add is not NULL; bf16 in and out.

@@ -59,6 +59,8 @@ SIGNATURES: dict[str, tuple] = {
     "moe_f32_combine_bwd": (_I, [_P, _P, _P, _P, _I64, _P, _I64, _I64, _I64, _P, _P, _P]),
     "moe_f32_permute_bwd": (_I, [_P, _P, _P, _I64, _I64, _I64, _I64, _P, _P, _P]),
     "moe_dispatch_meta": (_I, [_P, _P, _P, _I64, _I64, _I64, _P, _P, _P, _P]),
+    "moe_scatter_block": (_I, [_P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P]),
+    "moe_gather_block": (_I, [_P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P]),
     "moe_permute_bwd": (_I, [_P, _P, _P, _I64, _I64, _I64, _I64, _P, _P, _P]),
     "moe_combine_fwd": (_I, [_P, _P, _P, _I64, _P, _I64, _I64, _I64, _P, _P]),
     "moe_combine_bwd": (_I, [_P, _P, _P, _P, _I64, _P, _I64, _I64, _I64, _P, _P, _P]),

@@ -12,6 +12,7 @@ Ops (namespace ``parallel_amd``):
   permute_fwd                      stable sort of routed slots + row gather
   experts_fwd / experts_bwd        permute -> SwiGLU grouped GEMMs -> combine
   dispatch_fwd / dispatch_bwd      owner-rank sort for TokenDispatcher
+  scatter_block / gather_block     one owner's rows of that order, no others
   combine_rows_fwd / _bwd          gather-form index_add back to source tokens
   rmsnorm_fwd / rmsnorm_bwd        post_attention_layernorm of the block input (+ backward)
   router_aux_fwd                   router_fwd plus the aux loss from the same top-k
@@ -1275,3 +1276,117 @@ def _combine_backward(ctx, d_out):
 
 combine_rows_fwd.register_autograd(_combine_backward, setup_context=_combine_setup)
 run_combine_rows_fwd = _eager_route("combine_rows_fwd", combine_rows_fwd, _combine_setup, _combine_backward)
+
+
+# One rank's share of a dispatch whose other ranks are absent: only the rows of
+# its own block, [lo, lo + rows) of the owner-major order, are moved.  The full
+# order's rows with the others' dropped or zero-filled (dispatch_fwd and
+# combine_rows_fwd around variable_all_to_all) give the same values and remain
+# for calls that the ops' route takes.
+
+
+def _rows16(t: Tensor) -> Tensor:
+    """Contiguous rows at the 16-byte aligned address that the kernels load from."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+class _ScatterBlock(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, hidden, pos, top_k, lo, rows):
+        ctx.save_for_backward(pos)
+        ctx.block = (hidden.shape[0], top_k, lo)
+        T, H = hidden.shape
+        out = torch.empty(rows, H, dtype=BF16, device=hidden.device)
+        call("moe_scatter_block", ptr(hidden.contiguous()), ptr(pos), T, H, top_k, lo, rows, ptr(out), _stream(hidden))
+        return out
+
+    @staticmethod
+    def backward(ctx, d_block):
+        (pos,) = ctx.saved_tensors
+        return gather_block(d_block, pos, *ctx.block), None, None, None, None
+
+
+class _GatherBlock(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, block, pos, num_tokens, top_k, lo):
+        ctx.save_for_backward(pos)
+        ctx.block = (top_k, lo, block.shape[0])
+        rows, H = block.shape
+        out = torch.empty(num_tokens, H, dtype=BF16, device=block.device)
+        call("moe_gather_block", ptr(_rows16(block)), ptr(pos), num_tokens, H, top_k, lo, rows, ptr(out),
+             _stream(block))
+        return out
+
+    @staticmethod
+    def backward(ctx, d_out):
+        (pos,) = ctx.saved_tensors
+        return scatter_block(d_out, pos, *ctx.block), None, None, None, None
+
+
+class _BlockScores(torch.autograd.Function):
+    """The block's routed scores (already gathered in sorted order) as a function of the scores."""
+
+    @staticmethod
+    def forward(ctx, scores, sorted_scores, pos, lo, rows):
+        ctx.save_for_backward(pos)
+        ctx.scores = (scores.shape, scores.dtype, lo)
+        return sorted_scores[lo:lo + rows].to(scores.dtype, copy=True)
+
+    @staticmethod
+    def backward(ctx, d):
+        (pos,) = ctx.saved_tensors
+        shape, dtype, lo = ctx.scores
+        d = torch.nn.functional.pad(d, (lo, pos.numel() - lo - d.shape[0]))
+        return d.index_select(0, pos.long()).view(shape).to(dtype), None, None, None, None
+
+
+def scatter_block(hidden: Tensor, pos_of_slot: Tensor, top_k: int, lo: int, rows: int) -> Tensor:
+    """block[p - lo] = hidden[t] for the slots of token t with position p in [lo, lo + rows)."""
+    if _plain_eager((hidden, pos_of_slot)):
+        return _ScatterBlock.apply(hidden, pos_of_slot, top_k, lo, rows)
+    return _direct("combine_rows_bwd", hidden, pos_of_slot, top_k).narrow(0, lo, rows)
+
+
+def gather_block(block: Tensor, pos_of_slot: Tensor, num_tokens: int, top_k: int, lo: int) -> Tensor:
+    """out[t] = sum of block[p - lo] over the slots of token t with position p in [lo, lo + len(block))."""
+    if _plain_eager((block, pos_of_slot)):
+        return _GatherBlock.apply(block, pos_of_slot, num_tokens, top_k, lo)
+    rows = torch.nn.functional.pad(block, (0, 0, lo, num_tokens * top_k - lo - block.shape[0]))
+    return combine_rows_fwd(rows, pos_of_slot, num_tokens, top_k)
+
+
+def takes_block(*args) -> bool:
+    """Whether an exchange over these tensors may move the rank's own block only."""
+    rows = args[0]
+    return _plain_eager(args) and rows.dim() == 2 and rows.dtype == BF16
+
+
+def dispatch_sort(global_indices: Tensor, scores: Tensor, local_count: int,
+                  ep_size: int) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
+    """The owner-major order without its rows: (send_experts, sorted scores f32, source_tokens, pos_of_slot,
+    counts) as dispatch_fwd gives them."""
+    T, k = global_indices.shape
+    S = T * k
+    dev = global_indices.device
+    s = _stream(global_indices)
+    ids = _ids64(global_indices)
+    sc = scores.detach().float().contiguous()
+    perm, pos = torch.empty(2, S, dtype=torch.int32, device=dev).unbind()
+    counts, offsets = torch.empty(2, ep_size, dtype=torch.int32, device=dev).unbind()
+    ws = _ws(_lib.load().moe_permute_workspace_bytes(S, ep_size), dev)
+    call("moe_permute_fwd", None, T, 0, ptr(ids), k, local_count, ep_size, None, ptr(perm), ptr(pos), ptr(counts),
+         ptr(offsets), ptr(ws), ws.numel(), s)
+    send_experts = torch.empty(S, dtype=torch.int64, device=dev)
+    sorted_scores = torch.empty(S, dtype=torch.float32, device=dev)
+    source_tokens = torch.empty(S, dtype=torch.int64, device=dev)
+    call("moe_dispatch_meta", ptr(ids), ptr(sc), ptr(perm), S, local_count, k, ptr(send_experts), ptr(sorted_scores),
+         ptr(source_tokens), s)
+    return send_experts, sorted_scores, source_tokens, pos, counts
+
+
+def block_scores(scores: Tensor, sorted_scores: Tensor, pos_of_slot: Tensor, lo: int, rows: int) -> Tensor:
+    """The block's entries of sorted_scores, in the scores' dtype and differentiable in the scores."""
+    if _wants_grad((scores,)):
+        return _BlockScores.apply(scores, sorted_scores, pos_of_slot, lo, rows)
+    return sorted_scores.narrow(0, lo, rows).to(scores.dtype)

@@ -106,6 +106,9 @@ class TokenDispatcher:
         if global_indices.shape != scores.shape:
             raise ValueError("Expert indices and scores must have the same shape")
         tokens, top_k = global_indices.shape
+        if (self.world_size > 1 and ops.takes_block(hidden_states, global_indices, scores)
+                and hidden_states.shape[0] == tokens):
+            return self._dispatch_block(hidden_states, global_indices, scores)
         send_hidden, send_experts, send_scores, source_tokens, pos_of_slot, counts = ops.run_dispatch_fwd(
             hidden_states, global_indices, scores, self.partition.local_count, self.partition.ep_size
         )
@@ -116,7 +119,34 @@ class TokenDispatcher:
         state = DispatchState(send_splits, receive_splits, source_tokens, tokens, pos_of_slot, top_k)
         return received_hidden, received_experts.unsqueeze(-1), received_scores.unsqueeze(-1), state
 
+    def _dispatch_block(self, hidden_states, global_indices, scores):
+        """dispatch with only this rank's block of the send rows written: the others would be dropped by
+        the exchange, and they are most of the bytes."""
+        tokens, top_k = global_indices.shape
+        send_experts, sorted_scores, source_tokens, pos_of_slot, counts = ops.dispatch_sort(
+            global_indices, scores, self.partition.local_count, self.world_size
+        )
+        send, receive = self._exchange_splits(counts)
+        if sum(send) != tokens * top_k:  # routes to experts of no rank
+            raise ValueError(f"send splits {send} do not cover the {tokens * top_k} rows to send")
+        lo, rows = _block_start(send, self.rank), send[self.rank]
+        received_hidden = ops.scatter_block(hidden_states, pos_of_slot, top_k, lo, rows)
+        received_scores = ops.block_scores(scores, sorted_scores, pos_of_slot, lo, rows)
+        state = DispatchState(send, receive, source_tokens, tokens, pos_of_slot, top_k)
+        return (received_hidden, send_experts.narrow(0, lo, rows).unsqueeze(-1), received_scores.unsqueeze(-1), state)
+
+    def _own_block(self, expert_output, state):
+        """Whether expert_output is this rank's block of a well-formed state and nothing else."""
+        send, receive, rank = state.send_splits, state.receive_splits, self.rank
+        return (self.world_size > 1 and state.pos_of_slot is not None and len(send) == len(receive) == self.world_size
+                and send[rank] == receive[rank] == sum(receive) == expert_output.shape[0]
+                and sum(send) == state.pos_of_slot.numel() == state.num_source_tokens * state.top_k
+                and ops.takes_block(expert_output, state.pos_of_slot))
+
     def combine(self, expert_output: torch.Tensor, state: DispatchState):
+        if self._own_block(expert_output, state):
+            return ops.gather_block(expert_output, state.pos_of_slot, state.num_source_tokens, state.top_k,
+                                    _block_start(state.send_splits, self.rank))
         returned = self._exchange(expert_output, state.receive_splits, state.send_splits, "combine_hidden")
         if state.pos_of_slot is None:
             raise ValueError("DispatchState has no inverse permutation; it was not produced by this dispatcher")

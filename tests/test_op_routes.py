@@ -7,7 +7,7 @@ import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
-from parallel_amd import ops
+from parallel_amd import ExpertPartition, TokenDispatcher, _lib, ops
 
 BF = torch.bfloat16
 
@@ -107,3 +107,71 @@ def test_direct_calls_keep_hooks_and_in_place_outputs():
     h += 1  # a fresh tensor, not a view: in-place use stays legal
     (out.float().sum() + h.float().sum()).backward()
     assert all(v.grad is not None for v in (x, rw, gu, dn))
+
+
+def _dispatch_pass(T, E, k, H, ep, rank, layout):
+    """Dispatch, an elementwise stand-in for the experts and combine, forward and backward."""
+    g = torch.Generator().manual_seed(T + k)
+    ids = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]).cuda()
+    if layout == "none":  # no route of this rank
+        ids = (ids % (E // ep) + ((rank + 1) % ep) * (E // ep))
+    scores = torch.rand(T, k, generator=g).cuda().requires_grad_()
+    hidden = torch.randn(T, H, generator=g).to(BF).cuda().requires_grad_()
+    d_out = torch.randn(T, H, generator=g).to(BF).cuda()
+    dispatcher = TokenDispatcher(ExpertPartition(E, ep, rank), None)
+    received, experts, rscores, state = dispatcher.dispatch(hidden, ids, scores)
+    rows = received * 1.5
+    if layout == "strided":
+        rows = torch.cat([rows, rows], dim=1)[:, :H]
+    elif layout == "misaligned":
+        rows = torch.cat([rows.new_zeros(3), rows.reshape(-1)])[3:].view(-1, H)
+    out = dispatcher.combine(rows, state)
+    grads = torch.autograd.grad([out, rscores], [hidden, scores], [d_out, torch.ones_like(rscores)])
+    return [received.detach(), experts, rscores.detach(), state.source_tokens, state.pos_of_slot, out.detach(), *grads], (
+        state.send_splits, state.receive_splits)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,k,H,ep,rank,layout", [
+    (1, 8, 1, 8, 2, 0, "plain"),          # one row of one 16-byte chunk
+    (1, 8, 2, 2048, 4, 3, "plain"),
+    (37, 16, 3, 264, 4, 1, "strided"),    # slot count at run time, a partial pass of the lanes
+    (64, 128, 8, 2056, 2, 1, "plain"),    # 512 slots, the last size of the one-launch sort; one chunk past 2048
+    (65, 128, 8, 512, 2, 0, "misaligned"),
+    (300, 64, 6, 1536, 2, 1, "plain"),
+    (33, 16, 16, 64, 4, 2, "plain"),
+    (50, 16, 2, 128, 4, 2, "none"),
+])
+def test_own_block_exchange_gives_the_full_exchanges_bits(T, E, k, H, ep, rank, layout):
+    got, splits = _dispatch_pass(T, E, k, H, ep, rank, layout)
+    with _Seen() as seen:
+        want, want_splits = _dispatch_pass(T, E, k, H, ep, rank, layout)
+    assert any("combine_rows_fwd" in n for n in seen.names)
+    assert splits == want_splits
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), f"result {i}"
+
+
+@pytest.mark.gpu
+def test_own_block_exchange_differentiates_twice():
+    """Dispatch and combine are linear: the gradient as a function of d_out has the forward as its gradient."""
+    ids = torch.tensor([[0, 5], [6, 1], [7, 4]], device="cuda")
+    hidden = torch.randn(3, 64, device="cuda").to(BF).requires_grad_()
+    d_out = torch.randn(3, 64, device="cuda").to(BF).requires_grad_()
+    dispatcher = TokenDispatcher(ExpertPartition(8, 2, 1), None)
+    received, _, _, state = dispatcher.dispatch(hidden, ids, torch.rand(3, 2, device="cuda"))
+    (dh,) = torch.autograd.grad(dispatcher.combine(received, state), hidden, d_out, create_graph=True)
+    (dd,) = torch.autograd.grad(dh, d_out, torch.ones_like(dh))
+    count = torch.tensor([1, 1, 2], device="cuda").unsqueeze(1)
+    assert torch.equal(dh, count * d_out) and torch.equal(dd, count.to(BF).expand(3, 64))
+
+
+def test_block_entry_points_check_their_arguments():
+    lib, buf = _lib.load(), torch.zeros(64, dtype=torch.int64)
+    b = (buf.data_ptr() + 15) // 16 * 16
+    for entry in (lib.moe_scatter_block, lib.moe_gather_block):
+        assert entry(None, None, 0, 64, 2, 0, 0, None, None) == _lib.MOE_OK
+        for T, H, k, lo, rows in ((2, 64, 2, 3, 2), (2, 64, 2, -1, 1), (2, 60, 2, 0, 1), (2, 64, 17, 0, 1)):
+            assert entry(b, b, T, H, k, lo, rows, b, None) == _lib.MOE_ERR_INVALID
+        assert entry(b, None, 2, 64, 2, 0, 1, b, None) == _lib.MOE_ERR_INVALID
+        assert entry(b + 4, b, 2, 64, 2, 0, 1, b + 4, None) == _lib.MOE_ERR_INVALID
