@@ -15,6 +15,8 @@
 // (H <= 64 * 8 * kNormMaxChunks).  The weight gradient is a column sum over
 // the rows: per-block partials (each block's 4 rows, wave order), then row
 // groups, then the groups in order; every sum has a fixed order.
+#include <type_traits>
+
 #include "common.h"
 
 namespace moe {
@@ -77,31 +79,36 @@ __global__ __launch_bounds__(kNormWaves * kWave) void rmsnorm_fwd_kernel(const b
 }
 
 // dh per row, and per-block partial column sums of bf16(g * bf16(hs)) into
-// partials[block][H] (the block's rows added in wave order).
+// partials[block][H] (the block's rows added in wave order).  Instantiated for
+// the 16-byte chunks per lane that H needs: registers and LDS for
+// kNormMaxChunks of them, whatever H, left two blocks per CU (the whole entry
+// point at H 2048: 5000 rows 23.1 -> 19.1 us, 16384 rows 51.5 -> 44.7; H 1536,
+// 5000 rows 20.0 -> 16.1; H 4096 33.5 -> 31.9).  Bound by the row streams and
+// the partials.  Waves that walk several rows with the sums in registers write
+// fewer partials, but their registers leave one or two waves per SIMD: 21.7
+// and 42.7 at H 2048, and slower than this below 4000 rows and at H 4096 (44.3).
+template <int NC>
 __global__ __launch_bounds__(kNormWaves * kWave) void rmsnorm_bwd_kernel(
     const bf16_t* __restrict__ dx, const bf16_t* __restrict__ dx2, const bf16_t* __restrict__ h,
     const bf16_t* __restrict__ gamma, const float* __restrict__ rstd, int T, int H, bf16_t* __restrict__ dh,
     float* __restrict__ partials) {
-  __shared__ float part[kNormWaves][kNormMaxChunks * 8 * kWave];
+  // [wave][element of the chunk][chunk]: neighbouring lanes on neighbouring banks.
+  __shared__ float part[kNormWaves][8][NC * kWave];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
   const int t = blockIdx.x * kNormWaves + wave;
   const int nchunk = H / 8;
-  const bool live = t < T;
-  float dg[kNormMaxChunks][8];  // this row's contribution to the weight gradient
-  if (live) {
+  if (t < T) {
     const int64_t base = static_cast<int64_t>(t) * H;
     const uint4* hr = reinterpret_cast<const uint4*>(h + base);
     const uint4* gr = reinterpret_cast<const uint4*>(dx + base);
     const uint4* gr2 = dx2 ? reinterpret_cast<const uint4*>(dx2 + base) : nullptr;
     const uint4* gw = reinterpret_cast<const uint4*>(gamma);
     const float r = rstd[t];
-    float hv[kNormMaxChunks][8], dhs[kNormMaxChunks][8];
+    float hv[NC][8], dhs[NC][8];
     float dot = 0.0f;
 #pragma unroll
-    for (int i = 0; i < kNormMaxChunks; ++i) {
+    for (int i = 0; i < NC; ++i) {
       const int c = lane + i * kWave;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) dg[i][e] = hv[i][e] = dhs[i][e] = 0.0f;
       if (c < nchunk) {
         float g[8], g2[8], w[8];
         unpack8f(hr[c], hv[i]);
@@ -116,7 +123,7 @@ __global__ __launch_bounds__(kNormWaves * kWave) void rmsnorm_bwd_kernel(
         for (int e = 0; e < 8; ++e) {
           dhs[i][e] = round_bf16f(g[e] * w[e]);
           dot += dhs[i][e] * hv[i][e];
-          dg[i][e] = round_bf16f(g[e] * round_bf16f(hv[i][e] * r));
+          part[wave][e][c] = round_bf16f(g[e] * round_bf16f(hv[i][e] * r));
         }
       }
     }
@@ -124,7 +131,7 @@ __global__ __launch_bounds__(kNormWaves * kWave) void rmsnorm_bwd_kernel(
     const float k3 = r * r * r / static_cast<float>(H);
     uint4* out = reinterpret_cast<uint4*>(dh + base);
 #pragma unroll
-    for (int i = 0; i < kNormMaxChunks; ++i) {
+    for (int i = 0; i < NC; ++i) {
       const int c = lane + i * kWave;
       if (c < nchunk) {
         float o[8];
@@ -134,23 +141,20 @@ __global__ __launch_bounds__(kNormWaves * kWave) void rmsnorm_bwd_kernel(
       }
     }
   } else {
+    for (int c = lane; c < nchunk; c += kWave)
 #pragma unroll
-    for (int i = 0; i < kNormMaxChunks; ++i)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) dg[i][e] = 0.0f;
+      for (int e = 0; e < 8; ++e) part[wave][e][c] = 0.0f;
   }
-#pragma unroll
-  for (int i = 0; i < kNormMaxChunks; ++i)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) part[wave][(i * kWave + lane) * 8 + e] = dg[i][e];
   __syncthreads();
   float* prow = partials + static_cast<int64_t>(blockIdx.x) * H;
-  for (int j = threadIdx.x; j < H; j += blockDim.x) {
-    // column j lives at chunk j/8 = i*64 + lane, element j%8
-    float s = 0.0f;
+  for (int c = threadIdx.x; c < nchunk; c += kNormWaves * kWave) {
 #pragma unroll
-    for (int w = 0; w < kNormWaves; ++w) s += part[w][j];
-    prow[j] = s;
+    for (int e = 0; e < 8; ++e) {
+      float s = 0.0f;
+#pragma unroll
+      for (int w = 0; w < kNormWaves; ++w) s += part[w][e][c];
+      prow[8 * c + e] = s;
+    }
   }
 }
 
@@ -237,10 +241,22 @@ extern "C" int moe_rmsnorm_bwd(const void* dx, const void* dx2, const void* h, c
   float* partials = static_cast<float*>(workspace);
   float* sums = partials + static_cast<int64_t>(nblk) * H;
   if (T > 0) {
-    hipLaunchKernelGGL(rmsnorm_bwd_kernel, dim3(nblk), dim3(kNormWaves * kWave), 0, st,
-                       static_cast<const bf16_t*>(dx), static_cast<const bf16_t*>(dx2),
-                       static_cast<const bf16_t*>(h), static_cast<const bf16_t*>(gamma), rstd, static_cast<int>(T),
-                       static_cast<int>(H), static_cast<bf16_t*>(dh), partials);
+    auto launch = [&](auto NC) {
+      hipLaunchKernelGGL((rmsnorm_bwd_kernel<decltype(NC)::value>), dim3(nblk), dim3(kNormWaves * kWave), 0, st,
+                         static_cast<const bf16_t*>(dx), static_cast<const bf16_t*>(dx2),
+                         static_cast<const bf16_t*>(h), static_cast<const bf16_t*>(gamma), rstd, static_cast<int>(T),
+                         static_cast<int>(H), static_cast<bf16_t*>(dh), partials);
+    };
+    const int64_t nc = (H / 8 + kWave - 1) / kWave;  // 16-byte chunks per lane
+    if (nc <= 1) {
+      launch(std::integral_constant<int, 1>{});
+    } else if (nc <= 2) {
+      launch(std::integral_constant<int, 2>{});
+    } else if (nc <= 4) {
+      launch(std::integral_constant<int, 4>{});
+    } else {
+      launch(std::integral_constant<int, kNormMaxChunks>{});
+    }
     rc = launch_status("moe_rmsnorm_bwd(rows)");
     if (rc) return rc;
   }

@@ -8,7 +8,7 @@ import torch
 
 from conftest import GOLDEN, close_bf16, routing_check
 from oracle import moe_oracle as O
-from parallel_amd import norm_router_aux, ops
+from parallel_amd import _lib, norm_router_aux, ops
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -57,6 +57,37 @@ def test_rmsnorm_shapes_against_oracle(T, H):
     close_bf16(x, xr, f"x T{T} H{H}", max_rel=8e-3)
     close_bf16(hd.grad, hc.grad, f"dh T{T} H{H}", max_rel=1e-2)
     close_bf16(wd.grad, wc.grad, f"dweight T{T} H{H}", max_rel=1e-2)
+
+
+@pytest.mark.parametrize("T,H", [(1, 512), (2049, 520), (2048, 1024), (5, 1032), (6150, 2048), (1025, 2056),
+                                 (3000, 4088)])
+def test_rmsnorm_backward_chunk_counts(T, H):
+    """Chunk counts per lane (1, 2, 4, 8) at and past their edges, a last block with idle waves, and dx2:
+    against fp64 sums of the same bf16 products."""
+    g = gen(T + H)
+    h = (torch.randn(T, H, generator=g) * 2).to(DEV, BF)
+    w = (1 + 0.2 * torch.randn(H, generator=g)).to(DEV, BF)
+    dx, dx2 = (torch.randn(T, H, generator=g).to(DEV, BF) for _ in range(2))
+    rstd = torch.empty(T, dtype=torch.float32, device=DEV)
+    x, dh, dw = torch.empty_like(h), torch.empty_like(h), torch.empty_like(w)
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.call("moe_rmsnorm_fwd", h.data_ptr(), w.data_ptr(), T, H, EPS, x.data_ptr(), rstd.data_ptr(), stream)
+    n = _lib.load().moe_rmsnorm_bwd_workspace_bytes(T, H)
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    _lib.call("moe_rmsnorm_bwd", dx.data_ptr(), dx2.data_ptr(), h.data_ptr(), w.data_ptr(), rstd.data_ptr(), T, H,
+              dh.data_ptr(), dw.data_ptr(), ws.data_ptr(), n, stream)
+    hs = (h.float() * rstd.unsqueeze(1)).to(BF)
+    gsum = dx + dx2
+    prod = (gsum * hs).double()
+    want_dw = prod.sum(0)
+    # fp32 sums of at most T terms in any order, then one bf16 rounding
+    bound = want_dw.abs() * 2.0 ** -8 + prod.abs().sum(0) * T * 2.0 ** -24
+    assert bool(((dw.double() - want_dw).abs() <= bound).all())
+    dhs, hd, r = (gsum * w).double(), h.double(), rstd.double().unsqueeze(1)
+    want = r * dhs - r ** 3 * hd * (dhs * hd).mean(1, keepdim=True)
+    # a sum of two fp32 terms, the second's dot product of H terms, then one bf16 rounding
+    size = (r * dhs).abs() + r ** 3 * hd.abs() * (dhs * hd).abs().mean(1, keepdim=True)
+    assert bool(((dh.double() - want).abs() <= want.abs() * 2.0 ** -8 + size * (H + 8) * 2.0 ** -24).all())
 
 
 @pytest.mark.parametrize("T,H,E,k,masked,biased", [(4096, 2048, 128, 8, False, False), (300, 64, 64, 6, True, True),
