@@ -131,8 +131,8 @@ _GEMM_ORDER = {
 def tag_dispatches(names):
     """Bench timer tag of each kernel dispatch, given kernel names in dispatch order.
 
-    The expert GEMMs are the grouped_gemm instantiations with tiles of 256
-    columns (the router GEMMs use 128-column tiles); entry points that share a
+    The expert GEMMs are the grouped_gemm instantiations with tiles of 256 or
+    more rows or columns (the router GEMMs use 128x128 tiles); entry points that share a
     (mode, operand layout, epilogue) signature are told apart by their
     occurrence order (each step launches them in a fixed order)."""
     import re
@@ -143,7 +143,7 @@ def tag_dispatches(names):
     for n, m in zip(names, parsed):
         if m:
             key = (int(m[1]), m[2] == "true", int(m[3]))
-            if int(m[4].split(",")[1]) >= 256 and key in _GEMM_ORDER:
+            if max(map(int, m[4].split(",")[:2])) >= 256 and key in _GEMM_ORDER:
                 order = _GEMM_ORDER[key]
                 i = seen.get(key, 0)
                 seen[key] = i + 1
