@@ -1329,7 +1329,7 @@ int launch_expert(GemmParams& p, hipStream_t stream, const char* name) {
   const int out_cols = (EPI == EPI_SWIGLU_FWD) ? 2 * p.swiglu_I : p.N;
   const int64_t rows = p.rows, G = p.G;
   if constexpr (B_KCONTIG) {
-    if (rows <= kFewMaxMeanRows * G && few_rows_takes(p.K)) {
+    if (p.offs && rows <= kFewMaxMeanRows * G && few_rows_takes(p.K)) {  // (a single group without offsets: the tiles)
       constexpr bool swiglu = EPI == EPI_SWIGLU_FWD;
       return few_rows(FewRows{p.A, p.B, static_cast<bf16_t*>(p.C), static_cast<bf16_t*>(p.C2), p.offs, p.G, p.rows,
                               swiglu ? p.swiglu_I : p.N, p.K},

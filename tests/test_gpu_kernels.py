@@ -499,6 +499,25 @@ def test_few_rows_forward_is_exact_on_integers(name, cnt, N, K):
         assert (t[n:].float() == 7.0).all(), "rows past offs[-1] were written"
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 64, 512), (2, 72, 2048), (3, 64, 512), (2, 40, 264), (1, 64, 4096)])
+def test_forward_of_a_single_group_without_offsets(M, N, K):
+    """offs may be NULL for one group of M rows, however few: both forward entry points on exact integers."""
+    a = torch.randint(-1, 2, (M, K), generator=gen(41)).to(BF)
+    w = torch.randint(-1, 2, (2 * N, K), generator=gen(42)).to(BF)
+    ad, wd = a.to(DEV), w.to(DEV)
+    c, pre = (torch.full((M, 2 * N), 7.0, dtype=BF, device=DEV) for _ in range(2))
+    act = torch.full((M, N), 7.0, dtype=BF, device=DEV)
+    s = _lib.stream_of(c)
+    _lib.call("moe_grouped_gemm_fwd", ad.data_ptr(), wd.data_ptr(), None, 1, M, 2 * N, K, c.data_ptr(), s)
+    _lib.call("moe_grouped_gemm_swiglu_fwd", ad.data_ptr(), wd.data_ptr(), None, 1, M, K, N, act.data_ptr(),
+              pre.data_ptr(), s)
+    torch.cuda.synchronize()
+    ref = (a.double() @ w.double().t()).to(BF)
+    assert torch.equal(c.cpu(), ref) and torch.equal(pre.cpu(), ref)
+    gate, up = ref.float().chunk(2, dim=-1)
+    assert torch.allclose(act.cpu().float(), F.silu(gate).to(BF).float() * up, rtol=2 ** -6, atol=1e-6)
+
+
 # Mean rows per expert on both sides of every bound of the row-tile rule, counts at the edges of the
 # 64- and 128-row tiles, K tails inside a 64-deep k-tile, weight rows of 4096 elements.
 ROW_TILE_CASES = [
