@@ -3,44 +3,45 @@
 //
 // The tiled kernel (grouped_gemm.hip) gives such an expert ceil(N / 256) blocks
 // that each walk all of K, so one decoded token keeps 48 of 256 CUs busy, and
-// it stages the weights through LDS behind a block barrier per k-tile.  Here a
-// block takes 16 or more weight rows of one expert and splits K over its eight
-// waves, so that the same token gives 384 blocks; a wave loads its weights
-// straight into the MFMA operand registers, up to 16 loads of 1 KiB in flight,
-// with the next tile's loads issued as the current tile's operands are used.
-// The rows of the expert (16 at a time) stay in registers while the block
-// walks its run of tiles.  The waves' partial sums meet in LDS, one barrier
-// per tile.  Bound by the weights' bytes from a few tokens on (16 tokens at
-// H 2048, I 768, 128 experts, top-8: 5.1 TB/s; the tiled kernel 4.4), by
-// latency and the launch for one token.
-#include <algorithm>
-
+// it stages the weights through LDS behind a block barrier per k-tile.  Here
+// every wave is a block of its own and takes 16 weight rows (SwiGLU: 16 gate
+// rows and the matching 16 up rows) of one expert for 16 of its rows: 384 waves
+// for the same token.  A wave walks all of K in order, so that an output's
+// products are added exactly as the tiled kernel adds them: a token's results
+// are the same bits in a batch of any size.  Weights and rows go straight into
+// the MFMA operand registers, D k-steps of loads in flight; there is no LDS and
+// no barrier.  Bound by the weights' bytes from a few tokens on, by latency and
+// the launch for one token.
+//
+// Up / down projection in us, weights out of the caches, against the 64-row
+// tile: H 2048, I 768, 128 experts, 8 rows of 8 experts 25/16 against 38/22,
+// one row in each of 64 134/80 against 140/85, 256 rows 193/126 against 194/126;
+// H 4096, I 1536: 81/43 against 91/47 and 553/298 against 582/315 (8 and 256
+// rows).  Reductions that are no multiple of anything: K 2304 / 1000 (H 2304,
+// I 1000, 64 experts, 64 rows) 161/109 against 165/123, K 2560 (32 experts, 8
+// rows) 85/44 against 87/55, K 14336 (8 experts, 8 rows) 231 against 257.
+// Skewed (a sixteenth of the experts holds all rows, 16 rows each) 31/20 against
+// 40/22.  In flight: 12 k-steps of the up projection (8: 1.00 of the time, 4:
+// 1.05, 24: 1.04, over sizes), 16 of the down projection (8: 1.02, 24: 1.00).
 #include "dma.h"
 #include "gemm.h"
 
 namespace moe {
 namespace {
 
-constexpr int kFewWaves = 8;
 constexpr int kFewXcd = 8;
-constexpr int kPartRow = 20;  // floats per row of a 16 x 16 partial: the four row groups of a write hit distinct banks
 
-// KS: 32-deep k-steps per wave; NT: 16-row weight sub-tiles per tile (SWIGLU:
-// NT 2, the gate rows and the matching up rows).
-template <int KS, int NT, bool SWIGLU>
-__global__ __launch_bounds__(kFewWaves * kWave) void few_rows_kernel(const FewRows p, int n_tiles, uint32_t a_bytes,
-                                                                     uint32_t w_bytes) {
-  constexpr int L = KS * NT;             // loads per tile and wave
-  constexpr int R = L <= 16 ? L : 16;    // ... in flight
-  static_assert(L % R == 0 && (!SWIGLU || NT == 2), "a load's register is the same in every tile");
-  __shared__ float part[2][kFewWaves][NT][16][kPartRow];
-  const int tid = threadIdx.x, lane = tid & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+// D: k-steps (32 deep) of loads in flight.
+template <int D, bool SWIGLU>
+__global__ __launch_bounds__(kWave) void few_rows_kernel(const FewRows p, int n_tiles, uint32_t a_bytes,
+                                                         uint32_t w_bytes) {
+  constexpr int NT = SWIGLU ? 2 : 1;  // 16-row weight tiles: the gate rows and the matching up rows
+  const int lane = threadIdx.x;
   const int i16 = lane & 15, q = lane >> 4;
 
-  // Tiles in group-major order, then 16-row chunk, then weight rows; an XCD's
-  // blocks take neighbouring runs.
-  auto chunks_of = [&](int g, int& lo) {
+  // Tasks in group-major order, then weight tile, then 16-row chunk (whose
+  // waves read the same weights); an XCD's blocks take neighbouring tasks.
+  auto rows_of = [&](int g, int& lo) {
     int hi = 0;
     lo = 0;
     if (g < p.G) {
@@ -52,177 +53,119 @@ __global__ __launch_bounds__(kFewWaves * kWave) void few_rows_kernel(const FewRo
   int chunks = 0;  // 16-row chunks over all groups
   for (int c0 = 0; c0 < p.G; c0 += kWave) {
     int lo;
-    const int cnt = chunks_of(c0 + lane, lo);
+    const int cnt = rows_of(c0 + lane, lo);
     chunks += __builtin_amdgcn_readlane(wave_inclusive_scan((cnt + 15) / 16), kWave - 1);
   }
-  const int64_t total = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(chunks)) * n_tiles;
-  const int nb = gridDim.x, lb = (blockIdx.x % kFewXcd) * (nb / kFewXcd) + blockIdx.x / kFewXcd;
-  const int64_t t_begin = total * lb / nb, t_end = total * (lb + 1) / nb;
-  if (t_begin >= t_end) return;
-
-  struct Tile {
-    int g, r0, rows, nt;  // group, first row, rows (at most 16), weight tile
-  };
-  auto locate = [&](int64_t t) {
-    const int chunk = static_cast<int>(t / n_tiles);
-    Tile d{0, 0, 0, static_cast<int>(t - static_cast<int64_t>(chunk) * n_tiles)};
-    int base = 0;
-    for (int c0 = 0; c0 < p.G; c0 += kWave) {
-      int lo;
-      const int cnt = chunks_of(c0 + lane, lo);
-      const int n = (cnt + 15) / 16;
-      const int incl = wave_inclusive_scan(n);
-      const int tot = __builtin_amdgcn_readlane(incl, kWave - 1);
-      if (chunk < base + tot) {
-        const int w = __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(base + incl > chunk)));
-        const int local = chunk - base - __builtin_amdgcn_readlane(incl - n, w);
-        d.g = c0 + w;
-        d.r0 = __builtin_amdgcn_readlane(lo, w) + 16 * local;
-        d.rows = min(16, __builtin_amdgcn_readlane(cnt, w) - 16 * local);
-        break;
-      }
-      base += tot;
+  const int total = __builtin_amdgcn_readfirstlane(chunks) * n_tiles;
+  const int share = (total + kFewXcd - 1) / kFewXcd;
+  const int idx = blockIdx.x / kFewXcd, task = (blockIdx.x % kFewXcd) * share + idx;
+  if (idx >= share || task >= total) return;
+  int g = 0, r0 = 0, rows = 0, tile = 0;
+  for (int c0 = 0, base = 0; c0 < p.G; c0 += kWave) {
+    int lo;
+    const int cnt = rows_of(c0 + lane, lo);
+    const int n = n_tiles * ((cnt + 15) / 16);
+    const int incl = wave_inclusive_scan(n);
+    const int tot = __builtin_amdgcn_readlane(incl, kWave - 1);
+    if (task < base + tot) {
+      const int w = __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(base + incl > task)));
+      const int local = task - base - __builtin_amdgcn_readlane(incl - n, w);
+      const int gc = __builtin_amdgcn_readlane(cnt, w), nc = (gc + 15) / 16;
+      tile = local / nc;
+      const int chunk = local - tile * nc;
+      g = c0 + w;
+      r0 = __builtin_amdgcn_readlane(lo, w) + 16 * chunk;
+      rows = min(16, gc - 16 * chunk);
+      break;
     }
-    return d;
-  };
+    base += tot;
+  }
 
-  const int kb = wave * KS * 32 + 8 * q;  // this lane's first k
+  // Lane (i16, q): row i16 of each operand, k 8 q .. 8 q + 7 of a k-step.
   const __amdgpu_buffer_rsrc_t rsA = make_rsrc(p.A, a_bytes);
-  bf16x8_t xf[KS];
-  auto load_x = [&](const Tile& d) __attribute__((always_inline)) {
-    const uint32_t off = i16 < d.rows ? (static_cast<uint32_t>(d.r0 + i16) * static_cast<uint32_t>(p.K) +
-                                         static_cast<uint32_t>(kb)) * 2u
-                                      : kOOB;
+  const __amdgpu_buffer_rsrc_t rsW = make_rsrc(p.W + static_cast<int64_t>(g) * (SWIGLU ? 2 : 1) * p.N * p.K, w_bytes);
+  const uint32_t k2 = static_cast<uint32_t>(p.K) * 2u, lane_k = 16u * q;
+  const uint32_t x_row = i16 < rows ? static_cast<uint32_t>(r0 + i16) * k2 + lane_k : kOOB;
+  uint32_t w_row[NT];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      xf[ks] = __builtin_bit_cast(
-          bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rsA, kb + 32 * ks < p.K ? off + 64u * ks : kOOB, 0, 0));
-  };
-  // Byte offset of the lane's weight row and first k, per sub-tile.
-  auto w_off = [&](const Tile& d, int s) __attribute__((always_inline)) {
-    const int n = SWIGLU ? d.nt * 16 + i16 : (d.nt * NT + s) * 16 + i16;
-    const int row = SWIGLU ? s * p.N + n : n;
-    return n < p.N ? (static_cast<uint32_t>(row) * static_cast<uint32_t>(p.K) + static_cast<uint32_t>(kb)) * 2u : kOOB;
-  };
-  auto w_rsrc = [&](const Tile& d) __attribute__((always_inline)) {
-    return make_rsrc(p.W + static_cast<int64_t>(d.g) * (SWIGLU ? 2 : 1) * p.N * p.K, w_bytes);
-  };
-  u32x4_t wf[R];
-  auto load_w = [&](__amdgpu_buffer_rsrc_t rs, const uint32_t (&off)[NT], int i) __attribute__((always_inline)) {
-    const int s = i / KS, ks = i % KS;
+  for (int s = 0; s < NT; ++s) {
+    const int n = tile * 16 + i16;
+    w_row[s] = n < p.N ? static_cast<uint32_t>(s * p.N + n) * k2 + lane_k : kOOB;
+  }
+  u32x4_t xf[D], wf[D][NT];
+  auto load = [&](int u, int ks) __attribute__((always_inline)) {
+    const uint32_t off = 64u * ks;
+    const bool in = lane_k + off < k2;
     // (Not non-temporal: an operand load takes 64 bytes of each row, and the
-    // line has to stay for the next one: up and down projection of 16 tokens
-    // 109 + 58 us non-temporal against 105 + 52, H 2048, I 768, 128 experts.)
-    wf[i % R] = __builtin_amdgcn_raw_buffer_load_b128(rs, kb + 32 * ks < p.K ? off[s] + 64u * ks : kOOB, 0, 0);
+    // line has to stay for the next one.)
+#pragma unroll
+    for (int s = 0; s < NT; ++s) wf[u][s] = __builtin_amdgcn_raw_buffer_load_b128(rsW, in ? w_row[s] + off : kOOB, 0, 0);
+    xf[u] = __builtin_amdgcn_raw_buffer_load_b128(rsA, in ? x_row + off : kOOB, 0, 0);
   };
-
-  Tile cur = locate(t_begin);
-  __amdgpu_buffer_rsrc_t rs_cur = w_rsrc(cur);
-  uint32_t off_cur[NT];
+  f32x4_t acc[NT];
 #pragma unroll
-  for (int s = 0; s < NT; ++s) off_cur[s] = w_off(cur, s);
-  load_x(cur);
-#pragma unroll
-  for (int i = 0; i < R; ++i) load_w(rs_cur, off_cur, i);
-  int buf = 0;
-  for (int64_t t = t_begin; t < t_end; ++t) {
-    const bool more = t + 1 < t_end;
-    Tile nxt = cur;
-    ++nxt.nt;
-    if (more && nxt.nt == n_tiles) nxt = locate(t + 1);
-    const __amdgpu_buffer_rsrc_t rs_nxt = w_rsrc(nxt);
-    uint32_t off_nxt[NT];
-#pragma unroll
-    for (int s = 0; s < NT; ++s) off_nxt[s] = more ? w_off(nxt, s) : kOOB;
-    f32x4_t acc[NT];
-#pragma unroll
-    for (int s = 0; s < NT; ++s) acc[s] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int i = 0; i < L; ++i) {
-      acc[i / KS] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[i % KS], __builtin_bit_cast(bf16x8_t, wf[i % R]),
-                                                            acc[i / KS], 0, 0, 0);
-      if (i + R < L) {
-        load_w(rs_cur, off_cur, i + R);
-      } else {
-        load_w(rs_nxt, off_nxt, i + R - L);
-      }
-    }
-    if (more && (nxt.g != cur.g || nxt.r0 != cur.r0)) load_x(nxt);
-    // Lane (i16, q) holds rows 4 q + i, weight row i16 of each sub-tile.
+  for (int s = 0; s < NT; ++s) acc[s] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  auto multiply = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < NT; ++s)
+      acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[u][s]),
+                                                       __builtin_bit_cast(bf16x8_t, xf[u]), acc[s], 0, 0, 0);
+  };
+  const int nks = (p.K + 31) / 32;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) part[buf][wave][s][4 * q + i][i16] = acc[s][i];
-    // (The other buffer is read before the next tile's barrier and written after it.)
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    auto sum = [&](int s, int m, int n) __attribute__((always_inline)) {
-      float v = part[buf][0][s][m][n];
+  for (int u = 0; u < D; ++u) load(u, u);
+  int k0 = 0;
+  for (; k0 + D < nks; k0 += D) {
 #pragma unroll
-      for (int w = 1; w < kFewWaves; ++w) v += part[buf][w][s][m][n];
-      return v;
-    };
-    if constexpr (SWIGLU) {
-      const int m = tid >> 4, n = cur.nt * 16 + (tid & 15);
-      if (tid < 256 && m < cur.rows && n < p.N) {
-        const bf16_t g = f32_to_bf16(sum(0, m, tid & 15)), u = f32_to_bf16(sum(1, m, tid & 15));
-        const int64_t r = cur.r0 + m;
-        p.C[r * p.N + n] = f32_to_bf16(bf16_to_f32(f32_to_bf16(silu_f(bf16_to_f32(g)))) * bf16_to_f32(u));
-        if (p.pre) {
-          p.pre[r * 2 * p.N + n] = g;
-          p.pre[r * 2 * p.N + p.N + n] = u;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < (NT + 1) / 2; ++e) {
-        const int id = e * kFewWaves * kWave + tid;  // (m, column of the tile)
-        const int m = id / (16 * NT), col = id % (16 * NT), n = cur.nt * 16 * NT + col;
-        if (m < cur.rows && n < p.N)
-          p.C[static_cast<int64_t>(cur.r0 + m) * p.N + n] = f32_to_bf16(sum(col / 16, m, col % 16));
-      }
+    for (int u = 0; u < D; ++u) {
+      multiply(u);
+      load(u, k0 + D + u);
     }
-    buf ^= 1;
-    cur = nxt;
-    rs_cur = rs_nxt;
-#pragma unroll
-    for (int s = 0; s < NT; ++s) off_cur[s] = off_nxt[s];
   }
-}
+#pragma unroll
+  for (int u = 0; u < D; ++u) multiply(u);  // (past K: zeros)
 
-template <int KS, int NT, bool SWIGLU>
-int few_launch(const FewRows& p, hipStream_t stream, const char* name) {
-  const int n_tiles = (p.N + (SWIGLU ? 16 : 16 * NT) - 1) / (SWIGLU ? 16 : 16 * NT);
-  const int dev = current_device();
-  const int occ = cached_blocks_per_cu(dev, reinterpret_cast<const void*>(&few_rows_kernel<KS, NT, SWIGLU>),
-                                       kFewWaves * kWave, 0);
-  const int64_t most = static_cast<int64_t>((p.rows + 15) / 16 + std::min(p.G, p.rows)) * n_tiles;  // tiles at worst
-  const int64_t resident = static_cast<int64_t>(device_cus(dev)) * occ;
-  const int grid = static_cast<int>((std::min(most, resident) + kFewXcd - 1) / kFewXcd * kFewXcd);
-  hipLaunchKernelGGL((few_rows_kernel<KS, NT, SWIGLU>), dim3(grid), dim3(kFewWaves * kWave), 0, stream, p, n_tiles,
-                     static_cast<uint32_t>(static_cast<int64_t>(p.rows) * p.K * 2),
-                     static_cast<uint32_t>(static_cast<int64_t>(SWIGLU ? 2 : 1) * p.N * p.K * 2));
-  return launch_status(name);
+  // The operands are swapped, so the lane holds columns 4 q .. 4 q + 3 of row i16.
+  const int n = tile * 16 + 4 * q;
+  if (i16 >= rows || n >= p.N) return;
+  const int64_t r = r0 + i16;
+  bf16_t* c = p.C + r * p.N + n;
+  if constexpr (SWIGLU) {
+    float a[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      a[e] = bf16_to_f32(f32_to_bf16(silu_f(bf16_to_f32(f32_to_bf16(acc[0][e]))))) *
+             bf16_to_f32(f32_to_bf16(acc[1][e]));
+    *reinterpret_cast<uint2*>(c) = make_uint2(pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]));
+    if (p.pre) {
+      bf16_t* pre = p.pre + r * 2 * p.N + n;
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        *reinterpret_cast<uint2*>(pre + s * p.N) =
+            make_uint2(pack_bf16x2(acc[s][0], acc[s][1]), pack_bf16x2(acc[s][2], acc[s][3]));
+    }
+  } else {
+    *reinterpret_cast<uint2*>(c) = make_uint2(pack_bf16x2(acc[0][0], acc[0][1]), pack_bf16x2(acc[0][2], acc[0][3]));
+  }
 }
 
 }  // namespace
 
-// k-steps per wave of 2, 3, 4, 6, 8 and 16: K up to 4096, within a quarter of
-// the split (other reductions keep the tiled kernel).
-bool few_rows_takes(int64_t K) { return K > 256 && K <= 4096; }
-
 int few_rows(const FewRows& p, bool swiglu, hipStream_t stream, const char* name) {
-  const int ks = (p.K + 255) / 256;
-#define FEW(KS_, NT_)                                                   \
-  return swiglu ? few_launch<KS_, 2, true>(p, stream, name) : few_launch<KS_, NT_, false>(p, stream, name)
-  if (ks <= 2) FEW(2, 4);
-  if (ks <= 3) FEW(3, 4);
-  if (ks <= 4) FEW(4, 4);
-  if (ks <= 6) FEW(6, 2);
-  if (ks <= 8) FEW(8, 2);
-  FEW(16, 1);
-#undef FEW
+  const int n_tiles = (p.N + 15) / 16;
+  // At most one 16-row chunk per nonempty group and one more per 16 further rows.
+  const int64_t groups = p.G < p.rows ? p.G : p.rows;
+  const int64_t most = (groups + (p.rows - groups) / 16) * n_tiles;
+  MOE_REQUIRE(most < (1ll << 30), MOE_ERR_UNSUPPORTED, "%s: too many tiles", name);
+  const dim3 grid(static_cast<unsigned>((most + kFewXcd - 1) / kFewXcd * kFewXcd));
+  const uint32_t a_bytes = static_cast<uint32_t>(static_cast<int64_t>(p.rows) * p.K * 2);
+  const uint32_t w_bytes = static_cast<uint32_t>(static_cast<int64_t>(swiglu ? 2 : 1) * p.N * p.K * 2);
+  if (swiglu) {
+    hipLaunchKernelGGL((few_rows_kernel<12, true>), grid, dim3(kWave), 0, stream, p, n_tiles, a_bytes, w_bytes);
+  } else {
+    hipLaunchKernelGGL((few_rows_kernel<16, false>), grid, dim3(kWave), 0, stream, p, n_tiles, a_bytes, w_bytes);
+  }
+  return launch_status(name);
 }
 
 }  // namespace moe

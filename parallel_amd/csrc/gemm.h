@@ -29,8 +29,6 @@ struct FewRows {
   const int32_t* offs;
   int G, rows, N, K;
 };
-// Whether few_rows covers a reduction of K.
-bool few_rows_takes(int64_t K);
 int few_rows(const FewRows& p, bool swiglu, hipStream_t stream, const char* name);
 
 // partials[s][T][E] (f32) = x[T, s-th K range] . wr[E, s-th K range]^T.

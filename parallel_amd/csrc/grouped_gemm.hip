@@ -1318,18 +1318,14 @@ constexpr int64_t kLongRowMaxMeanRows = 64;
 // on the 256-row tile against 592 to 594, up_dgrad 501 on the 320-row tile
 // against 548 to 554.
 //
-// The forward GEMMs of a few decoded tokens go to few_rows (up / down, against
-// the 64-row tile; H 2048, I 768: 1 token 14/11 against 22/12, 4 tokens 34/18
-// against 35/18, 16 tokens 105/52 against 122/50, 48 tokens, 3 mean rows,
-// 147/72 against 141/71; H 4096, I 1536: 1 token 35/19 against 78/20, 16 tokens
-// 341/175 against 371/185).  It adds the products in another order, eight
-// partial sums over K.
+// The forward GEMMs of a few decoded tokens go to few_rows, which times both
+// sides.
 template <bool B_KCONTIG, int EPI>
 int launch_expert(GemmParams& p, hipStream_t stream, const char* name) {
   const int out_cols = (EPI == EPI_SWIGLU_FWD) ? 2 * p.swiglu_I : p.N;
   const int64_t rows = p.rows, G = p.G;
   if constexpr (B_KCONTIG) {
-    if (p.offs && rows <= kFewMaxMeanRows * G && few_rows_takes(p.K)) {  // (a single group without offsets: the tiles)
+    if (p.offs && rows <= kFewMaxMeanRows * G) {  // (a single group without offsets: the tiles)
       constexpr bool swiglu = EPI == EPI_SWIGLU_FWD;
       return few_rows(FewRows{p.A, p.B, static_cast<bf16_t*>(p.C), static_cast<bf16_t*>(p.C2), p.offs, p.G, p.rows,
                               swiglu ? p.swiglu_I : p.N, p.K},

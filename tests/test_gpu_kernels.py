@@ -452,8 +452,8 @@ def test_grouped_gemm_wgrad_skewed_routing(name, accumulate, f32):
 
 
 # At most 2 mean rows per expert (a decoding batch): one row, several 16-row chunks of one expert, more
-# groups than a wave has lanes, N off the multiples of 16 and 64, K inside a wave's last k-step, a K that
-# leaves waves idle, the largest K, and one past it (the tiled kernel).
+# groups than a wave has lanes, N off the multiples of 16 and 64, reductions of less, of just more and of
+# many times the k-steps in flight, with tails.
 FEW_ROWS_CASES = [
     ("one", [0] * 5 + [1] + [0] * 2, 64, 2048),
     ("chunks", [0] * 30 + [33, 16, 1] + [0] * 10, 72, 512),
@@ -463,6 +463,8 @@ FEW_ROWS_CASES = [
     ("k_tail", [1, 3, 0, 0], 40, 1000),
     ("k4096", [1, 0, 2, 0], 56, 4096),
     ("past_k", [1, 0, 2, 0], 56, 4104),
+    ("k_short", [1, 0, 2, 0, 3], 40, 8),
+    ("k520", [1, 0, 2, 0, 3], 24, 520),
 ]
 
 
@@ -497,6 +499,29 @@ def test_few_rows_forward_is_exact_on_integers(name, cnt, N, K):
     assert torch.equal(act, act2)
     for t in (c, act, pre):
         assert (t[n:].float() == 7.0).all(), "rows past offs[-1] were written"
+
+
+@pytest.mark.parametrize("name,cnt,N,K", FEW_ROWS_CASES, ids=[c[0] for c in FEW_ROWS_CASES])
+def test_few_rows_forward_gives_the_tiles_bits(name, cnt, N, K):
+    """A token's outputs do not depend on the batch: the same rows in a call whose row count puts it on the
+    tiled kernel (the rows past the groups are not touched) give the same bits, on sums that do round."""
+    counts, offs = _groups(cnt)
+    n, G = int(counts.sum()), len(cnt)
+    many = n + 8 * G  # 8 or more mean rows per expert
+    a = torch.randn(many, K, generator=gen(51)).to(BF).to(DEV)
+    w = torch.randn(G, 2 * N, K, generator=gen(52)).to(BF).to(DEV)
+    w_half, od = w[:, :N].contiguous(), offs.to(DEV)
+    outs = []
+    for M in (n, many):
+        c, act = (torch.zeros(M, N, dtype=BF, device=DEV) for _ in range(2))
+        pre = torch.zeros(M, 2 * N, dtype=BF, device=DEV)
+        s = _lib.stream_of(c)
+        _lib.call("moe_grouped_gemm_fwd", a.data_ptr(), w_half.data_ptr(), od.data_ptr(), G, M, N, K, c.data_ptr(), s)
+        _lib.call("moe_grouped_gemm_swiglu_fwd", a.data_ptr(), w.data_ptr(), od.data_ptr(), G, M, K, N, act.data_ptr(),
+                  pre.data_ptr(), s)
+        outs.append([t[:n].float().cpu() for t in (c, act, pre)])
+    for few, tiled in zip(*outs):
+        assert few.any() and torch.equal(few, tiled), name
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 64, 512), (2, 72, 2048), (3, 64, 512), (2, 40, 264), (1, 64, 4096)])
