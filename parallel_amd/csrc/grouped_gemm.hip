@@ -40,6 +40,7 @@
 // over the 8 XCDs) gets a contiguous run of logical tiles and the sharing
 // happens in that XCD's L2.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "dma.h"
@@ -185,7 +186,7 @@ struct TileCfg {
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, STAGES = STAGES_, PIPE = PIPE_;
   static constexpr int kThreads = 64 * WM * WN;
 };
-// Expert GEMMs and weight gradients: 160 KiB ring, 8 waves.
+// Weight gradients, and input gradients of one round of tiles: 160 KiB ring, 8 waves.
 using BigTile = TileCfg<256, 256, 32, 2, 4, 5>;
 // Expert GEMMs of few rows, bound by the weights' stream from HBM: 64-deep
 // k-tiles (a K-contiguous weight row's 128 bytes, a whole cache line, per
@@ -1318,6 +1319,30 @@ constexpr int64_t kLongRowMaxMeanRows = 64;
 // on the 256-row tile against 592 to 594, up_dgrad 501 on the 320-row tile
 // against 548 to 554.
 //
+// Calls of few tiles (small layers, a rank's share of the experts): a tile that
+// leaves CUs idle costs its whole time, so the smallest that runs all of them
+// at once is taken whatever the mean.  The input gradients' 256-row tiles, when
+// one round of them is all, leave the ping-pong loop, which pays for its longer
+// start from the second tile on.  us, the mean-row rule's choice -> now:
+//   H 512, I 256, 8 experts, mean 400: the four GEMMs 21/14/23/20 (256-row)
+//     -> 11/8/13/10 (64-row)
+//   H 1024, I 512, 32 experts, mean 400: down_dgrad 44 (256-row) -> 33 (128-row),
+//     up_dgrad 34 -> 32 (256-row, paired barriers)
+//   H 1536, I 640, 16 experts, mean 288: up_fwd 56 (320-row) -> 28 (128-row)
+//   H 2048, I 768, 32 experts, mean 352: down_dgrad 76 (128-row) -> 63 (256-row)
+//   H 4096, I 1536, 16 experts, mean 320: down_dgrad 123 (128-row) -> 103 (256-row)
+// Skewed routing: with few rows per expert on average a heavy expert takes
+// several of the small tiles.  Zipf(1) counts still prefer them (H 2048, I 768,
+// 128 experts, 32 mean rows: 64-row 169/84/88/148, 320-row 207/115/122/178; 96
+// mean rows: 128-row 209/101/131/173, 320-row 266/132/157/214).  Where a
+// sixteenth of the experts takes every row the larger tiles are up to 1.4
+// times faster (H 4096, I 1536, 32 mean rows: down_fwd 83 on 64-row, 56 on
+// 320-row tiles; 96 mean rows at H 2048: 90/51/76/91 on 128-row, 79/60/85/105).
+// Large outputs at few rows are a few percent faster on the 320-row tile in the
+// input gradients (H 2048, I 1408, 64 experts, 16 mean rows: up_dgrad 124 on
+// 64-row, 118 on 320-row tiles), which under Zipf counts costs a third (32 mean
+// rows: 192 against 142).
+//
 // The forward GEMMs of a few decoded tokens go to few_rows, which times both
 // sides.
 template <bool B_KCONTIG, int EPI>
@@ -1333,14 +1358,26 @@ int launch_expert(GemmParams& p, hipStream_t stream, const char* name) {
     }
   }
   const bool long_rows = p.ldb >= kLongRow && rows <= kLongRowMaxMeanRows * G;
-  if (!long_rows && rows <= kSlimMaxMeanRows * G) return launch<MODE_MG, B_KCONTIG, EPI, SlimTile>(p, stream, name);
-  if ((!long_rows && rows <= (out_cols <= 1024 ? kWideMaxMeanRows : kMidMaxMeanRows) * G) ||
-      (rows > kWideMaxMeanRows * G && rows <= kMidAgainMaxMeanRows * G))
+  // Whether tiles of bm rows, at `per` rows per expert, all run at once.
+  const int64_t n_tiles = (out_cols + 255) / 256, cus = device_cus(current_device());
+  auto one_round = [&](int bm, double per) {
+    return G * n_tiles * std::max<int64_t>(1, static_cast<int64_t>(std::ceil(per / bm))) <= cus;
+  };
+  const double mean = static_cast<double>(rows) / static_cast<double>(G);
+  const double high = mean + 3.0 * std::sqrt(mean);  // few experts have more, under uniform routing
+  if (!long_rows && (rows <= kSlimMaxMeanRows * G || one_round(SlimTile::BM, high)))
+    return launch<MODE_MG, B_KCONTIG, EPI, SlimTile>(p, stream, name);
+  if ((!long_rows && (rows <= (out_cols <= 1024 ? kWideMaxMeanRows : kMidMaxMeanRows) * G || one_round(MidTile::BM, high))) ||
+      (rows > kWideMaxMeanRows * G && rows <= kMidAgainMaxMeanRows * G &&
+       (one_round(MidTile::BM, mean) || !one_round(PingTile::BM, mean))))
     return launch<MODE_MG, B_KCONTIG, EPI, MidTile>(p, stream, name);
   // Up to 320 rows per expert in one m-tile, and the input gradients of long
   // weight rows.
   if (rows <= kWideMaxMeanRows * G && (rows > kBigMaxMeanRows * G || (long_rows && !B_KCONTIG)))
     return launch<MODE_MG, B_KCONTIG, EPI, WideTile>(p, stream, name);
+  if constexpr (!B_KCONTIG) {
+    if (one_round(BigTile::BM, mean)) return launch<MODE_MG, B_KCONTIG, EPI, BigTile>(p, stream, name);
+  }
   return launch<MODE_MG, B_KCONTIG, EPI, PingTile>(p, stream, name);
 }
 
@@ -1627,7 +1664,7 @@ int wgrad(const void* dc, const void* a, const int32_t* offs, int64_t G, int64_t
   p.bucket_rows = static_cast<int>(bucket_rows);
   p.bucket_stride = bucket_stride;
   if ((rc = set_bytes(p, M * N * 2, M * K * 2, N * K * (dw_is_f32 ? 4 : 2), name))) return rc;
-    return launch<MODE_KG, false, EPI_WGRAD, BigTile>(p, as_stream(stream), name);
+  return launch<MODE_KG, false, EPI_WGRAD, BigTile>(p, as_stream(stream), name);
 }
 }  // namespace
 

@@ -561,6 +561,20 @@ ROW_TILE_CASES = [
     ("mid_again", [320, 290, 330, 300], 1288, 136),
     ("long_rows_few", [64, 20, 0, 65], 1032, 4104),
     ("long_rows_mid", [130, 90, 0, 128], 1032, 4104),
+    # Outputs of many column tiles, whose tile the mean alone decides, in one direction and in the other (a
+    # call of few tiles takes the smallest that runs them at once, as most of the above do)
+    *[(f"{name}_{side}", cnt, *((8200, k) if side == "fwd" else (k, 8200)))
+      for name, cnt, k in (("mid", [128, 129, 1, 64, 0, 127, 200, 130], 200), ("big", [256, 257, 100, 224], 136),
+                           ("wide", [320, 321, 200, 230], 136), ("mid_again", [320, 290, 330, 300], 136),
+                           ("ping_one_kstep", [513, 0, 600, 511], 40), ("ping_odd", [256, 257, 1100, 0, 300], 168),
+                           ("ping_even", [400, 0, 512, 700], 232))
+      for side in ("fwd", "dgrad")],
+    # the few-tile rule's bounds: 64-row tiles of up to six per expert, 128-row ones, 256-row ones in one
+    # round (input gradients on the paired-barrier loop) and in two
+    ("slim_round", [300, 0, 257, 400, 290], 2056, 264),
+    ("mid_round", [300, 257, 310, 290, 0, 420, 305, 320], 1304, 1304),
+    ("big_round", [520, 513, 600, 0, 900, 511, 512, 600], 1800, 1800),
+    ("two_rounds", [520, 513, 0, 600, 511, 512, 900, 600, 500, 490, 530, 384, 700], 1832, 1832),
 ]
 
 
@@ -591,7 +605,8 @@ def test_row_tiles_give_the_exact_products(name, cnt, N, K):
 
 
 @pytest.mark.parametrize("cnt,I,H", [([256, 0, 300, 1, 128], 768, 2048), ([5, 64, 0, 17], 64, 96),
-                                     ([600, 0, 1500, 5, 257], 768, 2048)])  # the last on the ping-pong loop
+                                     ([600, 0, 1500, 5, 257], 768, 2048), ([600, 0, 1500, 5, 257], 1408, 1800)])
+# (the last forward on the ping-pong loop)
 def test_swiglu_fwd_and_fused_backward(cnt, I, H):
     counts, offs = _groups(cnt)
     M = int(counts.sum())
