@@ -71,7 +71,7 @@ struct F32Tile {
 // A(l % 32, r + l / 32) and B(r + l / 32, l % 32), and holds D rows
 // 8 (q / 4) + 4 (l / 32) + q % 4 (q = 0..15) of column l % 32.
 template <int LA, int LB, class T>
-__global__ __launch_bounds__(T::kThreads) void f32_grouped_gemm_kernel(const F32Gemm p, int tiles_j) {
+__global__ __launch_bounds__(T::kThreads) void f32_grouped_gemm_kernel(const F32Gemm p, int tiles_j, int part) {
   constexpr int BM = T::BM, BN = T::BN, BK = T::BK, SM = T::SM, SN = T::SN;
   constexpr int NVA = BM * BK / 4 / T::kThreads, NVB = BN * BK / 4 / T::kThreads;
   static_assert(NVA >= 1 && NVB >= 1 && NVA * T::kThreads * 4 == BM * BK && NVB * T::kThreads * 4 == BN * BK,
@@ -84,7 +84,8 @@ __global__ __launch_bounds__(T::kThreads) void f32_grouped_gemm_kernel(const F32
   const int l32 = lane & 31, half = lane >> 5;
 
   // The tile: block b is the (b / 8)-th of XCD b % 8's contiguous share of
-  // the real tiles (group-major, then m-tile, then n-tile).
+  // the real tiles (group-major, then m-tile, then n-tile), or with `part` of
+  // part tiles of every group.
   const int xcd = blockIdx.x % kNumXcd;
   const int64_t idx = blockIdx.x / kNumXcd;
   int mtiles = 0;  // m-tiles over all groups
@@ -98,8 +99,15 @@ __global__ __launch_bounds__(T::kThreads) void f32_grouped_gemm_kernel(const F32
     mtiles = p.G * ((p.M + BM - 1) / BM);
   }
   const int64_t real = static_cast<int64_t>(mtiles) * tiles_j, share = (real + kNumXcd - 1) / kNumXcd;
-  const int64_t tile = xcd * share + idx;
-  if (idx >= share || tile >= real) return;
+  int64_t tile = xcd * share + idx;
+  if (part > 0) {
+    const int per_group = static_cast<int>(real / p.G), gi = static_cast<int>(idx) / part;
+    const int local = xcd * part + static_cast<int>(idx) - gi * part;
+    if (gi >= p.G || local >= per_group) return;
+    tile = static_cast<int64_t>(gi) * per_group + local;
+  } else if (idx >= share || tile >= real) {
+    return;
+  }
   const int tj = static_cast<int>(tile % tiles_j);
   const int mt = static_cast<int>(tile / tiles_j);
   int g = 0, i0 = 0, i_end = p.M, r_begin = 0, r_end = p.K;
@@ -302,10 +310,23 @@ int f32_launch_tile(const F32Gemm& p, hipStream_t stream) {
   // mode 0: every group's rows in BM-row tiles, at most M / BM + G of them
   const int64_t tiles_i = p.mode == 0 ? (p.M + T::BM - 1) / T::BM + p.G
                                       : static_cast<int64_t>(p.G) * ((p.M + T::BM - 1) / T::BM);
-  const int64_t blocks = (tiles_i * tiles_j + kNumXcd - 1) / kNumXcd * kNumXcd;
+  // A weight gradient's tile costs its group's rows.  Where the tiles take
+  // several rounds, every XCD takes an eighth of each group's, so that skewed
+  // rows load all of them alike; in one round contiguous shares, which read a
+  // group's operands into one L2.  us, contiguous -> eighths, up / down
+  // projection: H 1536, I 640, 64 experts, 4096 rows, Zipf(1) 352/209 -> 231/139,
+  // uniform 210/102 -> 206/106; H 2048, I 768, 128 experts, 8192 rows, Zipf(1)
+  // 982/513 -> 670/362, uniform 641/334 -> 639/327; H 1024, I 512, 32 experts,
+  // 2048 rows, two experts with all of them 221/93 -> 152/85, Zipf(1) 99/56 ->
+  // 94/66.  H 256, I 128, 8 experts, 512 rows (one round) stays: 7.0/6.9, 7.6/7.8
+  // in eighths.
+  const int64_t per_group = static_cast<int64_t>((p.M + T::BM - 1) / T::BM) * tiles_j;
+  const int64_t part =
+      p.mode == 1 && p.G * per_group > device_cus(current_device()) ? (per_group + kNumXcd - 1) / kNumXcd : 0;
+  const int64_t blocks = part ? p.G * part * kNumXcd : (tiles_i * tiles_j + kNumXcd - 1) / kNumXcd * kNumXcd;
   MOE_REQUIRE(blocks < (1ll << 31) && tiles_i < (1ll << 31), MOE_ERR_UNSUPPORTED, "f32 grouped gemm: too many tiles");
   hipLaunchKernelGGL((f32_grouped_gemm_kernel<LA, LB, T>), dim3(static_cast<unsigned>(blocks)), dim3(T::kThreads), 0,
-                     stream, p, tiles_j);
+                     stream, p, tiles_j, static_cast<int>(part));
   return launch_status("moe_f32_grouped_gemm");
 }
 

@@ -205,6 +205,8 @@ F32_GEMMS = [
     (1, [63, 0, 17, 65, 1, 33], 132, 68, 0, "col", "row"),
     (1, [63, 0, 17, 65, 1, 33], 131, 67, 0, "row", "wide"),
     (1, [40, 0, 3, 70], 1024, 1028, 0, "col", "row"),
+    (1, [3, 0, 700, 1, 0, 2, 5, 4], 1024, 1028, 0, "col", "row"),  # skewed; 72 tiles of each group over the XCDs
+    (1, [2, 30, 0, 9] * 80, 260, 132, 0, "col", "row"),  # 320 groups of fewer tiles than XCDs
     (1, [1501], 36, 100, 0, "col", "row"),
     (1, [1501], 33, 99, 0, "row", "col"),
 ]
