@@ -106,48 +106,62 @@ class TokenDispatcher:
         if global_indices.shape != scores.shape:
             raise ValueError("Expert indices and scores must have the same shape")
         tokens, top_k = global_indices.shape
-        if (self.world_size > 1 and ops.takes_block(hidden_states, global_indices, scores)
+        splits = None
+        if (self._exchanges_own_block() and ops.takes_block(hidden_states, global_indices, scores)
                 and hidden_states.shape[0] == tokens):
-            return self._dispatch_block(hidden_states, global_indices, scores)
+            sort = ops.dispatch_sort(global_indices, scores, self.partition.local_count, self.world_size)
+            splits = self._exchange_splits(sort[-1])
+            if self._is_own_block(*splits, tokens * top_k):
+                return self._dispatch_block(hidden_states, scores, top_k, sort, *splits)
         send_hidden, send_experts, send_scores, source_tokens, pos_of_slot, counts = ops.run_dispatch_fwd(
             hidden_states, global_indices, scores, self.partition.local_count, self.partition.ep_size
         )
-        send_splits, receive_splits = self._exchange_splits(counts)
+        send_splits, receive_splits = splits or self._exchange_splits(counts)
         received_hidden = self._exchange(send_hidden, send_splits, receive_splits, "dispatch_hidden")
         received_experts = self._exchange(send_experts, send_splits, receive_splits, "dispatch_experts")
         received_scores = self._exchange(send_scores, send_splits, receive_splits, "dispatch_scores")
         state = DispatchState(send_splits, receive_splits, source_tokens, tokens, pos_of_slot, top_k)
         return received_hidden, received_experts.unsqueeze(-1), received_scores.unsqueeze(-1), state
 
-    def _dispatch_block(self, hidden_states, global_indices, scores):
+    def _exchanges_own_block(self):
+        """Whether this dispatcher's exchange keeps the rank's own block and drops the others: the one
+        defined here, not a subclass's, over a group that is still one process."""
+        if self.world_size == 1 or getattr(self._exchange, "__func__", None) is not _EXCHANGE:
+            return False
+        require_single_rank(self.group, "TokenDispatcher")
+        return True
+
+    def _is_own_block(self, send, receive, rows):
+        """Whether the splits send every one of ``rows`` rows and receive this rank's own block alone."""
+        return (len(send) == len(receive) == self.world_size and sum(send) == rows
+                and send[self.rank] == receive[self.rank] == sum(receive))
+
+    def _dispatch_block(self, hidden_states, scores, top_k, sort, send, receive):
         """dispatch with only this rank's block of the send rows written: the others would be dropped by
         the exchange, and they are most of the bytes."""
-        tokens, top_k = global_indices.shape
-        send_experts, sorted_scores, source_tokens, pos_of_slot, counts = ops.dispatch_sort(
-            global_indices, scores, self.partition.local_count, self.world_size
-        )
-        send, receive = self._exchange_splits(counts)
-        if sum(send) != tokens * top_k:  # routes to experts of no rank
-            raise ValueError(f"send splits {send} do not cover the {tokens * top_k} rows to send")
+        send_experts, sorted_scores, source_tokens, pos_of_slot, _ = sort
         lo, rows = _block_start(send, self.rank), send[self.rank]
         received_hidden = ops.scatter_block(hidden_states, pos_of_slot, top_k, lo, rows)
         received_scores = ops.block_scores(scores, sorted_scores, pos_of_slot, lo, rows)
-        state = DispatchState(send, receive, source_tokens, tokens, pos_of_slot, top_k)
+        state = DispatchState(send, receive, source_tokens, hidden_states.shape[0], pos_of_slot, top_k)
         return (received_hidden, send_experts.narrow(0, lo, rows).unsqueeze(-1), received_scores.unsqueeze(-1), state)
 
-    def _own_block(self, expert_output, state):
+    def _returns_own_block(self, expert_output, state):
         """Whether expert_output is this rank's block of a well-formed state and nothing else."""
-        send, receive, rank = state.send_splits, state.receive_splits, self.rank
-        return (self.world_size > 1 and state.pos_of_slot is not None and len(send) == len(receive) == self.world_size
-                and send[rank] == receive[rank] == sum(receive) == expert_output.shape[0]
-                and sum(send) == state.pos_of_slot.numel() == state.num_source_tokens * state.top_k
+        return (self._exchanges_own_block() and state.pos_of_slot is not None
+                and state.pos_of_slot.numel() == state.num_source_tokens * state.top_k
+                and self._is_own_block(state.send_splits, state.receive_splits, state.pos_of_slot.numel())
+                and state.receive_splits[self.rank] == expert_output.shape[0]
                 and ops.takes_block(expert_output, state.pos_of_slot))
 
     def combine(self, expert_output: torch.Tensor, state: DispatchState):
-        if self._own_block(expert_output, state):
+        if self._returns_own_block(expert_output, state):
             return ops.gather_block(expert_output, state.pos_of_slot, state.num_source_tokens, state.top_k,
                                     _block_start(state.send_splits, self.rank))
         returned = self._exchange(expert_output, state.receive_splits, state.send_splits, "combine_hidden")
         if state.pos_of_slot is None:
             raise ValueError("DispatchState has no inverse permutation; it was not produced by this dispatcher")
         return ops.run_combine_rows_fwd(returned, state.pos_of_slot, state.num_source_tokens, state.top_k)
+
+
+_EXCHANGE = TokenDispatcher._exchange

@@ -109,6 +109,59 @@ def test_direct_calls_keep_hooks_and_in_place_outputs():
     assert all(v.grad is not None for v in (x, rw, gu, dn))
 
 
+class _Recorded(TokenDispatcher):
+    """A subclass with an exchange of its own."""
+
+    def __init__(self, partition, group, extra=0):
+        super().__init__(partition, group)
+        self.modes, self.extra = [], extra
+
+    def _exchange(self, value, send_splits, receive_splits, mode):
+        self.modes.append(mode)
+        return super()._exchange(value, send_splits, receive_splits, mode)
+
+    def _exchange_splits(self, send_counts):
+        send, receive = super()._exchange_splits(send_counts)
+        return send, tuple(r + (self.extra if i == self.rank else 0) for i, r in enumerate(receive))
+
+
+class _Splits(TokenDispatcher):
+    def _exchange_splits(self, send_counts):
+        send, receive = super()._exchange_splits(send_counts)
+        return send, tuple(r + 1 for r in receive)
+
+
+def test_own_block_route_is_for_the_dispatchers_own_exchange(monkeypatch):
+    part = ExpertPartition(8, 2, 1)
+    plain, patched = TokenDispatcher(part, None), TokenDispatcher(part, None)
+    assert plain._exchanges_own_block() and not _Recorded(part, None)._exchanges_own_block()
+    assert not TokenDispatcher(ExpertPartition(8, 1, 0), None)._exchanges_own_block()
+    patched._exchange = lambda value, send, receive, mode: value
+    assert not patched._exchanges_own_block()
+    assert plain._is_own_block((3, 5), (0, 5), 8)
+    for send, receive, rows in (((3, 5), (0, 5), 9), ((3, 5), (0, 4), 8), ((3, 5), (1, 5), 8), ((3, 5), (5,), 8)):
+        assert not plain._is_own_block(send, receive, rows)
+    monkeypatch.setattr("parallel_amd.groups.group_size", lambda group: 2)  # a group that grew after construction
+    with pytest.raises(NotImplementedError):
+        plain._exchanges_own_block()
+
+
+@pytest.mark.gpu
+def test_a_subclass_exchange_is_used():
+    ids = torch.tensor([[0, 5], [6, 1], [7, 4]], device="cuda")
+    hidden, scores = torch.randn(3, 64, device="cuda").to(BF), torch.rand(3, 2, device="cuda")
+    part = ExpertPartition(8, 2, 1)
+    recorded, plain = _Recorded(part, None), TokenDispatcher(part, None)
+    got = recorded.dispatch(hidden, ids, scores)
+    want = plain.dispatch(hidden, ids, scores)
+    assert all(torch.equal(a, b) for a, b in zip(got[:3], want[:3]))
+    assert torch.equal(recorded.combine(got[0], got[3]), plain.combine(want[0], want[3]))
+    assert recorded.modes == ["dispatch_hidden", "dispatch_experts", "dispatch_scores", "combine_hidden"]
+    for dispatcher in (_Recorded(part, None, extra=1), _Splits(part, None)):  # receive splits that don't match
+        with pytest.raises(ValueError, match="expects"):
+            dispatcher.dispatch(hidden, ids, scores)
+
+
 def _dispatch_pass(T, E, k, H, ep, rank, layout):
     """Dispatch, an elementwise stand-in for the experts and combine, forward and backward."""
     g = torch.Generator().manual_seed(T + k)
