@@ -67,6 +67,11 @@ def _plain_eager(args) -> bool:
     GPU tensors: no tensor subclass, proxy, symbolic size or meta tensor among
     them, no compilation or tracing, no torch function or dispatch mode, no
     functorch transform, no forward-mode differentiation."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+            or torch._C._len_torch_function_stack() or torch._C._get_tracing_state() is not None
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0):
+        return False  # (before the tensors are looked at: a function mode sees that)
     for a in args:
         t = type(a)
         if t is Tensor or t is torch.nn.Parameter:
@@ -74,10 +79,7 @@ def _plain_eager(args) -> bool:
                 return False
         elif t not in _SCALARS:
             return False
-    return not (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
-                or torch._C._len_torch_function_stack() or torch._C._get_tracing_state() is not None
-                or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch.autograd.forward_ad._current_level >= 0)
+    return True
 
 
 def _wants_grad(args) -> bool:

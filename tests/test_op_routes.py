@@ -1,6 +1,6 @@
 """The route of the differentiable ops: ordinary eager GPU calls run their kernels directly, everything
-that observes or transforms an op (fake and meta tensors, symbolic tracing, tensor subclasses, dispatch
-modes, functorch) still gets the registered op."""
+that observes or transforms an op (fake and meta tensors, tracing, tensor subclasses, function and dispatch
+modes, functorch, forward mode) still gets the registered op; and the route of the one-process exchange."""
 
 import pytest
 import torch
@@ -107,6 +107,92 @@ def test_direct_calls_keep_hooks_and_in_place_outputs():
     h += 1  # a fresh tensor, not a view: in-place use stays legal
     (out.float().sum() + h.float().sum()).backward()
     assert all(v.grad is not None for v in (x, rw, gu, dn))
+
+
+class _Traced(torch.Tensor):
+    """A tensor subclass that sees the functions called on it."""
+
+    seen = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.seen.append(str(func))
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+def _outcome(fn):
+    """What a call does: its results, or the type of the exception that refuses it."""
+    try:
+        out = fn()
+    except Exception as e:  # noqa: BLE001
+        return type(e)
+    return [o.detach() for o in (out if isinstance(out, tuple) else (out,))]
+
+
+def _same(a, b):
+    return a == b if isinstance(a, type) or isinstance(b, type) else (
+        len(a) == len(b) and all(torch.equal(x, y) for x, y in zip(a, b)))
+
+
+@pytest.mark.gpu
+def test_the_direct_route_is_for_plain_eager_calls():
+    """What decides, inside each of the situations that must not take it (private torch calls tell)."""
+    x = torch.randn(4, 8, device="cuda")
+    plain = ops._plain_eager
+    assert plain((x, 2, True, None, 1.0)) and plain((torch.nn.Parameter(x),))
+    assert not plain((x.as_subclass(_Traced),)) and not plain((x.cpu(),)) and not plain((x, "text"))
+    seen = []
+
+    def ask(t):
+        seen.append(plain((x,)))
+        return t.sum()
+
+    torch.func.vmap(ask)(x)
+    torch.func.grad(ask)(x)
+    torch.func.jvp(ask, (x,), (x,))
+    torch.func.functionalize(ask)(x)
+    with torch.autograd.forward_ad.dual_level():
+        ask(x)
+    with _Seen():
+        ask(x)
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        seen.append(plain((x,)))
+    torch.jit.trace(ask, (x,), check_trace=False)
+    torch.fx.experimental.proxy_tensor.make_fx(ask)(x)
+    with torch.overrides.BaseTorchFunctionMode():
+        ask(x)
+    assert len(seen) == 10 and not any(seen), seen
+    assert plain((x,))  # and none of them leaves anything behind
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", ["subclass", "grad", "vjp", "vmap", "jvp", "forward_ad"])
+def test_transformed_calls_do_what_the_registered_op_does(how):
+    """The route under tensor subclasses, functorch transforms and forward mode: the registered op's
+    results, or its refusal."""
+    (x, rw, _, _), (k, norm) = _block_args(device="cuda")
+    t = torch.ones_like(x)
+
+    def call(op):
+        f = lambda v: op(v, rw, k, norm)[1].float().square().sum()  # noqa: E731
+        if how == "subclass":
+            return op(x.as_subclass(_Traced), rw, k, norm)
+        if how == "grad":
+            return torch.func.grad(f)(x)
+        if how == "vjp":
+            out, back = torch.func.vjp(f, x)
+            return out, *back(torch.ones_like(out))
+        if how == "vmap":
+            return torch.func.vmap(lambda v: op(v, rw, k, norm)[0])(x.unsqueeze(0))
+        if how == "jvp":
+            return torch.func.jvp(f, (x,), (t,))
+        with torch.autograd.forward_ad.dual_level():
+            return op(torch.autograd.forward_ad.make_dual(x, t), rw, k, norm)[0]
+
+    _Traced.seen.clear()
+    route = _outcome(lambda: call(ops.run_router_fwd))
+    assert how != "subclass" or any("parallel_amd.router_fwd" in n for n in _Traced.seen)
+    assert _same(route, _outcome(lambda: call(ops.router_fwd))), route
 
 
 class _Recorded(TokenDispatcher):
