@@ -3,23 +3,72 @@
 The kernel's DMA (buffer_load_dwordx4 ... lds) fills each 1 KiB block lane by
 lane, so a lane fetches whichever global 16-byte chunk belongs at its slot;
 fragment reads then locate each element with a per-lane offset.  This model
-restates both sides' index formulas and checks (1) that the reader finds
-every element where the writer put it and (2) that every read pass touches
-distinct banks of the 64-bank (256 B/clk) gfx950 LDS: 16 lanes per
-ds_read_b128 pass, 32 lanes per ds_read_b64_tr_b16 pass.  A swizzle designed
-for 32 banks fails (2), which is what the SQ_LDS_BANK_CONFLICT counter showed
-on the GPU before the change.
+evaluates the swizzles and both sides' index expressions as the kernel's source
+has them and checks (1) that the reader finds every element where the writer
+put it and (2) that every read pass touches distinct banks of the 64-bank (256
+B/clk) gfx950 LDS: 16 lanes per ds_read_b128 pass, 32 lanes per
+ds_read_b64_tr_b16 pass.  A swizzle designed for 32 banks fails (2), which is
+what the SQ_LDS_BANK_CONFLICT counter showed on the GPU before the change.
 """
+
+import re
+from pathlib import Path
 
 import pytest
 
-
-def kc_swizzle(r):  # K-contiguous: row bits 2-3
-    return (r >> 2) & 3
+SOURCE = (Path(__file__).resolve().parents[1] / "parallel_amd" / "csrc" / "grouped_gemm.hip").read_text()
 
 
-def mc_swizzle(kk):  # M/N-contiguous: k-row & 3 selects the 64-byte bank quarter, bit 3 the half of it
-    return 4 * (kk & 3) | 2 * ((kk >> 3) & 1)
+def _expression(pattern):
+    """The one C expression that ``pattern`` captures in the kernel's source, as a Python function of its
+    variables (integers, so / is //; swizzle templates take BK by name)."""
+    found = {" ".join(f.split()) for f in re.findall(pattern, SOURCE, re.S)}
+    assert len(found) == 1, f"{pattern}: {found}"
+    text = re.sub(r"kc_swizzle<BK>\((\w+)\)", r"kc_swizzle(\1, BK)", found.pop()).replace("/", "//")
+    text = re.sub(r"\((\w+) \? (\w+) : (\w+)\)", r"(\2 if \1 else \3)", text)
+    text = re.sub(r"^(.*?) \? (.*?) : (.*)$", r"(\2) if (\1) else (\3)", text)
+    code = compile(text.strip(), pattern, "eval")
+    return lambda **names: eval(code, {"kc_swizzle": kc_swizzle, "mc_swizzle": mc_swizzle,  # noqa: S307
+                                       "stg_swizzle": stg_swizzle, **names})
+
+
+_kc, _mc, _stg = (_expression(rf"constexpr int {name}\(int \w+\) {{\s*return (.*?);")
+                  for name in ("kc_swizzle", "mc_swizzle", "stg_swizzle"))
+
+
+def kc_swizzle(r, BK=32):
+    return _kc(r=r, BK=BK)
+
+
+def mc_swizzle(kk):
+    return _mc(kk=kk)
+
+
+def stg_swizzle(r):
+    return _stg(r=r)
+
+
+# DMA: the K-contiguous row and k that a lane's 16 bytes belong to, the M/N-contiguous k-row and column.
+DMA_KC_ROW = _expression(r"const int r = (li \* RPI \+ [^;]*);")
+DMA_KC_K = _expression(r"dma_k\[j\] = (\(\(lane % CPR\)[^;]*);")
+DMA_MC_KROW = _expression(r"dma_k\[j\] = (li \* \(64 / cpk\)[^;]*);")
+DMA_MC_COL = _expression(r"const int col = \(is_a \? dt\.m0 : dt\.n0\) \+ (\(\(lane % [^;]*);")
+# Fragment reads.
+READ_KC = _expression(r"const int lane_off = ([^;]*);")
+READ_KC_B = _expression(r"b_kc\[ks\] = B_OFF \+ ([^;]*);")
+READ_KC_T = _expression(r"base \+ b_kc\[ks\] \+ ([^)]*)\);")
+TR_KROW = _expression(r"const int tr_krow = ([^;]*);")
+TR_COL = _expression(r"const int tr_col = ([^;]*);")
+HALF8 = _expression(r"const int half8 = ([^;]*);")
+READ_MC = _expression(r"b_mc\[t\] = B_OFF \+ ([^;]*);")
+READ_MC_KS = _expression(r"tr_read\(base \+ b_mc\[t\] \+ ([^,]*),")
+READ_MC_HI = _expression(r"\(lds_i16x4_t\*\)\(at \+ ([^)]*)\)\);")
+# Epilogue staging.
+STG_LANE = _expression(r"const int stg_lane = ([^;]*);")
+STG_WRITE = _expression(r"uint2\*>\(slot \+ stg_lane \+ (hh[^;]*)\) = v;")
+STG_ROW = _expression(r"uint4 v = \*reinterpret_cast<const uint4\*>\(slot \+ ([^;]*)\);")
+STG_GATE = _expression(r"const uint4 gv = \*reinterpret_cast<const uint4\*>\(slot \+ ([^;]*)\);")
+STG_UP = _expression(r"const uint4 uv = \*reinterpret_cast<const uint4\*>\(slot \+ ([^;]*)\);")
 
 
 def bank_conflicts(addrs, lanes_per_pass, width):
@@ -31,67 +80,82 @@ def bank_conflicts(addrs, lanes_per_pass, width):
 
 
 def check_kc(R, swz, bk=32):
-    cpr = bk // 8  # chunks of 16 B per row of a k-tile
-    rb = 2 * bk
+    """A K-contiguous [R rows][bk] tile, with the kernel's swizzle or another."""
+    c = dict(BK=bk, RB=2 * bk, CPR=bk // 8, RPI=64 * 8 // bk, WTN=R, wn=0, kc_swizzle=lambda r, BK: swz(r))
     where = {}
-    for li in range(R * rb // 1024):
+    for li in range(R * c["RB"] // 1024):
         for lane in range(64):
-            r = li * (64 // cpr) + lane // cpr
-            where[(r, (lane % cpr) ^ swz(r))] = li * 1024 + lane * 16
+            r = DMA_KC_ROW(li=li, lane=lane, **c)
+            where[(r, DMA_KC_K(lane=lane, r=r, **c) // 8)] = li * 1024 + lane * 16
     conflicts = 0
-    for row0 in range(0, R, 16):  # a fragment: 16 rows x 32 k
+    for t in range(R // 16):  # a fragment: 16 rows x 32 k
         for ks in range(bk // 32):
             addrs = []
             for lane in range(64):
-                i16, q = lane & 15, lane >> 4
-                off = row0 * rb + i16 * rb + (((4 * ks + q) ^ swz(i16)) << 4)
-                assert where[(row0 + i16, 4 * ks + q)] == off
+                i16, q16 = lane & 15, lane >> 4
+                lane_off = READ_KC(i16=i16, q16=q16, ks=ks, **c)
+                off = READ_KC_B(lane_off=lane_off, **c) + READ_KC_T(t=t, **c)
+                assert where[(16 * t + i16, 4 * ks + q16)] == off
                 addrs.append(off)
             conflicts += bank_conflicts(addrs, 16, 16)
     return conflicts
 
 
 def check_mc(R, WT, swz, bk=32):
-    cpk = R // 8
+    """An M/N-contiguous [bk k-rows][R columns] tile, a wave's columns being WT wide."""
+    c = dict(BM=R, BN=R, WTN=WT, is_a=False, cpk=R // 8, mc_swizzle=swz)
     where = {}
     for li in range(R * bk * 2 // 1024):
         for lane in range(64):
-            kk = li * (64 // cpk) + lane // cpk
-            where[(kk, (lane % cpk) ^ swz(kk))] = li * 1024 + lane * 16
+            kk = DMA_MC_KROW(li=li, lane=lane, **c)
+            col = DMA_MC_COL(lane=lane, dma_k=[kk], j2=0, **c)
+            where[(kk, col // 8)] = li * 1024 + lane * 16
     conflicts = 0
-    for wcb in range(0, R, WT):
+    for wn in range(R // WT):
         for t in range(WT // 16):  # a fragment: 16 columns x 32 k, two transpose reads
             for ks in range(bk // 32):
                 for h in range(2):
                     addrs = []
                     for lane in range(64):
-                        q, i = lane >> 4, lane & 15
-                        krow = 8 * q + (i >> 2)
-                        col = 4 * (i & 3)
-                        off = (krow * R * 2 + ((((wcb + 16 * t + col) >> 3) ^ swz(krow)) << 4)
-                               + ((i & 1) << 3) + 32 * ks * R * 2 + h * 4 * R * 2)
-                        kr, gcol = 32 * ks + krow + 4 * h, wcb + 16 * t + col
+                        i16, q16 = lane & 15, lane >> 4
+                        krow, col = TR_KROW(i16=i16, q16=q16), TR_COL(i16=i16)
+                        off = (READ_MC(tr_krow=krow, tr_col=col, half8=HALF8(i16=i16), wn=wn, t=t, **c)
+                               + READ_MC_KS(ks=ks, **c) + h * READ_MC_HI(row_bytes=R * 2))
+                        kr, gcol = 32 * ks + krow + 4 * h, wn * WT + 16 * t + col
                         assert where[(kr, gcol >> 3)] + (gcol & 7) * 2 == off
                         addrs.append(off)
                     conflicts += bank_conflicts(addrs, 32, 8)
     return conflicts
 
 
-def test_epilogue_staging_is_conflict_free():
-    """A wave's 32 x 64 bf16 pass: 8-byte writes (row 16 hh + i16, chunk 2 tt + q16 / 2, half q16 & 1),
-    then row reads and the SwiGLU gate/up reads of whole chunks."""
-    def at(r, chunk):
-        return r * 128 + ((chunk ^ ((((r >> 1) & 1) << 2) | ((r >> 2) & 3))) << 4)
-
+def test_epilogue_staging_is_consistent_and_conflict_free():
+    """A wave's 32 x 64 bf16 pass: 8-byte writes (row 16 hh + i16, columns 16 tt + 4 q16 ..), then row
+    reads and the SwiGLU gate/up reads of whole 16-byte chunks."""
+    where = {}
     for hh in range(2):
         for tt in range(4):
-            writes = [at(16 * hh + (l & 15), 2 * tt + (l >> 5)) + ((l >> 4 & 1) << 3) for l in range(64)]
-            assert bank_conflicts(writes, 32, 8) == 0
+            addrs = []
+            for lane in range(64):
+                i16, q16 = lane & 15, lane >> 4
+                addrs.append(STG_LANE(i16=i16, q16=q16) + STG_WRITE(hh=hh, tt=tt, q16=q16, stg_swz=stg_swizzle(i16)))
+                where[(16 * hh + i16, 16 * tt + 4 * q16)] = addrs[-1]
+            assert bank_conflicts(addrs, 32, 8) == 0
+    assert len(set(where.values())) == 32 * 16
+
+    def reads(rows, chunk, at):
+        addrs = [at(r) for r in rows]
+        for r, cc, a in zip(rows, chunk, addrs):
+            assert where[(r, 8 * cc)] == a and where[(r, 8 * cc + 4)] == a + 8
+        assert bank_conflicts(addrs, 16, 16) == 0
+
     for n in range(4):
-        assert bank_conflicts([at(8 * n + (l >> 3), l & 7) for l in range(64)], 16, 16) == 0
+        lanes = range(64)
+        rows, c8 = [8 * n + (lane >> 3) for lane in lanes], [lane & 7 for lane in lanes]
+        reads(rows, c8, lambda r, it=iter(c8): STG_ROW(r=r, c8=next(it)))
     for n in range(2):
-        for half in (0, 4):
-            assert bank_conflicts([at(16 * n + (l >> 2), (l & 3) + half) for l in range(64)], 16, 16) == 0
+        rows, c4 = [16 * n + (lane >> 2) for lane in range(64)], [lane & 3 for lane in range(64)]
+        reads(rows, c4, lambda r, it=iter(c4): STG_GATE(r=r, c4=next(it), swz=stg_swizzle(r)))
+        reads(rows, [c + 4 for c in c4], lambda r, it=iter(c4): STG_UP(r=r, c4=next(it), swz=stg_swizzle(r)))
 
 
 @pytest.mark.parametrize("R", [128, 256])
@@ -106,7 +170,7 @@ def test_transpose_read_layout_is_consistent_and_conflict_free(R, WT):
 
 @pytest.mark.parametrize("R", [64, 128, 256])
 def test_64_deep_layouts_are_consistent_and_conflict_free(R):
-    assert check_kc(R, lambda r: (r >> 1) & 7, bk=64) == 0
+    assert check_kc(R, lambda r: kc_swizzle(r, 64), bk=64) == 0
     if R >= 128:
         assert check_mc(R, 64, mc_swizzle, bk=64) == 0
 
