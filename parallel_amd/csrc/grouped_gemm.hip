@@ -13,13 +13,14 @@
 // on random data these kernels run against the card's power limit, and this
 // shape reads and writes each accumulator once per 32 k where 32x32x16 does
 // once per 16 (65536 x 3072 x 4096 over 128 experts 1386 against 1528 us, the
-// same instruction time: on zeros both take 1125).  The expert GEMMs use 256-column
-// tiles of 64 to 320 rows, by the mean rows per expert, on 8 waves (two waves
-// per SIMD, one workgroup per CU); the small router GEMMs use 128x128 on 4
-// waves.  Operands move from HBM to LDS by DMA (buffer_load_dwordx4 ... lds,
-// no register staging) into a ring of 32- or 64-deep k-tiles that fills the 160
-// KiB of LDS, so that 64 to 96 KiB of loads are in flight while one k-tile is
-// multiplied; each wave fires its share of a k-tile's DMA between its
+// same instruction time: on zeros both take 1125).  The expert GEMMs use
+// 256-column tiles of 64 to 320 rows, by the mean rows per expert and by how
+// many tiles run at once, on 8 waves (two waves per SIMD, one workgroup per CU);
+// the small router GEMMs use 128x128 on 4 waves.  Operands move from HBM to LDS
+// by DMA (buffer_load_dwordx4 ... lds, no register staging) into a ring of 32-
+// or 64-deep k-tiles that fills the 160 KiB of LDS, so that 64 to 96 KiB of
+// loads are in flight while one k-tile is multiplied; each wave fires its share
+// of a k-tile's DMA between its
 // MFMA groups.  At the roughly 256 rows per expert of a training step the
 // expert GEMMs sit near the ridge of the roofline (about 256 flop per weight
 // byte), and the weights stream from HBM only as fast as the bytes in flight
@@ -860,27 +861,27 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
         const int row = t.m0 + sub_row(i / 2) + 16 * (i % 2) + i16;
 #pragma unroll
         for (int j = 0; j < 2 * SN; ++j) {
-            const int col = wcol0 + j * 16 + 4 * q16;
-            const uint32_t off = (row < row_limit && col < p.N)
-                                     ? (static_cast<uint32_t>(row) * static_cast<uint32_t>(p.ldc) +
-                                        static_cast<uint32_t>(col)) * 4u
-                                     : kOOB;
-            float4 v = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
-            if (EPI == EPI_WGRAD && p.accumulate) {
-              const uint4 o = load16(rsC, off);
-              v.x += __uint_as_float(o.x);
-              v.y += __uint_as_float(o.y);
-              v.z += __uint_as_float(o.z);
-              v.w += __uint_as_float(o.w);
-            }
-            const uint4 o4 = make_uint4(__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z),
-                                        __float_as_uint(v.w));
-            if constexpr (EPI == EPI_WGRAD) {
-              store16_nt(rsC, off, o4);
-            } else {
-              store16(rsC, off, o4);
-            }
+          const int col = wcol0 + j * 16 + 4 * q16;
+          const uint32_t off = (row < row_limit && col < p.N)
+                                   ? (static_cast<uint32_t>(row) * static_cast<uint32_t>(p.ldc) +
+                                      static_cast<uint32_t>(col)) * 4u
+                                   : kOOB;
+          float4 v = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+          if (EPI == EPI_WGRAD && p.accumulate) {
+            const uint4 o = load16(rsC, off);
+            v.x += __uint_as_float(o.x);
+            v.y += __uint_as_float(o.y);
+            v.z += __uint_as_float(o.z);
+            v.w += __uint_as_float(o.w);
           }
+          const uint4 o4 = make_uint4(__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z),
+                                      __float_as_uint(v.w));
+          if constexpr (EPI == EPI_WGRAD) {
+            store16_nt(rsC, off, o4);
+          } else {
+            store16(rsC, off, o4);
+          }
+        }
       }
       return;
     }

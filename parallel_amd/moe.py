@@ -60,7 +60,7 @@ class TopKRouter(nn.Module):
         if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16:
             with torch.autocast("cuda", enabled=False):
                 return ops.run_router_fwd_bf16(hidden_states.to(torch.bfloat16), self.weight.to(torch.bfloat16),
-                                           self.top_k, self.norm_topk_prob)[:3]
+                                               self.top_k, self.norm_topk_prob)[:3]
         return ops.run_router_fwd(hidden_states, self.weight, self.top_k, self.norm_topk_prob)
 
 

@@ -48,6 +48,6 @@ def norm_router_aux(
         tw = attention_mask.to(device=hidden.device, dtype=torch.float32).reshape(-1)
         if tw.numel() != x.numel() // H:
             raise ValueError(f"attention_mask has {tw.numel()} entries for {x.numel() // H} tokens")
-    logits, scores, idx, aux, _stats = ops.run_router_aux_fwd(x.reshape(-1, H), router_weight, top_k, norm_topk_prob, tw,
-                                                          logit_bias)
+    logits, scores, idx, aux, _stats = ops.run_router_aux_fwd(x.reshape(-1, H), router_weight, top_k, norm_topk_prob,
+                                                              tw, logit_bias)
     return x, (logits, scores, idx), aux
