@@ -12,20 +12,19 @@
 // v_mfma_f32_16x16x32_bf16 (four per sub-tile and 32 k, fp32 accumulators):
 // on random data these kernels run against the card's power limit, and this
 // shape reads and writes each accumulator once per 32 k where 32x32x16 does
-// once per 16 (65536 x 3072 x 4096 over 128 experts 1386 against 1528 us, the
-// same instruction time: on zeros both take 1125).  The expert GEMMs use
+// once per 16 (65536 x 3072 x 4096 over 128 experts 1387 us on random data, 1108
+// on zeros; 1528 on random data with 32x32x16).  The expert GEMMs use
 // 256-column tiles of 64 to 320 rows, by the mean rows per expert and by how
 // many tiles run at once, on 8 waves (two waves per SIMD, one workgroup per CU);
 // the small router GEMMs use 128x128 on 4 waves.  Operands move from HBM to LDS
 // by DMA (buffer_load_dwordx4 ... lds, no register staging) into a ring of 32-
 // or 64-deep k-tiles that fills the 160 KiB of LDS, so that 64 to 96 KiB of
 // loads are in flight while one k-tile is multiplied; each wave fires its share
-// of a k-tile's DMA between its
-// MFMA groups.  At the roughly 256 rows per expert of a training step the
-// expert GEMMs sit near the ridge of the roofline (about 256 flop per weight
-// byte), and the weights stream from HBM only as fast as the bytes in flight
-// per CU allow, so the ring takes all of the LDS: the epilogue stages its
-// output through the ring stage it has just multiplied.  Each operand
+// of a k-tile's DMA between its MFMA groups.  At the roughly 256 rows per expert
+// of a training step the expert GEMMs sit near the ridge of the roofline (about
+// 256 flop per weight byte), and the weights stream from HBM only as fast as the
+// bytes in flight per CU allow, so the ring takes all of the LDS: the epilogue
+// stages its output through the ring stage it has just multiplied.  Each operand
 // keeps its HBM layout in LDS (XOR swizzled): K-contiguous fragments are
 // ds_read_b128, M/N-contiguous ones (weights in the input gradient, both
 // operands of the weight gradient) are ds_read_b64_tr_b16 transpose reads.
