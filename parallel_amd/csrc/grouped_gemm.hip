@@ -9,8 +9,9 @@
 //
 // Tiling: WM x WN waves; each wave owns (BM/WM) x (BN/WN) of 32x32 sub-tiles,
 // its row sub-tiles interleaved with the other wave rows'.  The products are
-// v_mfma_f32_16x16x32_bf16 (four per sub-tile and 32 k, fp32 accumulators):
-// on random data these kernels run against the card's power limit, and this
+// v_mfma_f32_16x16x32_bf16 (four per sub-tile and 32 k, fp32 accumulators), but
+// the weight gradients' v_mfma_f32_32x32x16_bf16 (the same bits).  On random
+// data the others run against the card's power limit, and the 16x16x32
 // shape reads and writes each accumulator once per 32 k where 32x32x16 does
 // once per 16 (65536 x 3072 x 4096 over 128 experts 1387 us on random data, 1108
 // on zeros; 1528 on random data with 32x32x16).  The expert GEMMs use
@@ -272,11 +273,13 @@ __device__ __forceinline__ constexpr int kc_swizzle(int r) {
 }
 // A transpose-read pass reads 16 columns (2 chunks) of k-rows kk .. kk + 3 and
 // kk + 8 .. kk + 11: k-row kk & 3 selects the 64-byte bank quarter, bit 3 of kk
-// the half of it (needs >= 16 chunks per k-row).
+// the half of it (needs >= 16 chunks per k-row).  (32-column fragments: 4
+// chunks of kk .. kk + 3.)
 __device__ __forceinline__ constexpr int mc_swizzle(int kk) { return 4 * (kk & 3) | 2 * ((kk >> 3) & 1); }
 // Epilogue staging of a wave's 32 x 64 bf16 pass (128-byte rows): chunk cc of
 // row r at slot cc ^ stg_swizzle(r); the 8-byte writes (16 rows, both halves of
-// a chunk), the row reads and the SwiGLU gate/up reads are each on distinct
+// a chunk; from 32x32x16, 32 rows of one half, with the halves of rows 16 .. 31
+// exchanged), the row reads and the SwiGLU gate/up reads are each on distinct
 // banks.
 __device__ __forceinline__ constexpr int stg_swizzle(int r) { return (((r >> 1) & 1) << 2) | ((r >> 2) & 3); }
 
@@ -297,6 +300,15 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   constexpr int WTN = BN / WN;  // wave tile cols
   constexpr int SM = WTM / 32;  // 32x32 sub-tiles per wave along M
   constexpr int SN = WTN / 32;  // ... along N
+  // The MFMA: 16x16x32, but 32x32x16 for the weight gradients, whose operands
+  // are both read by transposes.  16x16x32 takes 1.054 of their time (geometric
+  // mean over 104 sizes, routings and outputs: 485 against 465 us at 65536 x
+  // 1536 x 2048 over 128 experts, 235 against 208 at 32768 x 1024 x 1024 over 32
+  // with Zipf routing) and was never the faster by more than 1%.
+  constexpr bool M32 = MODE == MODE_KG;
+  constexpr int FR = M32 ? 32 : 16, FK = M32 ? 16 : 32;  // rows (columns) and depth of an operand fragment
+  constexpr int FPS = 32 / FR;                           // fragments per 32-row sub-tile and k-slice
+  constexpr int AM = SM * FPS, AN = SN * FPS;            // a wave's fragments of A and of B per k-slice
   constexpr bool A_KC = (MODE == MODE_MG);
   constexpr bool B_KC = (MODE == MODE_MG) && B_KCONTIG;
   // A K-contiguous A tile occupies whole rounds of DMA instructions in LDS
@@ -357,7 +369,8 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   // 2 grp + 1; its four waves sit on the four SIMDs.
   const int grp = wave >> 2, w4 = wave & 3;
   const int wm = PING ? (w4 >> 1) : wave / WN, wn = PING ? grp * 2 + (w4 & 1) : wave % WN;
-  const int i16 = lane & 15, q16 = lane >> 4;  // the lane's row (column) and k-group in an MFMA operand
+  const int i16 = lane & 15, q16 = lane >> 4;  // the lane's row (column) and k-group in a 16x16x32 MFMA operand
+  const int l32 = lane & 31, khalf = lane >> 5;  // ... in a 32x32x16 one
 
   // ------------------------------------------------------ this block's tiles
   const int nbx = gridDim.x / kNumXcd;  // the grid is a multiple of kNumXcd
@@ -656,12 +669,21 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   // offset and issues it, dma_advance moves the cursor.  The compute loop
   // fires the slots between its MFMA groups (ping-pong: its fragment reads),
   // so that the texture unit works through the k-step's DMA while the matrix
-  // cores run instead of taking every wave's burst at once; the offsets live
-  // in registers only around their own load.  Every k-step fires exactly LPW
-  // instructions per wave.
+  // cores run instead of taking every wave's burst at once.  The offsets live
+  // in registers only around their own load, except in the weight gradients,
+  // which keep the k-step's (1% of their time; the other GEMMs lose that much
+  // by it).  Every k-step fires exactly LPW instructions per wave.
   uint32_t dma_at = 0;
   int dma_k0 = 0, dma_left = 0;  // the k-step's first k (or k-row) in the tile, and how many are left from there
   u32x4_t ra, rb;
+  uint32_t doff[LPW], dlds[LPW];
+  auto dma_offset = [&](int j) __attribute__((always_inline)) {
+    const bool is_a = slot_is_a(j);
+    const uint32_t step = (is_a ? A_KC : B_KC) ? 2u : (is_a ? lda2 : ldb2);
+    // Past the last tile dma_pre is kOOB and stays out of range (the added
+    // offset is below the 2 GiB operand limit).
+    return dma_k[j] < dma_left ? dma_pre[j] + static_cast<uint32_t>(dma_k0) * step : kOOB;
+  };
   // `at`: LDS byte offset of the stage (ping-pong: of the operand tile's slot).
   auto dma_prepare = [&](int at) __attribute__((always_inline)) {
     dma_k0 = dk * BK;
@@ -678,14 +700,20 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
       }
     }
     dma_at = lds_address(ring) + at;
+    if constexpr (M32) {
+#pragma unroll
+      for (int j = 0; j < LPW; ++j) {
+        doff[j] = dma_offset(j);
+        dlds[j] = __builtin_amdgcn_readfirstlane(dma_at + dma_lds[j]);
+      }
+    }
   };
   auto dma_fire = [&](int j) __attribute__((always_inline)) {
-    const bool is_a = slot_is_a(j);
-    const uint32_t step = (is_a ? A_KC : B_KC) ? 2u : (is_a ? lda2 : ldb2);
-    // Past the last tile dma_pre is kOOB and stays out of range (the added
-    // offset is below the 2 GiB operand limit).
-    const uint32_t off = dma_k[j] < dma_left ? dma_pre[j] + static_cast<uint32_t>(dma_k0) * step : kOOB;
-    dma16(PING || j < LPW_A ? ra : rb, off, __builtin_amdgcn_readfirstlane(dma_at + dma_lds[j]));
+    if constexpr (M32) {
+      dma16(j < LPW_A ? ra : rb, doff[j], dlds[j]);
+    } else {
+      dma16(PING || j < LPW_A ? ra : rb, dma_offset(j), __builtin_amdgcn_readfirstlane(dma_at + dma_lds[j]));
+    }
   };
   auto dma_advance = [&]() __attribute__((always_inline)) {
     if (dj < ntiles && ++dk == dt.nk) dma_seek(dj + 1);
@@ -703,14 +731,15 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   // partly filled tile spread over all waves (and SIMDs).  Its SN column
   // sub-tiles are contiguous: columns wn*WTN + 32 j.
   //
-  // A fragment is 16 rows (columns) x 32 k, lane l holding row l % 16, k
-  // 8 (l / 16) .. + 7; a 32-row sub-tile is two of them.  Each lane's byte
+  // A fragment is FR rows (columns) x FK k, lane l holding row l % FR, k
+  // 8 (l / FR) .. + 7; a 32-row sub-tile is FPS of them.  Each lane's byte
   // offset within a stage is precomputed per fragment class; a fragment
   // address is the stage base plus a lane offset plus a constant.
-  // K-contiguous [R rows][CPR chunks]: lane reads row (tile_row + i16), chunk
-  // 4 ks + q16; fragment rows start on 16-row boundaries, so the swizzle of
-  // row tile_row + i16 is that of i16.
-  constexpr int KS = BK / 32;
+  // K-contiguous [R rows][CPR chunks] (16-row fragments): lane reads row
+  // (tile_row + i16), chunk 4 ks + q16; fragment rows start on 16-row
+  // boundaries, so the swizzle of row tile_row + i16 is that of i16.
+  static_assert(!M32 || (!A_KC && !B_KC), "K-contiguous fragments are 16 rows x 32 k");
+  constexpr int KS = BK / FK;
   auto sub_row = [&](int i) { return (wm + WM * i) * 32; };
   constexpr int B_OFF = PING ? 0 : A_BYTES;  // B's offset from the base its fragments are read with
   int a_kc[KS], b_kc[KS];
@@ -721,78 +750,108 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
     b_kc[ks] = B_OFF + wn * WTN * RB + lane_off;
   }
   // M/N-contiguous [BK k-rows][R cols] (transpose reads): lane reads k-rows
-  // 32 ks + 8 q16 + 4 h + i16 / 4 and columns tile_col + 4 (i16 % 4).  The
-  // swizzle depends only on bits 0, 1 and 3 of the k-row, so each 16-column
-  // fragment has one lane offset; ks and h add constants.
-  const int tr_krow = 8 * q16 + (i16 >> 2);
-  const int tr_col = 4 * (i16 & 3);
+  // FK ks + 4 h + i16 / 4, + 8 q16 (16-column fragments) or + 8 (q16 / 2), and
+  // columns tile_col + 4 (i16 % 4), of 32-column fragments + 16 (q16 % 2).  The
+  // swizzle depends only on bits 0, 1 and 3 of the k-row (16-deep slices change
+  // bit 4 only), so each fragment has one lane offset; ks and h add constants.
+  const int tr_krow = 8 * (q16 >> M32) + (i16 >> 2);
+  const int tr_col = 4 * (i16 & 3) + 16 * (M32 & q16 & 1);
   const int half8 = (i16 & 1) << 3;
-  int a_mc[2 * SM], b_mc[2 * SN];
+  int a_mc[AM], b_mc[AN];
 #pragma unroll
-  for (int t = 0; t < 2 * SM; ++t)
-    a_mc[t] = tr_krow * BM * 2 + ((((sub_row(t / 2) + 16 * (t % 2) + tr_col) >> 3) ^ mc_swizzle(tr_krow)) << 4) + half8;
+  for (int t = 0; t < AM; ++t)
+    a_mc[t] = tr_krow * BM * 2 + ((((sub_row(t / FPS) + FR * (t % FPS) + tr_col) >> 3) ^ mc_swizzle(tr_krow)) << 4) + half8;
 #pragma unroll
-  for (int t = 0; t < 2 * SN; ++t)
-    b_mc[t] = B_OFF + tr_krow * BN * 2 + ((((wn * WTN + 16 * t + tr_col) >> 3) ^ mc_swizzle(tr_krow)) << 4) + half8;
+  for (int t = 0; t < AN; ++t)
+    b_mc[t] = B_OFF + tr_krow * BN * 2 + ((((wn * WTN + FR * t + tr_col) >> 3) ^ mc_swizzle(tr_krow)) << 4) + half8;
   auto tr_read = [](const char* at, int row_bytes) __attribute__((always_inline)) {
     const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)at);
     const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(at + 4 * row_bytes));
     return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  // Fragment t of A (sub-tile t / 2's rows 16 (t % 2) ..) or of B (columns
-  // 16 t .. of the wave's) for k's 32 ks .. of the k-tile at `base`.
+  // Fragment t of A (sub-tile t / FPS's rows FR (t % FPS) ..) or of B (columns
+  // FR t .. of the wave's) for k's FK ks .. of the k-tile at `base`.
   auto read_a = [&](const char* base, int ks, int t) __attribute__((always_inline)) {
     if constexpr (A_KC) {
       return *reinterpret_cast<const bf16x8_t*>(base + a_kc[ks] + ((t / 2) * WM * 32 + (t % 2) * 16) * RB);
     } else {
-      return tr_read(base + a_mc[t] + 32 * ks * BM * 2, BM * 2);
+      return tr_read(base + a_mc[t] + FK * ks * BM * 2, BM * 2);
     }
   };
   auto read_b = [&](const char* base, int ks, int t) __attribute__((always_inline)) {
     if constexpr (B_KC) {
       return *reinterpret_cast<const bf16x8_t*>(base + b_kc[ks] + t * 16 * RB);
     } else {
-      return tr_read(base + b_mc[t] + 32 * ks * BN * 2, BN * 2);
+      return tr_read(base + b_mc[t] + FK * ks * BN * 2, BN * 2);
     }
   };
 
-  // acc[2 i + h][t]: rows 16 h .. of row sub-tile i, columns 16 t .. of the wave's.
-  f32x4_t acc[2 * SM][2 * SN];
+  // acc[FPS i + h][t]: rows FR h .. of row sub-tile i, columns FR t .. of the wave's.
+  using Acc = std::conditional_t<M32, f32x16_t, f32x4_t>;
+  Acc acc[AM][AN];
   auto zero_acc = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 2 * SM; ++i)
+    for (int i = 0; i < AM; ++i)
 #pragma unroll
-      for (int j = 0; j < 2 * SN; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int j = 0; j < AN; ++j)
+#pragma unroll
+        for (int r = 0; r < (M32 ? 16 : 4); ++r) acc[i][j][r] = 0.0f;
   };
   // Operands swapped: the result holds C^T fragments, so each lane owns one
   // output row and runs of 4 consecutive output columns.
-  auto mfma_row = [&](int i, const bf16x8_t& a, const bf16x8_t (&b)[2 * SN]) __attribute__((always_inline)) {
+  auto mfma_row = [&](int i, const bf16x8_t& a, const bf16x8_t (&b)[AN]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 2 * SN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a, acc[i][j], 0, 0, 0);
+    for (int j = 0; j < AN; ++j) {
+      if constexpr (M32) {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a, acc[i][j], 0, 0, 0);
+      } else {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a, acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  // Run e (of 8) of 4 consecutive columns that the lane holds of row sub-tile
+  // i's columns 64 h ..: its values, and its row and first column in there.
+  struct Run {
+    float4 v;
+    int row, col;
+  };
+  auto acc_run = [&](int i, int h, int e) __attribute__((always_inline)) {
+    if constexpr (M32) {
+      const f32x16_t& c = acc[i][2 * h + e / 4];
+      const int q = e % 4;
+      return Run{make_float4(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]), l32, 8 * e + 4 * khalf};
+    } else {
+      const f32x4_t& c = acc[2 * i + e / 4][4 * h + e % 4];
+      return Run{make_float4(c[0], c[1], c[2], c[3]), 16 * (e / 4) + i16, 16 * (e % 4) + 4 * q16};
+    }
   };
 
   // One k-tile of MFMAs over the first `na` row sub-tiles (the others hold no
   // rows of this tile; `na` is wave-uniform, so the guards are scalar
   // branches), with the prepared DMA slots fired between the MFMA groups:
-  // slot s after group (ks, i) = s * KS SM / LPW.  The next row sub-tile's
-  // fragments are read before the current one's MFMAs.
+  // slot s after group (ks, i) = s * KS SM / LPW.  The fragments of AHEAD row
+  // sub-tiles are read before the first one's MFMAs, each further one's before
+  // those of the sub-tile AHEAD before it.
   auto compute = [&](int na, const char* stage) __attribute__((always_inline)) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      bf16x8_t af[2][2], bfr[2 * SN];
+      constexpr int AHEAD = M32 ? 2 : 1;
+      bf16x8_t af[AHEAD + 1][FPS], bfr[AN];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) af[0][h] = read_a(stage, ks, h);
+      for (int i = 0; i < AHEAD; ++i)
 #pragma unroll
-      for (int j = 0; j < 2 * SN; ++j) bfr[j] = read_b(stage, ks, j);
+        for (int h = 0; h < FPS; ++h) af[i][h] = read_a(stage, ks, FPS * i + h);
+#pragma unroll
+      for (int j = 0; j < AN; ++j) bfr[j] = read_b(stage, ks, j);
 #pragma unroll
       for (int i = 0; i < SM; ++i) {
-        if (i + 1 < SM) {
+        if (i + AHEAD < SM) {
 #pragma unroll
-          for (int h = 0; h < 2; ++h) af[(i + 1) & 1][h] = read_a(stage, ks, 2 * (i + 1) + h);
+          for (int h = 0; h < FPS; ++h) af[(i + AHEAD) % (AHEAD + 1)][h] = read_a(stage, ks, FPS * (i + AHEAD) + h);
         }
         if (i == 0 || i < na) {
 #pragma unroll
-          for (int h = 0; h < 2; ++h) mfma_row(2 * i + h, af[i & 1][h], bfr);
+          for (int h = 0; h < FPS; ++h) mfma_row(FPS * i + h, af[i % (AHEAD + 1)][h], bfr);
         }
 #pragma unroll
         for (int s2 = 0; s2 < LPW; ++s2) {
@@ -816,8 +875,8 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
   };
 
   // ------------------------------------------------------ epilogue
-  // Lane owns output rows m0 + sub_row(i) + 16 h + i16 and columns
-  // wcol0 + 16 t + 4 q16 + {0..3}, holding acc[2 i + h][t].
+  // Lane owns the runs acc_run(i, h, e) of output rows m0 + sub_row(i) + row and
+  // columns wcol0 + 64 h + col + {0..3}.
   // This wave's staging slot (no other wave touches it) in the ring stage
   // that the compute cursor has just finished: no DMA targets that stage
   // before the next block barrier, and a barrier before the epilogue
@@ -856,16 +915,17 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
     if (EPI == EPI_F32 || (EPI == EPI_WGRAD && p.ldp)) {
       // fp32 outputs (split-K partials, fp32 weight gradients): direct 16-byte stores.
 #pragma unroll
-      for (int i = 0; i < 2 * SM; ++i) {
-        const int row = t.m0 + sub_row(i / 2) + 16 * (i % 2) + i16;
+      for (int ih = 0; ih < SM * (SN / 2); ++ih) {
 #pragma unroll
-        for (int j = 0; j < 2 * SN; ++j) {
-          const int col = wcol0 + j * 16 + 4 * q16;
+        for (int e = 0; e < 8; ++e) {
+          const int i = ih / (SN / 2), h = ih % (SN / 2);
+          const Run run = acc_run(i, h, e);
+          const int row = t.m0 + sub_row(i) + run.row, col = wcol0 + 64 * h + run.col;
           const uint32_t off = (row < row_limit && col < p.N)
                                    ? (static_cast<uint32_t>(row) * static_cast<uint32_t>(p.ldc) +
                                       static_cast<uint32_t>(col)) * 4u
                                    : kOOB;
-          float4 v = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+          float4 v = run.v;
           if (EPI == EPI_WGRAD && p.accumulate) {
             const uint4 o = load16(rsC, off);
             v.x += __uint_as_float(o.x);
@@ -886,8 +946,15 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
     }
     // bf16 outputs go through this wave's LDS slot one 32-row pass at a time,
     // so that every store is 16 bytes per lane over whole 128-byte row segments.
-    const int stg_lane = i16 * 128 + ((q16 & 1) << 3);
-    const int stg_swz = stg_swizzle(i16);  // (row 16 + i16 has the same)
+    // The 8-byte halves of a chunk are exchanged in rows 16 .. 31 where a
+    // write's lanes hold 32 rows of one half (32x32x16).
+    auto stg_at = [&](int row, int col) __attribute__((always_inline)) {
+      return row * 128 + (((col >> 3) ^ stg_swizzle(row)) << 4) + ((((col >> 2) & 1) ^ (M32 & (row >> 4))) << 3);
+    };
+    auto stg_row = [&](int r, int chunk) __attribute__((always_inline)) {
+      const uint4 v = *reinterpret_cast<const uint4*>(slot + r * 128 + ((chunk ^ stg_swizzle(r)) << 4));
+      return M32 && (r & 16) ? make_uint4(v.z, v.w, v.x, v.y) : v;
+    };
     const int rr8 = lane >> 3, c8 = lane & 7;  // row-read lane mapping: row 8n + rr8, chunk c8
     // One pass per 32 rows (row sub-tile i) and 64 columns (column group h:
     // sub-tiles 2h and 2h + 1).
@@ -912,15 +979,11 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
         }
       }
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
-          const f32x4_t& c = acc[2 * i + hh][4 * h + tt];
-          uint2 v;
-          v.x = pack_bf16x2(c[0], c[1]);
-          v.y = pack_bf16x2(c[2], c[3]);
-          *reinterpret_cast<uint2*>(slot + stg_lane + hh * 16 * 128 + (((2 * tt + (q16 >> 1)) ^ stg_swz) << 4)) = v;
-        }
+      for (int e = 0; e < 8; ++e) {
+        const Run run = acc_run(i, h, e);
+        *reinterpret_cast<uint2*>(slot + stg_at(run.row, run.col)) =
+            make_uint2(pack_bf16x2(run.v.x, run.v.y), pack_bf16x2(run.v.z, run.v.w));
+      }
       if constexpr (EPI == EPI_SWIGLU_FWD) {
         // Slot columns 0-31 are gate, 32-63 the matching up columns.  A lane
         // takes one 8-column gate chunk and its up chunk: act = silu(gate) * up
@@ -931,9 +994,7 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
           const int r = 16 * n + rr;
-          const int swz = stg_swizzle(r);
-          const uint4 gv = *reinterpret_cast<const uint4*>(slot + r * 128 + ((c4 ^ swz) << 4));
-          const uint4 uv = *reinterpret_cast<const uint4*>(slot + r * 128 + (((c4 + 4) ^ swz) << 4));
+          const uint4 gv = stg_row(r, c4), uv = stg_row(r, c4 + 4);
           const int row = prow0 + r;
           const bool ok = row < row_limit && act_col < p.swiglu_I;
           float gf[8], uf[8], af[8];
@@ -955,7 +1016,7 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
           const int r = 8 * n + rr8;
-          uint4 v = *reinterpret_cast<const uint4*>(slot + r * 128 + ((c8 ^ stg_swizzle(r)) << 4));
+          uint4 v = stg_row(r, c8);
           if constexpr (EPI == EPI_BF16) {
             store16(rsC, out_off[n], v);
           } else if constexpr (EPI == EPI_WGRAD) {
@@ -1056,12 +1117,12 @@ __global__ __launch_bounds__(CFG::kThreads) void grouped_gemm_kernel(const GemmP
     // 4c + 7.
     constexpr int NF = 2 * (SM + SN);  // fragments of a half k-step
     static_assert(LPW == 8 && SLOT == 4096, "group 1 stages in the half of its DMA share fired last");
-    bf16x8_t fa[2 * SM], fb[2 * SN];
+    bf16x8_t fa[AM], fb[AN];
     auto read_frag = [&](const char* sa, const char* sb, int h, int n) __attribute__((always_inline)) {
-      if (n < 2 * SM) {
+      if (n < AM) {
         fa[n] = read_a(sa, h, n);
       } else {
-        fb[n - 2 * SM] = read_b(sb, h, n - 2 * SM);
+        fb[n - AM] = read_b(sb, h, n - AM);
       }
     };
     auto fire_range = [&](int lo, int hi) __attribute__((always_inline)) {

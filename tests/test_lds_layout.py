@@ -63,12 +63,18 @@ HALF8 = _expression(r"const int half8 = ([^;]*);")
 READ_MC = _expression(r"b_mc\[t\] = B_OFF \+ ([^;]*);")
 READ_MC_KS = _expression(r"tr_read\(base \+ b_mc\[t\] \+ ([^,]*),")
 READ_MC_HI = _expression(r"\(lds_i16x4_t\*\)\(at \+ ([^)]*)\)\);")
+# The row and first column of a lane's run e of four results in a 32 x 64 pass, by the MFMA (16x16x32, 32x32x16).
+RUN_ROW = [_expression(r"Run\{make_float4\(c\[0\][^)]*\), (16[^,]*),"),
+           _expression(r"Run\{make_float4\(c\[4 [^)]*\), ([^,]*),")]
+RUN_COL = [_expression(r"Run\{make_float4\(c\[0\][^)]*\), 16[^,]*, ([^}]*)\}"),
+           _expression(r"Run\{make_float4\(c\[4 [^)]*\), [^,]*, ([^}]*)\}")]
 # Epilogue staging.
-STG_LANE = _expression(r"const int stg_lane = ([^;]*);")
-STG_WRITE = _expression(r"uint2\*>\(slot \+ stg_lane \+ (hh[^;]*)\) = v;")
-STG_ROW = _expression(r"uint4 v = \*reinterpret_cast<const uint4\*>\(slot \+ ([^;]*)\);")
-STG_GATE = _expression(r"const uint4 gv = \*reinterpret_cast<const uint4\*>\(slot \+ ([^;]*)\);")
-STG_UP = _expression(r"const uint4 uv = \*reinterpret_cast<const uint4\*>\(slot \+ ([^;]*)\);")
+STG_AT = _expression(r"auto stg_at = .*?return ([^;]*);")
+STG_ROW = _expression(r"auto stg_row = .*?\(slot \+ ([^;]*)\);")
+STG_SWAP = _expression(r"return M32 && (\(r & 16\)) \? make_uint4\(v\.z, v\.w, v\.x, v\.y\) : v;")
+STG_C8 = _expression(r"uint4 v = stg_row\(r, ([^;]*)\);")
+STG_GATE = _expression(r"const uint4 gv = stg_row\(r, ([^,]*)\), uv")
+STG_UP = _expression(r", uv = stg_row\(r, ([^;]*)\);")
 
 
 def bank_conflicts(addrs, lanes_per_pass, width):
@@ -101,7 +107,7 @@ def check_kc(R, swz, bk=32):
     return conflicts
 
 
-def check_mc(R, WT, swz, bk=32):
+def check_mc(R, WT, swz, bk=32, M32=0):
     """An M/N-contiguous [bk k-rows][R columns] tile, a wave's columns being WT wide."""
     c = dict(BM=R, BN=R, WTN=WT, is_a=False, cpk=R // 8, mc_swizzle=swz)
     where = {}
@@ -111,51 +117,57 @@ def check_mc(R, WT, swz, bk=32):
             col = DMA_MC_COL(lane=lane, dma_k=[kk], j2=0, **c)
             where[(kk, col // 8)] = li * 1024 + lane * 16
     conflicts = 0
+    FR, FK = (32, 16) if M32 else (16, 32)
+    c.update(FR=FR, FK=FK, M32=M32)
     for wn in range(R // WT):
-        for t in range(WT // 16):  # a fragment: 16 columns x 32 k, two transpose reads
-            for ks in range(bk // 32):
+        for t in range(WT // FR):  # a fragment: FR columns x FK k, two transpose reads
+            for ks in range(bk // FK):
                 for h in range(2):
                     addrs = []
                     for lane in range(64):
                         i16, q16 = lane & 15, lane >> 4
-                        krow, col = TR_KROW(i16=i16, q16=q16), TR_COL(i16=i16)
+                        krow, col = TR_KROW(i16=i16, q16=q16, M32=M32), TR_COL(i16=i16, q16=q16, M32=M32)
                         off = (READ_MC(tr_krow=krow, tr_col=col, half8=HALF8(i16=i16), wn=wn, t=t, **c)
                                + READ_MC_KS(ks=ks, **c) + h * READ_MC_HI(row_bytes=R * 2))
-                        kr, gcol = 32 * ks + krow + 4 * h, wn * WT + 16 * t + col
+                        # The transpose hands lane l (column l % FR) the k's 8 (l / FR) + 4 h ..: the lanes that
+                        # read them are the 16 of l's quarter.
+                        k0, col0 = FK * ks + 8 * (lane // FR) + 4 * h, wn * WT + FR * t + (lane % FR) // 16 * 16
+                        kr, gcol = k0 + (i16 >> 2), col0 + 4 * (i16 & 3)
                         assert where[(kr, gcol >> 3)] + (gcol & 7) * 2 == off
                         addrs.append(off)
                     conflicts += bank_conflicts(addrs, 32, 8)
     return conflicts
 
 
-def test_epilogue_staging_is_consistent_and_conflict_free():
-    """A wave's 32 x 64 bf16 pass: 8-byte writes (row 16 hh + i16, columns 16 tt + 4 q16 ..), then row
-    reads and the SwiGLU gate/up reads of whole 16-byte chunks."""
+@pytest.mark.parametrize("M32", [0, 1])
+def test_epilogue_staging_is_consistent_and_conflict_free(M32):
+    """A wave's 32 x 64 bf16 pass: 8-byte writes of runs of four columns, then row reads and (16x16x32 only)
+    the SwiGLU gate/up reads of whole 16-byte chunks, with the halves of rows 16 .. 31 in exchange for 32x32x16."""
     where = {}
-    for hh in range(2):
-        for tt in range(4):
-            addrs = []
-            for lane in range(64):
-                i16, q16 = lane & 15, lane >> 4
-                addrs.append(STG_LANE(i16=i16, q16=q16) + STG_WRITE(hh=hh, tt=tt, q16=q16, stg_swz=stg_swizzle(i16)))
-                where[(16 * hh + i16, 16 * tt + 4 * q16)] = addrs[-1]
-            assert bank_conflicts(addrs, 32, 8) == 0
-    assert len(set(where.values())) == 32 * 16
+    for e in range(8):
+        addrs = []
+        for lane in range(64):
+            names = dict(i16=lane & 15, q16=lane >> 4, l32=lane & 31, khalf=lane >> 5, e=e)
+            row, col = RUN_ROW[M32](**names), RUN_COL[M32](**names)
+            addrs.append(STG_AT(row=row, col=col, M32=M32))
+            where[(row, col)] = addrs[-1]
+        assert bank_conflicts(addrs, 32, 8) == 0
+    assert len(where) == len(set(where.values())) == 32 * 16
 
-    def reads(rows, chunk, at):
-        addrs = [at(r) for r in rows]
-        for r, cc, a in zip(rows, chunk, addrs):
-            assert where[(r, 8 * cc)] == a and where[(r, 8 * cc + 4)] == a + 8
+    def reads(rows, chunks):
+        addrs = [STG_ROW(r=r, chunk=c) for r, c in zip(rows, chunks)]
+        for r, c, a in zip(rows, chunks, addrs):
+            swap = 8 if M32 and STG_SWAP(r=r) else 0
+            assert where[(r, 8 * c)] == a + swap and where[(r, 8 * c + 4)] == a + 8 - swap
         assert bank_conflicts(addrs, 16, 16) == 0
 
+    lanes = range(64)
     for n in range(4):
-        lanes = range(64)
-        rows, c8 = [8 * n + (lane >> 3) for lane in lanes], [lane & 7 for lane in lanes]
-        reads(rows, c8, lambda r, it=iter(c8): STG_ROW(r=r, c8=next(it)))
-    for n in range(2):
-        rows, c4 = [16 * n + (lane >> 2) for lane in range(64)], [lane & 3 for lane in range(64)]
-        reads(rows, c4, lambda r, it=iter(c4): STG_GATE(r=r, c4=next(it), swz=stg_swizzle(r)))
-        reads(rows, [c + 4 for c in c4], lambda r, it=iter(c4): STG_UP(r=r, c4=next(it), swz=stg_swizzle(r)))
+        reads([8 * n + (lane >> 3) for lane in lanes], [STG_C8(c8=lane & 7) for lane in lanes])
+    for n in range(0 if M32 else 2):
+        rows = [16 * n + (lane >> 2) for lane in lanes]
+        reads(rows, [STG_GATE(c4=lane & 3) for lane in lanes])
+        reads(rows, [STG_UP(c4=lane & 3) for lane in lanes])
 
 
 @pytest.mark.parametrize("R", [128, 256])
@@ -163,9 +175,10 @@ def test_k_contiguous_layout_is_consistent_and_conflict_free(R):
     assert check_kc(R, kc_swizzle) == 0
 
 
+@pytest.mark.parametrize("M32", [0, 1])
 @pytest.mark.parametrize("R,WT", [(128, 64), (256, 64), (256, 128)])
-def test_transpose_read_layout_is_consistent_and_conflict_free(R, WT):
-    assert check_mc(R, WT, mc_swizzle) == 0
+def test_transpose_read_layout_is_consistent_and_conflict_free(R, WT, M32):
+    assert check_mc(R, WT, mc_swizzle, M32=M32) == 0
 
 
 @pytest.mark.parametrize("R", [64, 128, 256])
@@ -173,6 +186,7 @@ def test_64_deep_layouts_are_consistent_and_conflict_free(R):
     assert check_kc(R, lambda r: kc_swizzle(r, 64), bk=64) == 0
     if R >= 128:
         assert check_mc(R, 64, mc_swizzle, bk=64) == 0
+        assert check_mc(R, 64, mc_swizzle, bk=64, M32=1) == 0
 
 
 def test_model_flags_32_bank_swizzles():
